@@ -1,0 +1,153 @@
+"""The filter scan: approximate float16 scores with an error bound decide which pairs are scored
+exactly, so every result must be the oracle's (within float32 rounding) whatever the approximation
+does. Sizes at its edges: rows of one chunk to 4 KB, whole and partial 256-byte pieces, 128-byte
+halves and 16-byte chunks, one and several rounds of pieces; one query to several launches; row
+counts that end in a partial block; masks that let through everything, some, and fewer rows than k."""
+
+import numpy as np
+import pytest
+
+import oracle
+from helpers import assert_topk_equivalent, float_tolerance, normalized
+
+pytestmark = pytest.mark.gpu
+
+INT8_SCALE = np.float32(1.0 / 127.0)
+
+
+def encode(capi, rows, kind):
+    """(stored array, dtype, decoded rows)."""
+    if kind == "f32":
+        return rows, capi.F32, rows
+    if kind == "f16":
+        half = oracle.f32_to_f16(rows)
+        return half, capi.F16, half.astype(np.float32)
+    codes = oracle.quantize_i8(rows, INT8_SCALE)
+    return codes, capi.I8, oracle.dequantize_i8(codes, INT8_SCALE)
+
+
+def run(capi, stored, dtype, queries, k, metric, mask=None, flags=0):
+    n, dim = stored.shape
+    d_rows, d_queries = capi.DeviceArray.from_host(stored), capi.DeviceArray.from_host(queries)
+    d_mask = None if mask is None else capi.DeviceArray.from_host(mask)
+    store = capi.store_desc(d_rows, n, dim, dtype, float(INT8_SCALE) if dtype == capi.I8 else 1.0)
+    desc = capi.search_desc(store, d_queries, queries.shape[0], k, metric, mask=d_mask, flags=flags)
+    return capi.search(desc)
+
+
+CASES = [
+    # kind, n, dim, batch, k, metric (0 cosine, 1 dot, 2 L2), share of rows a mask lets through
+    ("f16", 9_001, 64, 9, 10, 2, None),        # half a piece
+    ("f16", 9_001, 72, 17, 10, 0, 0.5),        # a chunk past half a piece
+    ("f16", 20_011, 100, 1, 10, 0, None),      # rows of 200 bytes, one query
+    ("f16", 20_011, 136, 33, 10, 2, None),     # a chunk past a piece
+    ("f16", 20_011, 300, 65, 20, 0, 0.3),      # rows of 600 bytes
+    ("f16", 20_011, 333, 5, 10, 2, None),      # rows at 2-byte alignment
+    ("f16", 9_001, 640, 33, 10, 0, None),      # 5 pieces: two rounds, the last slot empty
+    ("f16", 9_001, 768, 130, 100, 1, None),    # three launches of query groups
+    ("f16", 9_001, 1000, 16, 10, 2, 0.9),      # 8 pieces, the last one partial
+    ("f16", 9_001, 2048, 7, 10, 0, None),      # the widest rows
+    ("f32", 9_001, 64, 20, 10, 2, None),       # one piece
+    ("f32", 20_011, 100, 40, 10, 0, 0.2),      # 400 bytes
+    ("f32", 20_011, 333, 3, 10, 0, None),      # rows at 4-byte alignment
+    ("f32", 9_001, 600, 12, 10, 2, None),      # 10 pieces: three rounds of 4, two slots empty
+    ("f32", 9_001, 1024, 128, 10, 1, None),    # the widest rows
+    ("f32", 20_011, 384, 64, 100, 0, 0.5),
+    ("i8", 40_013, 100, 9, 10, 0, None),       # rows at 4-byte alignment
+    ("i8", 20_011, 128, 17, 10, 2, None),      # half a piece
+    ("i8", 20_011, 384, 128, 10, 1, 0.4),      # a piece and a half
+    ("i8", 20_011, 777, 33, 10, 0, None),      # rows at any alignment
+    ("i8", 9_001, 1024, 5, 200, 2, None),
+    ("f16", 20_011, 768, 9, 50, 0, 0.0),       # (only the rows added below): fewer rows than k
+    ("f32", 20_011, 301, 9, 50, 2, 0.0),
+    ("f16", 20_011, 768, 9, 10, 0, 1.0),
+]
+
+
+@pytest.mark.parametrize("kind,n,dim,batch,k,metric,share", CASES)
+def test_filter_scan(gpu, kind, n, dim, batch, k, metric, share):
+    capi = gpu
+    stored, dtype, decoded = encode(capi, normalized(n, dim, 300 + dim), kind)
+    queries = normalized(batch, dim, 400 + batch)
+    mask = None
+    if share is not None:
+        mask = (np.random.default_rng(dim).random(n) < share).astype(np.uint8)
+        mask[[3, n - 1, n // 2]] = 1
+    idx, val, flags = run(capi, stored, dtype, queries, k, metric, mask)
+    assert not flags.any()
+    assert_topk_equivalent(idx, val, oracle.scores_f32(decoded, queries, metric, mask), k,
+                           float_tolerance(queries, decoded, metric))
+
+
+@pytest.mark.parametrize("kind,dim,scale", [("f32", 768, 1e6), ("f32", 768, 1e-6), ("f32", 1024, 3e18), ("f16", 768, 1e-5),
+                                            ("f16", 1024, 3e4)])
+def test_magnitudes(gpu, kind, dim, scale):
+    # float32 rows outside float16's range, float16 rows that are mostly subnormal or near the largest
+    capi = gpu
+    n, batch, k = 9_001, 9, 10
+    rows = (normalized(n, dim, 61) * np.float32(scale)).astype(np.float32)
+    stored, dtype, decoded = encode(capi, rows, kind)
+    queries = normalized(batch, dim, 62)
+    idx, val, _ = run(capi, stored, dtype, queries, k, 1)
+    assert_topk_equivalent(idx, val, oracle.scores_f32(decoded, queries, 1), k,
+                           float_tolerance(queries, decoded, 1) - np.float64(1e-7) * (scale < 1e-3))
+
+
+def test_mixed_magnitudes(gpu):
+    # rows whose scales span forty binary orders: most approximate to zero or overflow float16
+    capi = gpu
+    n, dim, batch, k = 9_001, 640, 5, 10
+    rng = np.random.default_rng(63)
+    rows = normalized(n, dim, 64) * np.exp2(rng.integers(-20, 21, (n, 1))).astype(np.float32)
+    queries = normalized(batch, dim, 65)
+    idx, val, _ = run(capi, rows, capi.F32, queries, k, 1)
+    assert_topk_equivalent(idx, val, oracle.scores_f32(rows, queries, 1), k, float_tolerance(queries, rows, 1))
+
+
+@pytest.mark.parametrize("kind,dim,metric", [("f16", 768, 0), ("f32", 300, 2), ("i8", 333, 0)])
+def test_ties_take_the_lowest_rows(gpu, kind, dim, metric):
+    # 40 distinct rows, 500 copies of each: the k best are the lowest copies of the best row
+    capi = gpu
+    n, batch, k = 20_000, 6, 30
+    distinct = normalized(40, dim, 71)
+    stored, dtype, decoded = encode(capi, distinct[np.arange(n) % 40], kind)
+    queries = normalized(batch, dim, 72)
+    idx, val, _ = run(capi, stored, dtype, queries, k, metric)
+    best = np.argmax(oracle.scores_f32(decoded[:40], queries, metric), axis=1)
+    assert np.array_equal(idx, best[:, None] + 40 * np.arange(k)[None, :])
+    assert (val == val[:, :1]).all()
+
+
+def test_non_finite(gpu):
+    # infinite and NaN components follow the float32 sum: +inf ranks first, NaN last; a query with a
+    # NaN scores NaN everywhere and takes the lowest rows
+    capi = gpu
+    n, dim, batch, k = 9_001, 768, 8, 10
+    rows = normalized(n, dim, 81)
+    rows[17, 3], rows[4_321, 3], rows[900, 5] = np.inf, np.inf, np.nan
+    queries = normalized(batch, dim, 82)
+    queries[:, 3] = np.abs(queries[:, 3]) + np.float32(0.01)
+    queries[2, 9] = np.nan
+    queries[3, 3] = -queries[3, 3]
+    idx, val, _ = run(capi, rows, capi.F32, queries, k, 0)
+    assert np.array_equal(idx[2], np.arange(k)) and np.isnan(val[2]).all()
+    assert not np.isin(idx[3], [17, 4_321, 900]).any()
+    for q in (0, 1, 4, 7):
+        assert idx[q, :2].tolist() == [17, 4_321] and np.isinf(val[q, :2]).all()
+    assert not (np.delete(idx, 2, axis=0) == 900).any()
+
+
+@pytest.mark.parametrize("kind,dim,metric", [("f16", 768, 0), ("f16", 301, 2), ("i8", 100, 0), ("f32", 333, 1)])
+def test_overflowing_segments_fall_back(gpu, kind, dim, metric):
+    capi = gpu
+    n, batch, k = 20_011, 11, 150
+    stored, dtype, decoded = encode(capi, normalized(n, dim, 91), kind)
+    queries = normalized(batch, dim, 92)
+    mask = np.ones(n, np.uint8)
+    mask[::3] = 0
+    idx, val, flags = run(capi, stored, dtype, queries, k, metric, mask, capi.SEARCH_TEST_TINY_SEGMENTS)
+    assert flags.any()
+    plain = run(capi, stored, dtype, queries, k, metric, mask)
+    assert np.array_equal(idx, plain[0]) and np.array_equal(val, plain[1])
+    assert_topk_equivalent(idx, val, oracle.scores_f32(decoded, queries, metric, mask), k,
+                           float_tolerance(queries, decoded, metric))

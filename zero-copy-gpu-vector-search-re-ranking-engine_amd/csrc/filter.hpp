@@ -1,0 +1,83 @@
+// Filter scan (filter_scan.hip): float32, float16 and matrix-scale int8 corpora of any row width,
+// cosine, dot or L2, with or without an allow-mask, against a batch of float32 queries.
+//
+// Each (row, query) pair first gets an approximate score from the matrix cores, rounded to
+// float16 operands, with a bound on its distance from the exact score; only pairs whose
+// approximation plus bound reaches the query's threshold are scored exactly, as the VALU scan
+// scores them (scan_core.hpp), and only exact scores become keys. So results are those of the VALU
+// scan bit for bit, and the approximation decides nothing but how many pairs are scored twice.
+#pragma once
+
+#include "common.hpp"
+#include "fused.hpp"
+
+namespace zcgvs_hip {
+
+// Queries are prepared per 16 (a query group): float16 matrix-core operands and FilterQuery
+// constants. Rows are read in 256-byte pieces, kFilterSteps(kind) 32-dimension products each.
+constexpr int kFilterGroup = 16;
+constexpr int kFilterMaxGroups = 8;                  // query groups per launch
+constexpr int kFilterWaves = 8;                      // wavefronts per workgroup
+constexpr std::size_t kFilterOperandBytes = 128 * 1024;  // LDS of a launch's query operands
+constexpr int kFilterSketchSlots = kFilterWaves;     // sketch slots per workgroup
+constexpr int kFilterBlockRows = 16;                 // rows of a sketch phase's work item
+
+// 256-byte pieces of a row kept in flight: whole rows of up to 4 pieces, wider ones in rounds of 3
+// or 4.
+constexpr int filterSlots(int pieces) {
+    return pieces <= 4 ? pieces : pieces == 5 || pieces == 6 || pieces == 9 ? 3 : 4;
+}
+
+// 16-row blocks of a wavefront's tile, which make it 8 to 16 KB in flight.
+constexpr int filterBlocks(int slots, int groups) {
+    return slots == 1 ? (groups <= 2 ? 4 : 2) : slots == 2 && groups <= 2 ? 2 : 1;
+}
+
+struct FilterQuery {
+    float scale;  // the power of two the operands were multiplied by
+    float norm2;  // sum q_j^2
+    float usable; // 0: not finite or out of range, every pair is scored exactly
+    float pad;
+};
+
+struct FilterArgs {
+    std::uint8_t* operands = nullptr;  // [groups][steps][64 lanes][16 bytes]
+    FilterQuery* queries = nullptr;    // [groups * 16]
+    float* row_unit = nullptr;         // one float: stored value = unit * operand value (float32 rows)
+    std::uint32_t* list = nullptr;     // allow-mask: row numbers to scan (bit 31: a masked row), or null
+    std::uint32_t* list_count = nullptr;
+    int steps = 0;                     // 32-dimension steps of a row, whole pieces
+    int groups = 0;                    // query groups prepared (launches * groups per launch)
+    int groups_per_launch = 0;
+    int width = 0;                     // keys selected per query
+    // Launches of 32 to 128 queries over float32 rows of 256 or 384 components take NaN for an
+    // infinite score, as the split scan (fused_mfma_split.hip) does.
+    int infinite_as_nan = 0;
+};
+
+// How a search of this shape runs, or supported = false.
+struct FilterShape {
+    bool supported = false;
+    int steps = 0;
+    int groups = 0;
+    int groups_per_launch = 0;
+    int tile_rows = 0;  // rows of a threshold phase's work item
+};
+FilterShape filterShape(const ScanArgs& scan, int width);
+inline std::size_t filterOperandBytes(const FilterShape& shape) {
+    return static_cast<std::size_t>(shape.groups) * shape.steps * 1024;
+}
+// Entries of the row list: every row, and room for a whole tile.
+inline std::size_t filterListEntries(long long rows) { return static_cast<std::size_t>(rows) + 64; }
+
+// The query operands, the row unit and, with a mask, the row list.
+int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_t stream);
+// After a sketch phase: tau[q] (and tau_safe[q]), a key below the width-th best of query q's rows.
+int launchFilterThreshold(const float* sketch, int slots, int batch, int width, std::uint64_t* tau,
+                          std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream);
+// A sketch phase (emit.sketch: the best certain lower bound of every slot's rows; items of 16 rows)
+// or a threshold phase (items of tile_rows rows; over every listed row when there is a row list).
+int launchFilterScan(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,
+                     int workgroups, hipStream_t stream);
+
+}  // namespace zcgvs_hip

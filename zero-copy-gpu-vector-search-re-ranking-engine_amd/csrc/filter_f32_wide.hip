@@ -1,0 +1,9 @@
+// The filter scan (filter_kernel.hpp) over float32 rows of more than 512 bytes.
+#include "filter_kernel.hpp"
+
+namespace zcgvs_hip {
+
+template int launchFilterKind<ZCGVS_DTYPE_F32, true>(const ScanArgs&, const FilterArgs&, const PhaseArgs&, const EmitArgs&,
+                                               int, hipStream_t);
+
+}  // namespace zcgvs_hip

@@ -1,0 +1,769 @@
+// The filter scan's kernel (filter.hpp); filter_f32.hip, filter_f16.hip and filter_i8.hip
+// instantiate it for their row type.
+//
+// Work split. One workgroup of 8 wavefronts per compute unit. The launch's query operands (up to
+// 8 groups of 16 queries) lie in LDS for the whole launch; every wavefront streams rows of its own
+// straight into registers, in the layout the matrix core wants, so no barrier runs in the loop. A
+// wavefront's tile is kBlocks blocks of 16 rows, of which it keeps kPieces pieces of 256 bytes of
+// every row in flight (whole rows up to 1 KB), four 16-byte loads a lane, block and piece: as it
+// consumes a load it starts the same one of the next tile. That is 8 to 16 KB of consecutive
+// memory per wavefront, read at about one time; registers take rows at any alignment, which is why rows of no
+// whole 16-byte chunks come this way too.
+//
+// A load instruction reads 8 lanes of 16 bytes per row, whole 128-byte lines, and goes through 2 KB of
+// LDS per wavefront into the matrix core's layout (16 rows side by side); loads in that layout
+// touch 16 lines of 16 bytes each per quarter-wavefront and stream half as fast.
+//
+// What bounds it: HBM. Measured (kernel alone; the VALU scan it replaces took 17 to 6 times as long for
+// the whole search, the bf16 split scan 1.3): 1M x 768 float16, 32 queries, k = 100 272 us (5.6 of
+// the 7.07 TB/s a streaming read reaches), 1M x 384 float32, 64 queries 263 us (5.8), 500,009 x 256
+// float32 L2 87 us, 400,009 x 300 float16 49 us (4.9), 300,000 allowed rows of 1M x 384 float16 42 us
+// (5.5), 1M x 384 int8, 8 queries 94 us (4.1: it also converts its codes
+// to halves). A ring of more registers (6 and 8 pieces) made the compiler spill: 297-310 us for the
+// first; tiles of 64 rows a piece at a time 577 us.
+//
+// MFMA layout (16x16x32 f16): the queries are the first operand (lane l supplies query l % 16 and 8
+// dimensions), the rows the second (row l % 16, the same 8 dimensions), so a lane's results belong
+// to one row (l % 16), queries 4 (l / 16) + i, and row properties (norm, mask) stay in their lane.
+// Lane group h = l / 16 loads chunk 16 g + 4 j + h of piece g (j < 4). The products may sum the
+// dimensions in any order, so float32 rows pair chunks j and j + 1 into one operand.
+//
+// A row's last chunk may be partial: it is then read as the row's last 16 bytes and the bytes that
+// repeat earlier ones are cleared; chunks past it re-read it and are cleared whole. No load leaves
+// its row.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "filter.hpp"
+#include "scan_core.hpp"
+#include "select.hpp"
+
+namespace zcgvs_hip {
+
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef unsigned int v4uAny __attribute__((ext_vector_type(4), aligned(1)));
+typedef float v4fAny __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int kFilterThreads = kFilterWaves * kWave;
+constexpr int kPieceBytes = 256;
+constexpr int kPieceLoads = 4;  // 16-byte chunks of a piece per lane
+constexpr std::uint32_t kMaskedRow = 0x80000000u;
+constexpr std::uint32_t kNoRow = 0xFFFFFFFFu;
+constexpr int kParkSlots = 160;  // pairs a wavefront parks
+
+template <int kKind>
+struct FilterKind {
+    static constexpr int kElems = elementsPerChunk(kKind);
+    static constexpr int kSteps = kKind == ZCGVS_DTYPE_F32 ? 2 : kKind == ZCGVS_DTYPE_F16 ? 4 : 8;  // per piece
+};
+
+// Relative error of an approximate dot product, in units of |q| |x|: operand rounding (float16
+// queries to nearest, 2^-11; float32 rows toward zero, another 2^-10), float32 accumulation over
+// `steps` products of 32 (each taken at 2^-21, four times a rounding of every addition inside),
+// and the exact score's own rounding.
+__host__ __device__ inline float filterRelative(int kind, int steps) {
+    const float operands = kind == ZCGVS_DTYPE_F32 ? 1.48e-3f : 4.95e-4f;
+    return operands + 4.8e-7f * static_cast<float>(steps) + 3.1e-5f;
+}
+
+// (Through a pointer to global memory: a flat load counts as an LDS operation as well, and every
+// operand read would wait for the rows in flight.)
+template <bool kOnce>
+__device__ __forceinline__ v4u loadRowChunk(const std::uint8_t* p) {
+    typedef const __attribute__((address_space(1))) v4uAny* GlobalChunk;
+    const GlobalChunk at = (GlobalChunk)(reinterpret_cast<std::uintptr_t>(p));
+    if constexpr (kOnce) {
+        return __builtin_nontemporal_load(at);
+    } else {
+        return *at;
+    }
+}
+
+// Words of a chunk with its first `skip` bytes cleared (skip >= 16: all).
+__device__ __forceinline__ v4u keepFrom(v4u v, int skip) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const int s = skip - 4 * w;
+        v[w] = s <= 0 ? v[w] : s >= 4 ? 0u : v[w] & (0xFFFFFFFFu << (8 * s));
+    }
+    return v;
+}
+
+// The exact score of `row` (allowed) for query q, by the L lanes of a group, as the VALU scan
+// computes it: lane g of the group takes chunks g, g + L, ... in turn, groupSum adds the lanes.
+template <int kKind, int L>
+__device__ __forceinline__ float exactScoreLanes(const ScanArgs& scan, std::uint32_t row, int q, int lane) {
+    using Traits = ChunkTraits<kKind>;
+    constexpr int E = Traits::kElems;
+    constexpr int kPer = 8;
+    const int dim = scan.dim;
+    const int row_bytes = static_cast<int>(rowBytes(kKind, dim));
+    const int chunks = row_bytes / 16;
+    const std::uint8_t* base = static_cast<const std::uint8_t*>(scan.corpus) + static_cast<std::size_t>(row) * row_bytes;
+    const float* query = static_cast<const float*>(scan.queries) + static_cast<std::size_t>(q) * dim;
+    const bool l2 = scan.metric == ZCGVS_METRIC_L2;
+    // (every load without a branch, so that all are in flight together; the opaque copy keeps their
+    // addresses from being computed, and kept in memory, outside the caller's loop)
+    v4u raw[kPer];
+    int group = lane % L;
+    asm volatile("" : "+v"(group));
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+        if (t * L < chunks) {  // (uniform)
+            raw[t] = loadRowChunk<false>(base + min(group + t * L, chunks - 1) * 16);
+        }
+    }
+    float qe[kPer][E];
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+        if (t * L < chunks) {  // (uniform)
+            const float* qv = query + min((group + t * L) * E, dim - E);
+#pragma unroll
+            for (int e = 0; e < E; e += 4) {
+                const v4f part = *reinterpret_cast<const v4fAny*>(qv + e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    qe[t][e + i] = part[i];
+                }
+            }
+        }
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+        if (group + t * L < chunks) {
+            float v[E];
+            Traits::decode(make_uint4(raw[t][0], raw[t][1], raw[t][2], raw[t][3]), scan.scale, v);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const float d = l2 ? qe[t][e] - v[e] : v[e];
+                acc = fmaf(l2 ? d : qe[t][e], d, acc);
+            }
+        }
+    }
+    const float total = groupSum<L>(acc);
+    return l2 ? -total : total;
+}
+
+// The same for rows of no whole 16-byte chunks, by a whole wavefront, as the launchers' scalar
+// scan computes it.
+template <int kKind>
+__device__ __forceinline__ float exactScoreStrided(const ScanArgs& scan, std::uint32_t row, int q, int lane) {
+    const int dim = scan.dim;
+    const std::uint8_t* values = static_cast<const std::uint8_t*>(scan.corpus) + static_cast<std::size_t>(row) * rowBytes(kKind, dim);
+    const float* query = static_cast<const float*>(scan.queries) + static_cast<std::size_t>(q) * dim;
+    const bool l2 = scan.metric == ZCGVS_METRIC_L2;
+    float acc = 0.0f;
+#pragma unroll 4
+    for (int j = lane; j < dim; j += kWave) {
+        const float x = loadScalar<kKind>(values, j, scan.scale);
+        const float d = l2 ? query[j] - x : x;
+        acc = fmaf(l2 ? d : query[j], d, acc);
+    }
+    const float total = groupSum<kWave>(acc);
+    return l2 ? -total : total;
+}
+
+template <int kKind>
+__device__ __forceinline__ float exactScore(const ScanArgs& scan, std::uint32_t row, int q, int lane, int lanes) {
+    switch (lanes) {  // (uniform)
+        case 8: return exactScoreLanes<kKind, 8>(scan, row, q, lane);
+        case 16: return exactScoreLanes<kKind, 16>(scan, row, q, lane);
+        case 32: return exactScoreLanes<kKind, 32>(scan, row, q, lane);
+        default: return exactScoreStrided<kKind>(scan, row, q, lane);
+    }
+}
+
+// A sketch phase (phase.sketch) scores one block of 16 rows per tile and keeps the best lower
+// bound of each query per wavefront.
+template <int kKind, int kPieces, int kBlocks, int kGroups>
+__global__ __launch_bounds__(kFilterThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs emit, int q_offset, int q_count,
+                      int lanes_per_row) {
+    constexpr int kSteps = FilterKind<kKind>::kSteps;
+    constexpr int kQueries = kGroups * kFilterGroup;
+    constexpr bool kF32 = kKind == ZCGVS_DTYPE_F32;
+    constexpr bool kF16 = kKind == ZCGVS_DTYPE_F16;
+
+    __shared__ __attribute__((aligned(16))) std::uint8_t lds_operands[kFilterOperandBytes];
+    __shared__ __attribute__((aligned(16))) float lds_slope[kQueries];  // threshold = slope * row term + base
+    __shared__ __attribute__((aligned(16))) float lds_base[kQueries];
+    __shared__ __attribute__((aligned(16))) float lds_gain[kQueries];   // sketch: bound = gain * acc + that
+    __shared__ std::uint64_t lds_tau[kQueries];
+    __shared__ std::uint32_t lds_count[kQueries];
+    __shared__ std::uint64_t lds_lowest[kQueries];  // the lowest of the first `width` keys appended
+    __shared__ std::uint32_t lds_placed[kQueries];  // how many of those it covers
+    __shared__ __attribute__((aligned(16))) std::uint8_t lds_stage[kFilterWaves][kFilterBlockRows * kPieceBytes / 2];
+    __shared__ uint2 lds_park[kFilterWaves][kParkSlots];
+
+    const bool sketch = phase.sketch != 0;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int r16 = lane & 15;
+    const int h = lane >> 4;
+    const int dim = scan.dim;
+    const int row_bytes = static_cast<int>(rowBytes(kKind, dim));
+    const int rounds = (row_bytes + kPieces * kPieceBytes - 1) / (kPieces * kPieceBytes);
+    const int steps = args.steps;
+    const bool l2 = scan.metric == ZCGVS_METRIC_L2;
+    const std::uint8_t* corpus = static_cast<const std::uint8_t*>(scan.corpus);
+    const std::uint32_t* list = args.list;
+    const long long rows = list != nullptr ? static_cast<long long>(*args.list_count) : scan.doc_count;
+
+    // ---- tiles ----
+    const long long row_blocks = (rows + kFilterBlockRows - 1) / kFilterBlockRows;
+    long long tiles = list != nullptr ? (row_blocks + kBlocks - 1) / kBlocks : phase.items;
+    long long stride = 1;  // sketch: one block of every `stride`
+    if (sketch) {
+        // (with a row list the host knows only an upper bound of the rows: the stride that visits
+        // about as many blocks as planned)
+        stride = list != nullptr ? max(1LL, (row_blocks + phase.items - 1) / phase.items) : phase.stride;
+        tiles = (row_blocks + stride - 1) / stride;
+    }
+    const long long waves = static_cast<long long>(gridDim.x) * kFilterWaves;
+    long long tile = static_cast<long long>(wave) * gridDim.x + blockIdx.x;
+
+    // Place of threshold tile t among the corpus's (the list's) tiles.
+    auto tileAt = [&](long long t) __attribute__((always_inline)) -> long long {
+        return list != nullptr ? t : phaseBlock(t, phase.stride, phase.skip);
+    };
+    // Entry (row number, kMaskedRow with it for a masked one) of place `local` of tile t.
+    auto entryOf = [&](long long t, int local) __attribute__((always_inline)) -> std::uint32_t {
+        const long long at = (sketch ? t * stride : tileAt(t) * kBlocks) * kFilterBlockRows + local;
+        std::uint32_t entry = kNoRow;
+        if (at < rows && !(sketch && local >= kFilterBlockRows)) {
+            entry = list != nullptr ? list[at] : static_cast<std::uint32_t>(at);
+        }
+        return entry;
+    };
+    // The rows this lane reads: places 16 b + 8 i + lane / 8 (no row: the corpus's first, whose
+    // lines all such lanes share; never used for a result).
+    auto readRows = [&](long long t, std::uint32_t (&row)[kBlocks][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const std::uint32_t entry = t < tiles ? entryOf(t, kFilterBlockRows * b + 8 * i + (lane >> 3)) : kNoRow;
+                row[b][i] = entry == kNoRow ? 0u : entry & ~kMaskedRow;
+            }
+        }
+    };
+    const int last_chunk = row_bytes - 16;
+    // Rows of whole 128-byte lines are read with the non-temporal hint (256 -> 293 us without it at
+    // 1M x 384 float32); others share lines between loads, and the hint fetches those twice (65 ->
+    // 92 us with it at 400,000 x 300 float16).
+    const bool whole_lines = row_bytes % 128 == 0;
+    v4u ring[kPieces][kBlocks][2][2];
+    // Refills half `half` of slot p with that of piece `piece`: chunk 8 half + lane % 8 of the rows.
+    auto issue = [&](const std::uint32_t (&row)[kBlocks][2], int p, int piece, int half) __attribute__((always_inline)) {
+        const int off = min(piece * kPieceBytes + 128 * half + 16 * (lane & 7), last_chunk);
+        const std::uint8_t* at[kBlocks][2];
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                at[b][i] = corpus + (static_cast<std::uint64_t>(row[b][i]) * static_cast<std::uint32_t>(row_bytes) +
+                                     static_cast<std::uint32_t>(off));
+                if (p == kPieces - 1 && piece * kPieceBytes + 128 * half >= row_bytes) {
+                    at[b][i] = corpus;  // nothing of the row is there: one line for all (but as many loads in
+                                        // flight, which the waits count)
+                }
+            }
+        }
+        if (whole_lines) {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                ring[p][b][half][0] = loadRowChunk<true>(at[b][0]);
+                ring[p][b][half][1] = loadRowChunk<true>(at[b][1]);
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                ring[p][b][half][0] = loadRowChunk<false>(at[b][0]);
+                ring[p][b][half][1] = loadRowChunk<false>(at[b][1]);
+            }
+        }
+    };
+    auto issueTile = [&](const std::uint32_t (&row)[kBlocks][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+            issue(row, p, p, 0);
+            issue(row, p, p, 1);
+        }
+    };
+
+    // the first tile's rows are on their way while the operands are
+    std::uint32_t row[kBlocks][2];
+    readRows(tile, row);
+    issueTile(row);
+
+    // ---- the launch's operands: groups q_offset / 16 .. + kGroups ----
+    {
+        const v4u* src = reinterpret_cast<const v4u*>(args.operands) +
+                         static_cast<std::size_t>(q_offset / kFilterGroup) * steps * kWave;
+        v4u* dst = reinterpret_cast<v4u*>(lds_operands);
+        const int words = kGroups * steps * kWave;
+#pragma unroll 6
+        for (int i = tid; i < words; i += kFilterThreads) {
+            dst[i] = src[i];
+        }
+    }
+    const float unit = kF32 ? *args.row_unit : kF16 ? 1.0f : scan.scale;  // stored value = unit * operand
+    const float inverse_unit = kF32 ? 1.0f / unit : 1.0f;                 // (float32: a power of two)
+    const float relative = filterRelative(kKind, steps);
+    // Absolute part, in operand units per |q|: float32 rows below float16's smallest normal lose up
+    // to 2^-24 a component; products of float16 subnormals may be dropped from the norm.
+    const float root_dim = sqrtf(static_cast<float>(dim));
+    const float floor_abs = kF32 ? root_dim * 5.97e-8f : kF16 ? root_dim * 6.2e-5f * relative : 0.0f;
+    const float norm_abs = unit * unit * static_cast<float>(dim) * 3.8e-9f;
+    for (int i = tid; i < kQueries; i += kFilterThreads) {
+        const bool valid = i < q_count;
+        const FilterQuery query = args.queries[q_offset + i];
+        const float qnorm = sqrtf(query.norm2) * 1.00001f;
+        if (sketch) {
+            // lower bound = gain * acc + slope * row term + base
+            float gain = unit / query.scale;
+            float slope = -relative * qnorm * unit;
+            float base = -qnorm * unit * floor_abs;
+            if (l2) {
+                gain *= 2.0f;
+                slope = -(1.0f + 2.0f * relative) * unit * unit;
+                base = 2.0f * (base - norm_abs) - (1.0f + 2.0f * relative) * query.norm2;
+            }
+            lds_gain[i] = valid && query.usable != 0.0f ? gain : __uint_as_float(0x7FC00000u);  // NaN: no bound
+            lds_slope[i] = slope;
+            lds_base[i] = base;
+        } else {
+            // a pair survives unless acc < slope * row term + base
+            bool gated = false;
+            const std::uint64_t tau = valid ? emit.tau[q_offset + i] : ~0ull;
+            const float floor_score = keyFloor(tau, &gated);
+            const float to_acc = query.scale / unit;  // dot product -> accumulator
+            float slope = -relative * qnorm * query.scale;
+            float base = to_acc * floor_score - qnorm * query.scale * floor_abs;
+            if (l2) {
+                slope = 0.5f * (1.0f - 2.0f * relative) * unit * query.scale;
+                base = to_acc * (0.5f * (floor_score + (1.0f - 2.0f * relative) * query.norm2) - qnorm * unit * floor_abs -
+                                 norm_abs);
+            }
+            const bool filter = gated && query.usable != 0.0f && fabsf(base) < 3.0e38f && fabsf(slope) < 3.0e38f &&
+                                floor_score > kMaskedScore;
+            lds_slope[i] = valid && filter ? slope : 0.0f;
+            // (a query past the batch takes no pair: nothing but NaN fails acc < inf, and those
+            // pairs are dropped by its threshold key)
+            lds_base[i] = !valid ? INFINITY : filter ? base : -INFINITY;
+            lds_tau[i] = tau;
+            lds_count[i] = 0u;
+            lds_lowest[i] = ~0ull;
+            lds_placed[i] = 0u;
+        }
+    }
+    __syncthreads();
+
+    v4f acc[kBlocks][kGroups];
+    float norm[kBlocks];
+    int norm_codes[kBlocks];
+    // Consumes slot p (piece `piece`) half by half and refills it with piece `next_piece` of the rows
+    // `next_row`. A half goes through the wavefront's 2 KB of LDS, which turns the loads' layout (8
+    // lanes per row, whole 128-byte lines) into the matrix core's (16 rows side by side); slot c ^
+    // (row / 2 % 8) of a row's 128 bytes keeps both sides free of bank conflicts. One wavefront's LDS
+    // operations run in order, so neither side waits for more than its data.
+    std::uint8_t* stage = lds_stage[wave];
+    const int write_at = (lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 4) & 3)) * 16);
+    auto multiplyPiece = [&](int p, int piece, const std::uint32_t (&next_row)[kBlocks][2],
+                             int next_piece) __attribute__((always_inline)) {
+        // (a piece past the end of a row of several rounds is cleared whole: any operands do)
+        const v8h* operands = reinterpret_cast<const v8h*>(lds_operands) +
+                              static_cast<std::size_t>(min(piece * kSteps, steps - kSteps)) * kWave + lane;
+        const int group_stride = steps * kWave;
+        auto product = [&](int step, const v8h (&x)[kBlocks]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) {
+                const v8h q = operands[g * group_stride + step * kWave];
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    acc[b][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(q, x[b], acc[b][g], 0, 0, 0);
+                }
+            }
+        };
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int half_at = piece * kPieceBytes + half * (kPieceBytes / 2);
+            const bool clip = half_at + kPieceBytes / 2 > row_bytes;  // (uniform)
+            if (p == kPieces - 1 && half_at >= row_bytes) {  // (a row's last slot may be half or wholly empty)
+                issue(next_row, p, next_piece, half);
+                continue;
+            }
+            v4u chunk[kBlocks][2];  // chunks 8 half + 4 i + h of this lane's row
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    v4u raw = ring[p][b][half][i];
+                    if (clip) {  // bytes that repeat earlier ones
+                        raw = keepFrom(raw, min(16, max(0, half_at + 16 * (lane & 7) - last_chunk)));
+                    }
+                    // (row 8 i + lane / 8: its swizzle has the bit 8 i / 2 = 4 i on top of the lane's)
+                    *reinterpret_cast<v4u*>(stage + i * 1024 + (write_at ^ (64 * i))) = raw;
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    chunk[b][i] = *reinterpret_cast<const v4u*>(stage + r16 * 128 + (((4 * i + h) ^ (r16 >> 1)) * 16));
+                }
+            }
+            issue(next_row, p, next_piece, half);
+            if constexpr (kF32) {
+                v8h x[kBlocks];
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    v4u halves;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        float f[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            f[e] = __uint_as_float(chunk[b][i][e]) * inverse_unit;
+                            norm[b] = fmaf(f[e], f[e], norm[b]);
+                        }
+                        halves[2 * i] = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(f[0], f[1]));
+                        halves[2 * i + 1] = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(f[2], f[3]));
+                    }
+                    x[b] = __builtin_bit_cast(v8h, halves);
+                }
+                product(half, x);
+            } else if constexpr (kF16) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    v8h x[kBlocks];
+#pragma unroll
+                    for (int b = 0; b < kBlocks; ++b) {
+                        x[b] = __builtin_bit_cast(v8h, chunk[b][i]);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            const unsigned int word = chunk[b][i][w];  // (a value of its own: a bit cast of the
+                            const v2h pair = __builtin_bit_cast(v2h, word);  // element yields element 0)
+                            norm[b] = __builtin_amdgcn_fdot2(pair, pair, norm[b], false);
+                        }
+                    }
+                    product(2 * half + i, x);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                    for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            norm_codes[b] = __builtin_amdgcn_sdot4(static_cast<int>(chunk[b][i][w]), static_cast<int>(chunk[b][i][w]),
+                                                                   norm_codes[b], false);
+                        }
+                    }
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        v8h x[kBlocks];
+#pragma unroll
+                        for (int b = 0; b < kBlocks; ++b) {
+                            // code c as the half 1024 + (c + 128) (its byte under 0x64), less 1152
+                            v4u halves;
+#pragma unroll
+                            for (int w = 0; w < 2; ++w) {
+                                const unsigned int biased = chunk[b][i][2 * s + w] ^ 0x80808080u;
+                                const v2h offset = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
+                                const v2h lo =
+                                    __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, biased, 0x04010400u)) + offset;
+                                const v2h hi =
+                                    __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, biased, 0x04030402u)) + offset;
+                                halves[2 * w] = __builtin_bit_cast(unsigned int, lo);
+                                halves[2 * w + 1] = __builtin_bit_cast(unsigned int, hi);
+                            }
+                            x[b] = __builtin_bit_cast(v8h, halves);
+                        }
+                        product(4 * half + 2 * i + s, x);
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // ---- exact scores, a row per group of lanes_per_row lanes ----
+    // The pair (row as listed, query of the launch) of this lane's group; `take` clear: no pair.
+    auto scorePair = [&](std::uint32_t listed, int q, bool take) __attribute__((always_inline)) {
+        const std::uint32_t row = listed & ~kMaskedRow;
+        const int query = min(q_offset + q, scan.batch - 1);  // (a query past the batch parks NaN pairs only)
+        float score = exactScore<kKind>(scan, row, query, lane, lanes_per_row);
+        if (args.infinite_as_nan != 0 && scan.batch - query / 128 * 128 >= 32 && fabsf(score) == INFINITY) {
+            score = __uint_as_float(0x7FC00000u);
+        }
+        const std::uint64_t key = makeKey((listed & kMaskedRow) != 0u ? kMaskedScore : score, row);
+        if (take && lane % lanes_per_row == 0 && key > lds_tau[q]) {
+            const std::uint32_t slot = atomicAdd(&lds_count[q], 1u);
+            if (slot < (1u << emit.seg_log2)) {
+                emit.seg[((static_cast<std::size_t>(blockIdx.x) * scan.batch + q_offset + q) << emit.seg_log2) + slot] = key;
+            }
+            // Once the workgroup holds `width` keys of a query, no key below the lowest of them can be
+            // selected any more: rows that tie by the thousand (copies of one row) stop filling the
+            // segment.
+            if (slot < static_cast<std::uint32_t>(args.width)) {
+                atomicMin(&lds_lowest[q], key);
+                if (atomicAdd(&lds_placed[q], 1u) + 1u == static_cast<std::uint32_t>(args.width)) {
+                    lds_tau[q] = max(lds_tau[q], lds_lowest[q]);
+                }
+            }
+        }
+    };
+    const int per_round = kWave / lanes_per_row;
+
+    float best[kGroups * 4];  // sketch
+#pragma unroll
+    for (int i = 0; i < kGroups * 4; ++i) {
+        best[i] = -INFINITY;
+    }
+    std::uint32_t parked = 0u;  // pairs that wait for their exact score (uniform)
+    // The stream runs until its surviving pairs fill the wavefront's park, which is then scored with
+    // the stream's registers free; a tile whose pairs do not fit (or would not even an empty park) is
+    // streamed again (scored whole) after it.
+    bool crowded = false;
+    while (tile < tiles) {
+        while (tile < tiles) {
+            const long long next = tile + waves;
+            std::uint32_t id[kBlocks];  // this lane's rows in the results
+            std::uint32_t next_row[kBlocks][2];
+            readRows(next, next_row);
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                id[b] = entryOf(tile, kFilterBlockRows * b + r16);
+                norm[b] = 0.0f;
+                norm_codes[b] = 0;
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    acc[b][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+            }
+            for (int round = 0; round < rounds; ++round) {
+                const bool last = round + 1 == rounds;
+                std::uint32_t refill_row[kBlocks][2];
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    refill_row[b][0] = last ? next_row[b][0] : row[b][0];
+                    refill_row[b][1] = last ? next_row[b][1] : row[b][1];
+                }
+                const int refill_piece = last ? 0 : (round + 1) * kPieces;
+#pragma unroll
+                for (int p = 0; p < kPieces; ++p) {
+                    multiplyPiece(p, round * kPieces + p, refill_row, refill_piece + p);
+                }
+            }
+
+            // ---- the tile's scores (the thresholds are read again for every tile: kept, they would
+            //      take the accumulators' registers) ----
+            asm volatile("" ::: "memory");
+            float term[kBlocks];
+            bool live[kBlocks];
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                float n2 = kF32 || kF16 ? norm[b] : static_cast<float>(norm_codes[b]);
+                n2 += waveXor(n2, 16);
+                n2 += waveXor(n2, 32);
+                term[b] = l2 ? n2 : sqrtf(n2) * 1.00001f;
+                live[b] = id[b] != kNoRow;
+                if (list != nullptr && (id[b] & kMaskedRow) != 0u) {
+                    term[b] = 0.0f;  // a masked row passes only where everything passes
+#pragma unroll
+                    for (int g = 0; g < kGroups; ++g) {
+                        acc[b][g] = v4f{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+                    }
+                }
+            }
+            if (sketch) {
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    const v4f gain = *reinterpret_cast<const v4f*>(&lds_gain[kFilterGroup * g + 4 * h]);
+                    const v4f slope = *reinterpret_cast<const v4f*>(&lds_slope[kFilterGroup * g + 4 * h]);
+                    const v4f offset = *reinterpret_cast<const v4f*>(&lds_base[kFilterGroup * g + 4 * h]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float bound = fmaf(gain[i], acc[0][g][i], fmaf(slope[i], term[0], offset[i]));
+                        // (an infinite or NaN bound is none)
+                        best[4 * g + i] = live[0] && bound < 3.0e38f ? fmaxf(best[4 * g + i], bound) : best[4 * g + i];
+                    }
+                }
+            } else {
+                bool any = false;
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    const v4f slope = *reinterpret_cast<const v4f*>(&lds_slope[kFilterGroup * g + 4 * h]);
+                    const v4f offset = *reinterpret_cast<const v4f*>(&lds_base[kFilterGroup * g + 4 * h]);
+#pragma unroll
+                    for (int b = 0; b < kBlocks; ++b) {
+                        bool here = false;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            here |= !(acc[b][g][i] < fmaf(slope[i], term[b], offset[i]));
+                        }
+                        any |= here && live[b];
+                    }
+                }
+                if (__any(any)) {
+                    // bit 4 b + i of survivors[g]: block b's row and query 16 g + 4 h + i (the opaque copies
+                    // keep the thresholds above from being kept for here)
+#pragma unroll
+                    for (int b = 0; b < kBlocks; ++b) {
+                        asm volatile("" : "+v"(term[b]));
+                    }
+                    std::uint32_t survivors[kGroups];
+#pragma unroll
+                    for (int g = 0; g < kGroups; ++g) {
+                        const v4f slope = *reinterpret_cast<const v4f*>(&lds_slope[kFilterGroup * g + 4 * h]);
+                        const v4f offset = *reinterpret_cast<const v4f*>(&lds_base[kFilterGroup * g + 4 * h]);
+                        survivors[g] = 0u;
+#pragma unroll
+                        for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                if (live[b] && !(acc[b][g][i] < fmaf(slope[i], term[b], offset[i]))) {
+                                    survivors[g] |= 1u << (4 * b + i);
+                                }
+                            }
+                        }
+                    }
+                    int own = 0;
+#pragma unroll
+                    for (int g = 0; g < kGroups; ++g) {
+                        own += __popc(survivors[g]);
+                    }
+                    const std::uint32_t found = __builtin_amdgcn_readlane(waveInclusiveSum(static_cast<std::uint32_t>(own)), kWave - 1);
+                    if (parked + found > static_cast<std::uint32_t>(kParkSlots)) {
+                        crowded = found > static_cast<std::uint32_t>(kParkSlots);
+                        break;
+                    }
+#pragma unroll 1
+                    for (int g = 0; g < kGroups; ++g) {
+                        std::uint32_t word = survivors[0];
+#pragma unroll
+                        for (int other = 1; other < kGroups; ++other) {
+                            word = g == other ? survivors[other] : word;  // (registers have no index)
+                        }
+                        while (__any(word != 0u)) {
+                            const bool mine = word != 0u;
+                            const unsigned long long who = __ballot(mine);
+                            if (mine) {
+                                const int bit = __ffs(word) - 1;
+                                word &= word - 1u;
+                                std::uint32_t row = id[0];
+#pragma unroll
+                                for (int b = 1; b < kBlocks; ++b) {
+                                    row = (bit >> 2) == b ? id[b] : row;
+                                }
+                                const std::uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                                    static_cast<std::uint32_t>(who >> 32),
+                                    __builtin_amdgcn_mbcnt_lo(static_cast<std::uint32_t>(who), 0u));
+                                lds_park[wave][parked + below] =
+                                    make_uint2(row, static_cast<std::uint32_t>(kFilterGroup * g + 4 * h + (bit & 3)));
+                            }
+                            parked += static_cast<std::uint32_t>(__popcll(who));
+                        }
+                    }
+                }
+            }
+            tile = next;
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                row[b][0] = next_row[b][0];
+                row[b][1] = next_row[b][1];
+            }
+        }
+        if (crowded) {
+            // every pair of the tile, its rows from the list or the tile's place
+            const int tile_rows = kBlocks * kFilterBlockRows;
+            for (int first = 0; first < tile_rows * q_count; first += per_round) {
+                const int pair = first + lane / lanes_per_row;
+                const long long at = tileAt(tile) * tile_rows + pair % tile_rows;
+                const bool take = pair < tile_rows * q_count && at < rows;
+                const long long place = min(at, rows - 1);
+                scorePair(list != nullptr ? list[place] : static_cast<std::uint32_t>(place),
+                          min(pair / tile_rows, q_count - 1), take);
+            }
+            crowded = false;
+            tile += waves;
+        }
+        for (std::uint32_t first = 0; first < parked; first += static_cast<std::uint32_t>(per_round)) {
+            const std::uint32_t e = first + static_cast<std::uint32_t>(lane / lanes_per_row);
+            const uint2 pair = lds_park[wave][min(e, parked - 1u)];
+            scorePair(pair.x, static_cast<int>(pair.y), e < parked);
+        }
+        parked = 0u;
+        readRows(tile, row);  // (past the last tile too: with a branch the ring would be kept across all this)
+        issueTile(row);
+    }
+    if (sketch) {
+        // one slot per wavefront: the best over its 16 row lanes
+#pragma unroll
+        for (int i = 0; i < kGroups * 4; ++i) {
+            float v = best[i];
+#pragma unroll
+            for (int x = 1; x < 16; x <<= 1) {
+                v = fmaxf(v, waveXor(v, x));
+            }
+            const int q = kFilterGroup * (i / 4) + 4 * h + (i & 3);
+            if (r16 == 0 && q < q_count) {
+                emit.sketch[static_cast<std::size_t>(blockIdx.x * kFilterWaves + wave) * scan.batch + q_offset + q] = v;
+            }
+        }
+    } else {
+        __syncthreads();
+        for (int i = tid; i < q_count; i += kFilterThreads) {
+            emit.seg_count[static_cast<std::size_t>(blockIdx.x) * scan.batch + q_offset + i] = lds_count[i];
+        }
+    }
+}
+
+template <int kKind, int kPieces>
+int launchFilterPieces(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,
+                       int workgroups, hipStream_t stream) {
+    const int chunks = static_cast<int>((rowBytes(kKind, scan.dim) + 15) / 16);
+    // The lane groups of the VALU scan (a row of fewer chunks leaves lanes of its 8 at zero, which
+    // changes no sum), or a wavefront per row.
+    const int lanes = rowBytes(kKind, scan.dim) % 16 != 0 ? kWave
+                      : lanesPerRow(chunks, 8, 8) < 8     ? 8
+                                                          : lanesPerRow(chunks, 8, 8);
+    const dim3 grid(static_cast<unsigned>(workgroups));
+    const int per_launch = args.groups_per_launch * kFilterGroup;
+    for (int q0 = 0; q0 < scan.batch; q0 += per_launch) {
+        const int count = scan.batch - q0 < per_launch ? scan.batch - q0 : per_launch;
+        switch (args.groups_per_launch) {
+            case 1: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 1), 1><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
+            case 2: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 2), 2><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
+            case 4: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 4), 4><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
+            default: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 8), 8><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
+        }
+        ZCGVS_LAUNCH_CHECK("filter scan");
+    }
+    return ZCGVS_OK;
+}
+
+}  // namespace
+
+// The filter scan of rows of one or two pieces (kWide clear) or more; filterSlots(pieces) of them
+// are in flight.
+template <int kKind, bool kWide>
+int launchFilterKind(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,
+                     int workgroups, hipStream_t stream) {
+    const int slots = filterSlots(static_cast<int>((rowBytes(kKind, scan.dim) + kPieceBytes - 1) / kPieceBytes));
+    if constexpr (kWide) {
+        return slots == 3 ? launchFilterPieces<kKind, 3>(scan, args, phase, emit, workgroups, stream)
+                          : launchFilterPieces<kKind, 4>(scan, args, phase, emit, workgroups, stream);
+    } else {
+        return slots == 1 ? launchFilterPieces<kKind, 1>(scan, args, phase, emit, workgroups, stream)
+                          : launchFilterPieces<kKind, 2>(scan, args, phase, emit, workgroups, stream);
+    }
+}
+
+}  // namespace zcgvs_hip

@@ -434,7 +434,7 @@ __device__ __forceinline__ bool mergeQuery(const MergeInputs& in, int k, int bat
     __syncthreads();  // lds_kth and the threshold written above
     if (t == 0) {
         if (threshold != nullptr && taken < static_cast<std::uint32_t>(k)) {
-            threshold[q] = 0ull;
+            threshold[q] = in.fallback_tau != nullptr ? in.fallback_tau[q] : 0ull;
         }
         if (in.final_merge) {
             const bool earlier = !in.reset_overflow && overflow[q] != 0u;

@@ -230,7 +230,9 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
     const int group = lane % L;
     constexpr int kRowsPerPass = kRecoverThreads / L;
     constexpr int kPer = kRecoverChunksPerLane;
-    const std::size_t row_bytes = static_cast<std::size_t>(chunks) * 16;
+    const std::size_t row_bytes = rowBytes(scan.dtype, dim);
+    // rows of no whole 16-byte chunks: one wavefront per row, summed as the launchers' scalar scan
+    const bool strided = row_bytes % 16 != 0;
     const std::uint8_t* corpus = static_cast<const std::uint8_t*>(scan.corpus);
     const bool l2 = scan.metric == ZCGVS_METRIC_L2;
 
@@ -242,7 +244,7 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
         for (int i = 0; i < kPer; ++i) {
             const int c = group + i * L;
             raw[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (!masked && c < chunks) {
+            if (!masked && !strided && c < chunks) {
                 raw[i] = loadChunk(corpus + static_cast<std::size_t>(row) * row_bytes + static_cast<std::size_t>(c) * 16);
             }
         }
@@ -278,10 +280,18 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
             constexpr int E = Traits::kElems;
             const float* staged = reinterpret_cast<const float*>(lds_query);
             float acc = 0.0f;
+            if (strided && !masked) {
+                const std::uint8_t* values = corpus + static_cast<std::size_t>(row) * row_bytes;
+                for (int j = group; j < dim; j += L) {
+                    const float x = loadScalar<kKind>(values, j, scan.scale);
+                    const float d = l2 ? staged[j] - x : x;
+                    acc = fmaf(l2 ? d : staged[j], d, acc);
+                }
+            }
 #pragma unroll
             for (int i = 0; i < kPer; ++i) {
                 const int c = group + i * L;
-                if (c < chunks) {
+                if (!strided && c < chunks) {
                     float v[E];
                     Traits::decode(raw[i], scan.scale, v);
                     const float* qv = staged + c * E;
@@ -479,6 +489,13 @@ int kindOf(const ScanArgs& scan) {
     return scan.dtype;
 }
 
+// Lanes per row: the VALU scan's, or a whole wavefront for rows of no whole 16-byte chunks.
+int recoverLanes(const ScanArgs& scan) {
+    const std::size_t bytes = rowBytes(scan.dtype, scan.dim);
+    return bytes % 16 != 0 ? kWave
+                           : lanesPerRow(static_cast<int>(bytes / 16), kRecoverChunksPerLane, kRecoverMinLanes);
+}
+
 template <int kKind>
 int launchKind(int lanes, std::size_t shared, const ScanArgs& scan, const RecoverArgs& args, int chunks,
                hipStream_t stream) {
@@ -524,13 +541,14 @@ int launchMergeKind(int lanes, const MergeInputs& in, int k, int batch, std::uin
 
 bool recoverSupported(const ScanArgs& scan) {
     const std::size_t bytes = rowBytes(scan.dtype, scan.dim);
-    if (bytes % 16 != 0 || !aligned16(scan.corpus)) {
+    const bool whole = bytes % 16 == 0;
+    if ((!whole && (scan.dtype == ZCGVS_DTYPE_BINARY || kindOf(scan) == kKindI8I8)) || !aligned16(scan.corpus)) {
         return false;
     }
-    const int chunks = static_cast<int>(bytes / 16);
-    const int lanes = lanesPerRow(chunks, kRecoverChunksPerLane, kRecoverMinLanes);
+    const int chunks = static_cast<int>((bytes + 15) / 16);
+    const int lanes = recoverLanes(scan);
     const std::size_t staged = static_cast<std::size_t>(chunks) * stagedWordsPerChunk(kindOf(scan)) * 4;
-    return (chunks + lanes - 1) / lanes <= kRecoverChunksPerLane && staged <= 48 * 1024;
+    return (!whole || (chunks + lanes - 1) / lanes <= kRecoverChunksPerLane) && staged <= 48 * 1024;
 }
 
 int launchRecover(const ScanArgs& scan, const RecoverArgs& args, hipStream_t stream) {
@@ -540,8 +558,8 @@ int launchRecover(const ScanArgs& scan, const RecoverArgs& args, hipStream_t str
     if (!recoverSupported(scan)) {
         return setError(ZCGVS_ERR_RUNTIME, "zcgvs recovery: row layout not supported");
     }
-    const int chunks = static_cast<int>(rowBytes(scan.dtype, scan.dim) / 16);
-    const int lanes = lanesPerRow(chunks, kRecoverChunksPerLane, kRecoverMinLanes);
+    const int chunks = static_cast<int>((rowBytes(scan.dtype, scan.dim) + 15) / 16);
+    const int lanes = recoverLanes(scan);
     const int kind = kindOf(scan);
     const std::size_t shared = static_cast<std::size_t>(chunks) * stagedWordsPerChunk(kind) * 4;
     switch (kind) {
@@ -567,8 +585,8 @@ int launchMergeRecover(const MergeInputs& in, int k, int batch, std::uint64_t* o
     if (!recoverSupported(scan)) {
         return setError(ZCGVS_ERR_RUNTIME, "zcgvs recovery: row layout not supported");
     }
-    const int chunks = static_cast<int>(rowBytes(scan.dtype, scan.dim) / 16);
-    const int lanes = lanesPerRow(chunks, kRecoverChunksPerLane, kRecoverMinLanes);
+    const int chunks = static_cast<int>((rowBytes(scan.dtype, scan.dim) + 15) / 16);
+    const int lanes = recoverLanes(scan);
     const int kind = kindOf(scan);
     // the staged query goes to the end of the merge's candidate LDS, before it the running list of
     // at least kMaxK keys and a step's rows

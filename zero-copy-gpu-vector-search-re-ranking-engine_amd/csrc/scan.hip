@@ -128,17 +128,6 @@ __global__ __launch_bounds__(kScanThreads) void scanStoreKernel(
 
 // ---- scalar path for rows that are not a whole number of 16-byte chunks ----------------------
 template <int kDtype>
-__device__ __forceinline__ float loadScalar(const std::uint8_t* row, int j, float scale) {
-    if constexpr (kDtype == ZCGVS_DTYPE_F32) {
-        return reinterpret_cast<const float*>(row)[j];
-    } else if constexpr (kDtype == ZCGVS_DTYPE_F16) {
-        return __half2float(reinterpret_cast<const __half*>(row)[j]);
-    } else {
-        return static_cast<float>(reinterpret_cast<const std::int8_t*>(row)[j]) * scale;
-    }
-}
-
-template <int kDtype>
 __global__ __launch_bounds__(kScanThreads) void scanScalarKernel(
     const std::uint8_t* __restrict__ corpus, int doc_count, int dim, std::size_t row_bytes,
     float scale, const float* __restrict__ queries, int batch,

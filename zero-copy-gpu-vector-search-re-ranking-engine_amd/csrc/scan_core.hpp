@@ -151,6 +151,18 @@ __device__ __forceinline__ T groupSum(T value) {
     return value;
 }
 
+// Component j of a stored row, for the scans of rows that are no whole number of 16-byte chunks.
+template <int kDtype>
+__device__ __forceinline__ float loadScalar(const std::uint8_t* row, int j, float scale) {
+    if constexpr (kDtype == ZCGVS_DTYPE_F32) {
+        return reinterpret_cast<const float*>(row)[j];
+    } else if constexpr (kDtype == ZCGVS_DTYPE_F16) {
+        return __half2float(reinterpret_cast<const __half*>(row)[j]);
+    } else {
+        return static_cast<float>(reinterpret_cast<const std::int8_t*>(row)[j]) * scale;
+    }
+}
+
 // Lanes per row for a row of `chunks` 16-byte chunks: the smallest power of two giving each
 // lane at most `per_lane` chunks, capped at a full wavefront, and at least min_lanes (or as
 // many as the row has chunks), so one load instruction reads whole cache lines of a row.

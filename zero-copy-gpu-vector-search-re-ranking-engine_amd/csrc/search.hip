@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "filter.hpp"
 #include "fused.hpp"
 #include "rescore.hpp"
 #include "select.hpp"
@@ -44,6 +45,7 @@ constexpr std::size_t kAlign = 256;
 // one threshold phase).
 constexpr long long kPhaseGrowth = 8;
 constexpr long long kCandidateBudget = 1LL << 18;
+constexpr long long kFilterMinRows = 1024;
 constexpr long long kMergeLdsKeys = 12288;  // candidate keys a query's merge gathers in LDS (topk.hip)
 
 std::size_t alignUp(std::size_t value) { return (value + kAlign - 1) / kAlign * kAlign; }
@@ -77,6 +79,9 @@ struct Plan {
     bool use_mfma = false;
     bool use_mfma_float = false;
     bool use_mfma_binary = false;
+    bool use_filter = false;     // filter scan (filter.hpp)
+    FilterShape filter;
+    PhaseArgs filter_sketch;     // its sketch, when that is no phase of its own (planFilter)
     bool direct_scales = false;  // MFMA path without a mask: only the tail tile's scales are copied
     bool lex_sorted = false;     // hybrid with postings ascending by document: sliced BM25 stage
     bool recover = false;        // threshold phases ran: the exact fallback follows them
@@ -106,7 +111,8 @@ struct Plan {
                 segcnt = 0, keys = 0, tau = 0, overflow = 0, rescored = 0, scores = 0, lexmat = 0,
                 topk_a = 0, topk_b = 0, topk_c = 0, topk_d = 0, cand_idx = 0, cand_val = 0, sp_level = 0,
                 local_idx = 0, rescore_val = 0, lexmax_m = 0, lexbounds = 0, sketchbuf = 0, tau_safe = 0,
-                flag_list = 0, flag_count = 0;
+                flag_list = 0, flag_count = 0, filter_operands = 0, filter_queries = 0, filter_unit = 0,
+                filter_list = 0, filter_count = 0;
     std::size_t total = 0;
 };
 
@@ -269,7 +275,133 @@ ScanArgs recoverArgsOf(const zcgvs_search_desc& d, const Plan& plan, std::uint8_
     return scan;
 }
 
-Plan makePlan(const zcgvs_search_desc& d) {
+// Workspace of zcgvs_search_topk_noalloc: one library-owned array per device, so a caller that
+// cannot allocate still runs the pipeline. Its size caps the searches that entry point accepts.
+constexpr std::size_t kStaticScratchBytes = std::size_t(64) << 20;
+
+FilterArgs filterArgsOf(const zcgvs_search_desc& d, const Plan& plan, std::uint8_t* ws) {
+    FilterArgs args;
+    args.operands = ws + plan.filter_operands;
+    args.queries = reinterpret_cast<FilterQuery*>(ws + plan.filter_queries);
+    args.row_unit = reinterpret_cast<float*>(ws + plan.filter_unit);
+    if (d.mask != nullptr) {
+        args.list = reinterpret_cast<std::uint32_t*>(ws + plan.filter_list);
+        args.list_count = reinterpret_cast<std::uint32_t*>(ws + plan.filter_count);
+    }
+    args.steps = plan.filter.steps;
+    args.groups = plan.filter.groups;
+    args.groups_per_launch = plan.filter.groups_per_launch;
+    args.width = plan.width;
+    args.infinite_as_nan = d.corpus.dtype == ZCGVS_DTYPE_F32 && d.mask == nullptr && d.metric != ZCGVS_METRIC_L2 &&
+                                   (d.corpus.dim == 256 || d.corpus.dim == 384)
+                               ? 1
+                               : 0;
+    return args;
+}
+
+// The filter scan's plan: a sketch over a sample of 16-row blocks finds a certain threshold (the
+// width-th best of its slots' best lower bounds), then one phase scans every row. Shapes the
+// float matrix-core scan also takes keep its partition of the corpus into threshold phases: the
+// sketch belongs to the launches of a first phase over every 8th tile, whose merge gives the exact
+// threshold of a second one over the rest. `layout` holds what precedes the scan's buffers.
+void planFilter(const zcgvs_search_desc& d, Plan& plan, Layout& layout) {
+    const long long n = d.corpus.doc_count;
+    const int batch = d.batch;
+    plan.workgroups = deviceComputeUnits();
+    plan.segments = plan.workgroups;
+    plan.block_rows = kFilterBlockRows;
+    plan.sketch = true;
+    plan.sketch_slots = kFilterSketchSlots * plan.workgroups;
+    plan.sketch_rank = plan.width;
+    const long long blocks = (n + kFilterBlockRows - 1) / kFilterBlockRows;
+    // A sample of f of the rows costs f of the scan and lets about width / f pairs per query through
+    // to be scored exactly, each at about twice the cost of a row in the stream: the sum is least near
+    // f = sqrt(2 * batch * width / n). The sample is a whole number of blocks per wavefront.
+    const double f = std::sqrt(2.0 * batch * plan.width / static_cast<double>(n));
+    const long long per_wave = std::max<long long>(1, std::llround(f * static_cast<double>(blocks) / plan.sketch_slots));
+    const long long wanted = std::min<long long>(blocks, per_wave * plan.sketch_slots);
+    PhaseArgs sketch;
+    sketch.stride = (blocks + wanted - 1) / wanted;
+    sketch.items = phaseItems(blocks, sketch.stride, 0);
+    sketch.sketch = 1;
+    sketch.block_rows = plan.block_rows;
+    plan.block_rows = plan.filter.tile_rows;
+    const long long tiles = (n + plan.block_rows - 1) / plan.block_rows;
+    PhaseArgs scan;
+    scan.block_rows = plan.block_rows;
+    scan.items = tiles;
+    if (plan.use_mfma_float) {
+        constexpr long long kFirst = 8;
+        scan.stride = kFirst;
+        scan.items = phaseItems(tiles, kFirst, 0);
+        PhaseArgs rest = scan;
+        rest.stride = 1;
+        rest.skip = kFirst;
+        rest.items = phaseItems(tiles, 1, kFirst);
+        plan.filter_sketch = sketch;
+        plan.phases = {scan, rest};
+    } else {
+        plan.phases = {sketch, scan};
+    }
+    plan.recover = true;
+    const long long expected = plan.width * sketch.stride / plan.segments;
+    plan.seg_log2 = std::max(6, ceilLog2(4 * expected + 16));
+    if ((d.flags & ZCGVS_SEARCH_TEST_TINY_SEGMENTS) != 0) {
+        plan.seg_log2 = 1;
+    }
+    plan.seg = layout.add((static_cast<std::size_t>(plan.segments) * batch << plan.seg_log2) * 8);
+    plan.segcnt = layout.add(static_cast<std::size_t>(plan.segments) * batch * 4);
+    plan.keys = layout.add(static_cast<std::size_t>(batch) * plan.width * 8);
+    plan.tau = layout.add(static_cast<std::size_t>(batch) * 8);
+    plan.tau_safe = layout.add(static_cast<std::size_t>(batch) * 8);
+    plan.flag_list = layout.add(static_cast<std::size_t>(batch) * 4);
+    plan.flag_count = layout.add(4);
+    plan.sketchbuf = layout.add(static_cast<std::size_t>(plan.sketch_slots) * batch * 4);
+    plan.filter_operands = layout.add(filterOperandBytes(plan.filter));
+    plan.filter_queries = layout.add(static_cast<std::size_t>(plan.filter.groups) * kFilterGroup * sizeof(FilterQuery));
+    plan.filter_unit = layout.add(4);
+    if (d.mask != nullptr) {
+        plan.filter_list = layout.add(filterListEntries(n) * 4);
+        plan.filter_count = layout.add(4);
+    }
+    if (plan.rescore) {
+        plan.rescored = layout.add(static_cast<std::size_t>(batch) * plan.width * 8);
+    }
+    plan.total = layout.total;
+}
+
+// Whether the filter scan is the fastest plan for a shape it takes. Its five launches cost 31 us
+// (and 0.4 per query group) before any row, so small searches keep the plans they had; the lines lie
+// where both measured the same (us, that plan against the filter scan).
+bool filterPays(const ScanArgs& scan, const Plan& plan) {
+    const long long n = scan.doc_count;
+    // (few rows: the sketch has a slot per 16 of them, and needs more slots than keys)
+    if (n < std::max<long long>(kFilterMinRows, 2LL * kFilterBlockRows * plan.width)) {
+        return false;
+    }
+    if (singlePassShape(scan, plan.width).supported) {
+        return false;  // a few queries: one launch that HBM bounds
+    }
+    const long long tiles = (scan.batch + 7) / 8;  // of the queries the VALU kernels take at a time
+    if (rowBytes(scan.dtype, scan.dim) % 16 != 0) {
+        // The materialized pipeline's scalar scan: 20,000 x 100 int8, 2 queries 26 against 33;
+        // 5,000 x 300 float16, 16 queries 31 / 31; 100,000 x 100 float16, 1 query 47 / 35.
+        return n * tiles * ((scan.dim + 63) / 64) >= 50'000;
+    }
+    if (plan.use_mfma_float) {
+        // Up to 8191 rows that scan is one dense phase (5,000 x 384 float32, 64 queries 26 against 42;
+        // 10,000 rows 47 / 42). Beyond, float16 rows and few queries time the same on both (1M x 384:
+        // float16, 16 queries 155 / 160, 64 queries 169 / 176; float32, 16 queries 278 / 282); float32
+        // batches, which that scan splits into six products, do not (64 queries 381 / 299, 128
+        // queries 575 / 329).
+        return n >= 8192 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32;
+    }
+    // The same line for the VALU scan's plan, or where its dense phase alone takes longer: float16
+    // 2,000 x 768, 5 queries 37 / 34, 16 queries 82 / 38; int8 2,000 x 384, 8 queries 30 / 35.
+    return n >= 8192 || tiles * scan.dim >= 640;
+}
+
+Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
     Plan plan = validate(d);
     if (plan.status != ZCGVS_OK) {
         return plan;
@@ -309,6 +441,21 @@ Plan makePlan(const zcgvs_search_desc& d) {
     if (plan.per_vector && plan.materialized && dim % 16 != 0) {
         return fail(ZCGVS_ERR_INVALID_ARGUMENT,
                     "zcgvs: per-vector int8 mode needs dim % 16 == 0 and a 16-byte aligned corpus");
+    }
+
+    if (!forced && allow_filter && !plan.hybrid && !plan.binary && !plan.per_vector) {
+        ScanArgs exact = probe;
+        exact.mask = d.mask;
+        plan.filter = filterShape(exact, plan.width);
+        plan.use_filter = plan.filter.supported && recoverSupported(exact) && filterPays(exact, plan);
+    }
+    if (plan.use_filter) {
+        Layout layout;
+        plan.overflow = layout.add(static_cast<std::size_t>(batch) * 4);
+        planFilter(d, plan, layout);
+        plan.materialized = plan.use_mfma_float = false;
+        // (a search that fits the no-allocation entry's scratch on another plan still does)
+        return plan.total <= kStaticScratchBytes ? plan : makePlan(d, false);
     }
 
     Layout layout;
@@ -656,10 +803,6 @@ __global__ void zeroWordsKernel(std::uint32_t* __restrict__ dst, std::size_t cou
     }
 }
 
-// Workspace of zcgvs_search_topk_noalloc: one library-owned array per device, so a caller that
-// cannot allocate still runs the pipeline. Its size caps the searches that entry point accepts.
-constexpr std::size_t kStaticScratchBytes = std::size_t(64) << 20;
-
 }  // namespace
 
 }  // namespace zcgvs_hip
@@ -930,6 +1073,14 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
             (plan.use_mfma_binary && !mfmaBinarySupported(scan))) {
             return setError(ZCGVS_ERR_INVALID_ARGUMENT, "zcgvs: corpus or queries are not 16-byte aligned");
         }
+        FilterArgs filter;
+        if (plan.use_filter) {
+            filter = filterArgsOf(d, plan, ws);
+            status = launchFilterPrepare(scan, filter, s);
+            if (status != ZCGVS_OK) {
+                return status;
+            }
+        }
         EmitArgs emit;
         emit.tau = at<std::uint64_t>(ws, plan.tau);
         emit.dense = at<std::uint64_t>(ws, plan.dense);
@@ -963,7 +1114,20 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
             if (timed) {
                 ZCGVS_HIP_RETURN(hipEventRecord(reinterpret_cast<hipEvent_t>(events[2 * p]), s));
             }
-            if (plan.use_mfma) {
+            const bool sketch_first = plan.use_filter && p == 0 && !phase.sketch;
+            if (sketch_first) {
+                status = launchFilterScan(scan, filter, plan.filter_sketch, emit, plan.workgroups, s);
+                if (status == ZCGVS_OK) {
+                    status = launchFilterThreshold(emit.sketch, plan.sketch_slots, batch, plan.width, tau,
+                                                   at<std::uint64_t>(ws, plan.tau_safe), flag_count, s);
+                }
+                if (status != ZCGVS_OK) {
+                    return status;
+                }
+            }
+            if (plan.use_filter) {
+                status = launchFilterScan(scan, filter, phase, emit, plan.workgroups, s);
+            } else if (plan.use_mfma) {
                 status = launchMfmaScan(scan, phase, emit, plan.workgroups, s);
             } else if (plan.use_mfma_float) {
                 status = launchMfmaFloatScan(scan, phase, emit, plan.workgroups, s);
@@ -981,8 +1145,12 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
             const bool last = p + 1 == plan.phases.size();
             if (phase.sketch) {
                 // the speculative threshold and the guaranteed one; clears the flagged list
-                status = launchSketchThreshold(emit.sketch, plan.sketch_slots, batch, plan.sketch_rank, plan.width,
-                                               tau, at<std::uint64_t>(ws, plan.tau_safe), flag_count, s);
+                std::uint64_t* tau_safe = at<std::uint64_t>(ws, plan.tau_safe);
+                status = plan.use_filter
+                             ? launchFilterThreshold(emit.sketch, plan.sketch_slots, batch, plan.width, tau, tau_safe,
+                                                     flag_count, s)
+                             : launchSketchThreshold(emit.sketch, plan.sketch_slots, batch, plan.sketch_rank, plan.width,
+                                                     tau, tau_safe, flag_count, s);
                 if (status != ZCGVS_OK) {
                     return status;
                 }
@@ -990,13 +1158,19 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
             }
             MergeInputs in;
             if (plan.sketch) {
-                // the one merge of the speculative scan
+                // the one merge of the speculative or the filter scan, or the merges of a filter scan in
+                // two phases, whose first leaves its threshold alone where it finds fewer keys than k
+                const bool first_scan = p == 0 || plan.phases[p - 1].sketch;
+                if (!first_scan) {
+                    in.prev = keys;
+                    in.k_prev = plan.width;
+                }
                 in.seg = emit.seg;
                 in.seg_count = emit.seg_count;
                 in.n_seg = plan.segments;
                 in.seg_log2 = plan.seg_log2;
-                in.reset_overflow = true;
-                in.require_full = true;
+                in.reset_overflow = first_scan;
+                in.require_full = last;
                 in.fallback_tau = at<std::uint64_t>(ws, plan.tau_safe);
             } else if (p == 0) {
                 in.dense = emit.dense;
