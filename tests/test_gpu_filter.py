@@ -151,3 +151,31 @@ def test_overflowing_segments_fall_back(gpu, kind, dim, metric):
     assert np.array_equal(idx, plain[0]) and np.array_equal(val, plain[1])
     assert_topk_equivalent(idx, val, oracle.scores_f32(decoded, queries, metric, mask), k,
                            float_tolerance(queries, decoded, metric))
+
+
+# per-vector int8 at row widths the int8 matrix-core scan does not take, with masks, and small batches
+@pytest.mark.parametrize("n,dim,batch,k,share", [
+    (9_001, 16, 6, 10, None),       # one chunk
+    (20_011, 272, 33, 10, None),    # a chunk past a piece
+    (20_011, 640, 130, 100, 0.5),   # two launches
+    (9_001, 1008, 17, 50, 0.0),     # fewer rows than k
+    (20_011, 768, 128, 10, 0.3),
+    (100_003, 768, 5, 10, None),
+])
+def test_per_vector_int8_bit_exact(gpu, n, dim, batch, k, share):
+    capi = gpu
+    codes, scales = oracle.quantize_rows_i8(normalized(n, dim, 500 + dim))
+    queries = normalized(batch, dim, 501)
+    mask = None
+    if share is not None:
+        mask = (np.random.default_rng(dim).random(n) < share).astype(np.uint8)
+        mask[[3, n - 1]] = 1
+    d_codes, d_scales, d_queries = (capi.DeviceArray.from_host(a) for a in (codes, scales, queries))
+    d_mask = None if mask is None else capi.DeviceArray.from_host(mask)
+    desc = capi.search_desc(capi.store_desc(d_codes, n, dim, capi.I8, 1.0, d_scales), d_queries, batch, k, capi.COSINE,
+                            mask=d_mask, int8_mode=capi.INT8_PER_VECTOR)
+    idx, val, flags = capi.search(desc)
+    qcodes, qscales = oracle.quantize_rows_i8(queries)
+    ref_idx, ref_val = oracle.topk(oracle.scores_i8i8(codes, scales, qcodes, qscales, mask), k)
+    assert not flags.any()
+    assert np.array_equal(idx, ref_idx) and np.array_equal(val, ref_val)

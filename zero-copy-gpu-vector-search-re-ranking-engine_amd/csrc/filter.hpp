@@ -1,5 +1,6 @@
 // Filter scan (filter_scan.hip): float32, float16 and matrix-scale int8 corpora of any row width,
-// cosine, dot or L2, with or without an allow-mask, against a batch of float32 queries.
+// cosine, dot or L2, with or without an allow-mask, against a batch of float32 queries; and
+// per-vector int8 corpora against int8 queries.
 //
 // Each (row, query) pair first gets an approximate score from the matrix cores, rounded to
 // float16 operands, with a bound on its distance from the exact score; only pairs whose
@@ -12,6 +13,11 @@
 #include "fused.hpp"
 
 namespace zcgvs_hip {
+
+constexpr int kFilterPerVector = 4;  // scan kind beside the zcgvs_dtype ones: per-vector int8
+inline int filterKind(const ScanArgs& scan) {
+    return scan.dtype == ZCGVS_DTYPE_I8 && scan.row_scales != nullptr ? kFilterPerVector : scan.dtype;
+}
 
 // Queries are prepared per 16 (a query group): float16 matrix-core operands and FilterQuery
 // constants. Rows are read in 256-byte pieces, kFilterSteps(kind) 32-dimension products each.
@@ -34,7 +40,7 @@ constexpr int filterBlocks(int slots, int groups) {
 }
 
 struct FilterQuery {
-    float scale;  // the power of two the operands were multiplied by
+    float scale;  // the power of two the operands were multiplied by; per-vector int8: the query's scale
     float norm2;  // sum q_j^2
     float usable; // 0: not finite or out of range, every pair is scored exactly
     float pad;

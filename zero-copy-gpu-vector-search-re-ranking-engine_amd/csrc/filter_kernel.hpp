@@ -44,6 +44,7 @@ namespace zcgvs_hip {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef int v4i __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
@@ -59,8 +60,18 @@ constexpr int kParkSlots = 160;  // pairs a wavefront parks
 
 template <int kKind>
 struct FilterKind {
-    static constexpr int kElems = elementsPerChunk(kKind);
-    static constexpr int kSteps = kKind == ZCGVS_DTYPE_F32 ? 2 : kKind == ZCGVS_DTYPE_F16 ? 4 : 8;  // per piece
+    static constexpr bool kInteger = kKind == kFilterPerVector;
+    static constexpr int kDtype = kInteger ? ZCGVS_DTYPE_I8 : kKind;
+    // products of 32 components (64 of int8 by int8) per piece
+    static constexpr int kSteps = kKind == ZCGVS_DTYPE_F32 ? 2 : kKind == ZCGVS_DTYPE_I8 ? 8 : 4;
+};
+template <bool kInteger>
+struct FilterSums {
+    typedef v4f type;
+};
+template <>
+struct FilterSums<true> {
+    typedef v4i type;
 };
 
 // Relative error of an approximate dot product, in units of |q| |x|: operand rounding (float16
@@ -170,8 +181,45 @@ __device__ __forceinline__ float exactScoreStrided(const ScanArgs& scan, std::ui
     return l2 ? -total : total;
 }
 
+// The exact per-vector int8 score, (float)(integer dot) * (query scale * row scale).
+template <int L>
+__device__ __forceinline__ float exactScorePerVector(const ScanArgs& scan, std::uint32_t row, int q, int lane) {
+    constexpr int kPer = 8;
+    const int dim = scan.dim;
+    const int chunks = dim / 16;
+    const std::uint8_t* codes = static_cast<const std::uint8_t*>(scan.corpus) + static_cast<std::size_t>(row) * dim;
+    const std::uint8_t* query = static_cast<const std::uint8_t*>(scan.queries) + static_cast<std::size_t>(q) * dim;
+    const float scale = scan.row_scales[row];
+    int group = lane % L;
+    asm volatile("" : "+v"(group));
+    v4u raw[kPer], qe[kPer];
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+        if (t * L < chunks) {  // (uniform)
+            const int at = min(group + t * L, chunks - 1) * 16;
+            raw[t] = loadRowChunk<false>(codes + at);
+            qe[t] = loadRowChunk<false>(query + at);
+        }
+    }
+    int acc = 0;
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+        if (group + t * L < chunks) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                acc = __builtin_amdgcn_sdot4(static_cast<int>(raw[t][w]), static_cast<int>(qe[t][w]), acc, false);
+            }
+        }
+    }
+    const float combined = scan.query_scales[q] * scale;
+    return static_cast<float>(groupSum<L>(acc)) * combined;
+}
+
 template <int kKind>
 __device__ __forceinline__ float exactScore(const ScanArgs& scan, std::uint32_t row, int q, int lane, int lanes) {
+    if constexpr (kKind == kFilterPerVector) {
+        return lanes == 8 ? exactScorePerVector<8>(scan, row, q, lane) : exactScorePerVector<32>(scan, row, q, lane);
+    } else
     switch (lanes) {  // (uniform)
         case 8: return exactScoreLanes<kKind, 8>(scan, row, q, lane);
         case 16: return exactScoreLanes<kKind, 16>(scan, row, q, lane);
@@ -190,6 +238,9 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     constexpr int kQueries = kGroups * kFilterGroup;
     constexpr bool kF32 = kKind == ZCGVS_DTYPE_F32;
     constexpr bool kF16 = kKind == ZCGVS_DTYPE_F16;
+    constexpr bool kInteger = FilterKind<kKind>::kInteger;
+    constexpr int kDtype = FilterKind<kKind>::kDtype;
+    typedef typename FilterSums<kInteger>::type Sums;
 
     __shared__ __attribute__((aligned(16))) std::uint8_t lds_operands[kFilterOperandBytes];
     __shared__ __attribute__((aligned(16))) float lds_slope[kQueries];  // threshold = slope * row term + base
@@ -209,7 +260,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     const int r16 = lane & 15;
     const int h = lane >> 4;
     const int dim = scan.dim;
-    const int row_bytes = static_cast<int>(rowBytes(kKind, dim));
+    const int row_bytes = static_cast<int>(rowBytes(kDtype, dim));
     const int rounds = (row_bytes + kPieces * kPieceBytes - 1) / (kPieces * kPieceBytes);
     const int steps = args.steps;
     const bool l2 = scan.metric == ZCGVS_METRIC_L2;
@@ -315,7 +366,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             dst[i] = src[i];
         }
     }
-    const float unit = kF32 ? *args.row_unit : kF16 ? 1.0f : scan.scale;  // stored value = unit * operand
+    const float unit = kF32 ? *args.row_unit : kF16 || kInteger ? 1.0f : scan.scale;  // stored value = unit * operand
     const float inverse_unit = kF32 ? 1.0f / unit : 1.0f;                 // (float32: a power of two)
     const float relative = filterRelative(kKind, steps);
     // Absolute part, in operand units per |q|: float32 rows below float16's smallest normal lose up
@@ -327,7 +378,19 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         const bool valid = i < q_count;
         const FilterQuery query = args.queries[q_offset + i];
         const float qnorm = sqrtf(query.norm2) * 1.00001f;
-        if (sketch) {
+        if constexpr (kInteger) {
+            // score = acc * (query scale * row scale), compared with the threshold's itself
+            bool gated = false;
+            const std::uint64_t tau = valid && !sketch ? emit.tau[q_offset + i] : ~0ull;
+            const float floor_score = keyFloor(tau, &gated);
+            lds_gain[i] = valid ? query.scale : __uint_as_float(0x7FC00000u);
+            lds_slope[i] = query.scale;
+            lds_base[i] = !valid ? INFINITY : gated && floor_score > kMaskedScore ? floor_score : -INFINITY;
+            lds_tau[i] = tau;
+            lds_count[i] = 0u;
+            lds_lowest[i] = ~0ull;
+            lds_placed[i] = 0u;
+        } else if (sketch) {
             // lower bound = gain * acc + slope * row term + base
             float gain = unit / query.scale;
             float slope = -relative * qnorm * unit;
@@ -367,7 +430,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     }
     __syncthreads();
 
-    v4f acc[kBlocks][kGroups];
+    Sums acc[kBlocks][kGroups];
     float norm[kBlocks];
     int norm_codes[kBlocks];
     // Consumes slot p (piece `piece`) half by half and refills it with piece `next_piece` of the rows
@@ -389,7 +452,12 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 const v8h q = operands[g * group_stride + step * kWave];
 #pragma unroll
                 for (int b = 0; b < kBlocks; ++b) {
-                    acc[b][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(q, x[b], acc[b][g], 0, 0, 0);
+                    if constexpr (kInteger) {
+                        acc[b][g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, q),
+                                                                          __builtin_bit_cast(v4i, x[b]), acc[b][g], 0, 0, 0);
+                    } else {
+                        acc[b][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(q, x[b], acc[b][g], 0, 0, 0);
+                    }
                 }
             }
         };
@@ -438,7 +506,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                     x[b] = __builtin_bit_cast(v8h, halves);
                 }
                 product(half, x);
-            } else if constexpr (kF16) {
+            } else if constexpr (kF16 || kInteger) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     v8h x[kBlocks];
@@ -446,7 +514,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                     for (int b = 0; b < kBlocks; ++b) {
                         x[b] = __builtin_bit_cast(v8h, chunk[b][i]);
 #pragma unroll
-                        for (int w = 0; w < 4; ++w) {
+                        for (int w = 0; w < (kInteger ? 0 : 4); ++w) {
                             const unsigned int word = chunk[b][i][w];  // (a value of its own: a bit cast of the
                             const v2h pair = __builtin_bit_cast(v2h, word);  // element yields element 0)
                             norm[b] = __builtin_amdgcn_fdot2(pair, pair, norm[b], false);
@@ -535,16 +603,18 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         while (tile < tiles) {
             const long long next = tile + waves;
             std::uint32_t id[kBlocks];  // this lane's rows in the results
+            float row_scale[kBlocks];
             std::uint32_t next_row[kBlocks][2];
             readRows(next, next_row);
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) {
                 id[b] = entryOf(tile, kFilterBlockRows * b + r16);
+                row_scale[b] = kInteger ? scan.row_scales[id[b] == kNoRow ? 0u : id[b] & ~kMaskedRow] : 0.0f;
                 norm[b] = 0.0f;
                 norm_codes[b] = 0;
 #pragma unroll
                 for (int g = 0; g < kGroups; ++g) {
-                    acc[b][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+                    acc[b][g] = Sums{0, 0, 0, 0};
                 }
             }
             for (int round = 0; round < rounds; ++round) {
@@ -566,22 +636,31 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             //      take the accumulators' registers) ----
             asm volatile("" ::: "memory");
             float term[kBlocks];
-            bool live[kBlocks];
+            bool live[kBlocks], masked[kBlocks];
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) {
-                float n2 = kF32 || kF16 ? norm[b] : static_cast<float>(norm_codes[b]);
-                n2 += waveXor(n2, 16);
-                n2 += waveXor(n2, 32);
-                term[b] = l2 ? n2 : sqrtf(n2) * 1.00001f;
-                live[b] = id[b] != kNoRow;
-                if (list != nullptr && (id[b] & kMaskedRow) != 0u) {
-                    term[b] = 0.0f;  // a masked row passes only where everything passes
-#pragma unroll
-                    for (int g = 0; g < kGroups; ++g) {
-                        acc[b][g] = v4f{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-                    }
+                if constexpr (kInteger) {
+                    term[b] = row_scale[b];
+                } else {
+                    float n2 = kF32 || kF16 ? norm[b] : static_cast<float>(norm_codes[b]);
+                    n2 += waveXor(n2, 16);
+                    n2 += waveXor(n2, 32);
+                    term[b] = l2 ? n2 : sqrtf(n2) * 1.00001f;
                 }
+                live[b] = id[b] != kNoRow;
+                masked[b] = list != nullptr && (id[b] & kMaskedRow) != 0u;
             }
+            // Whether the pair of block b's row and query 16 g + 4 h + i can reach the query's threshold.
+            // (A masked row does where every row does; a NaN survives.)
+            auto survives = [&](int b, int g, int i, const v4f& slope, const v4f& offset) __attribute__((always_inline)) -> bool {
+                if constexpr (kInteger) {
+                    const float score = static_cast<float>(acc[b][g][i]) * (slope[i] * term[b]);
+                    return masked[b] ? offset[i] == -INFINITY : !(score < offset[i]);
+                } else {
+                    const float sum = masked[b] ? -INFINITY : acc[b][g][i];
+                    return !(sum < fmaf(slope[i], masked[b] ? 0.0f : term[b], offset[i]));
+                }
+            };
             if (sketch) {
 #pragma unroll
                 for (int g = 0; g < kGroups; ++g) {
@@ -590,9 +669,14 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                     const v4f offset = *reinterpret_cast<const v4f*>(&lds_base[kFilterGroup * g + 4 * h]);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const float bound = fmaf(gain[i], acc[0][g][i], fmaf(slope[i], term[0], offset[i]));
+                        float bound;
+                        if constexpr (kInteger) {
+                            bound = static_cast<float>(acc[0][g][i]) * (gain[i] * term[0]);
+                        } else {
+                            bound = fmaf(gain[i], acc[0][g][i], fmaf(slope[i], term[0], offset[i]));
+                        }
                         // (an infinite or NaN bound is none)
-                        best[4 * g + i] = live[0] && bound < 3.0e38f ? fmaxf(best[4 * g + i], bound) : best[4 * g + i];
+                        best[4 * g + i] = live[0] && !masked[0] && bound < 3.0e38f ? fmaxf(best[4 * g + i], bound) : best[4 * g + i];
                     }
                 }
             } else {
@@ -606,7 +690,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                         bool here = false;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            here |= !(acc[b][g][i] < fmaf(slope[i], term[b], offset[i]));
+                            here |= survives(b, g, i, slope, offset);
                         }
                         any |= here && live[b];
                     }
@@ -628,7 +712,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                         for (int b = 0; b < kBlocks; ++b) {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
-                                if (live[b] && !(acc[b][g][i] < fmaf(slope[i], term[b], offset[i]))) {
+                                if (live[b] && survives(b, g, i, slope, offset)) {
                                     survivors[g] |= 1u << (4 * b + i);
                                 }
                             }
@@ -728,10 +812,11 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
 template <int kKind, int kPieces>
 int launchFilterPieces(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,
                        int workgroups, hipStream_t stream) {
-    const int chunks = static_cast<int>((rowBytes(kKind, scan.dim) + 15) / 16);
+    constexpr int kDtype = FilterKind<kKind>::kDtype;
+    const int chunks = static_cast<int>((rowBytes(kDtype, scan.dim) + 15) / 16);
     // The lane groups of the VALU scan (a row of fewer chunks leaves lanes of its 8 at zero, which
     // changes no sum), or a wavefront per row.
-    const int lanes = rowBytes(kKind, scan.dim) % 16 != 0 ? kWave
+    const int lanes = rowBytes(kDtype, scan.dim) % 16 != 0 ? kWave
                       : lanesPerRow(chunks, 8, 8) < 8     ? 8
                                                           : lanesPerRow(chunks, 8, 8);
     const dim3 grid(static_cast<unsigned>(workgroups));
@@ -756,7 +841,7 @@ int launchFilterPieces(const ScanArgs& scan, const FilterArgs& args, const Phase
 template <int kKind, bool kWide>
 int launchFilterKind(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,
                      int workgroups, hipStream_t stream) {
-    const int slots = filterSlots(static_cast<int>((rowBytes(kKind, scan.dim) + kPieceBytes - 1) / kPieceBytes));
+    const int slots = filterSlots(static_cast<int>((rowBytes(FilterKind<kKind>::kDtype, scan.dim) + kPieceBytes - 1) / kPieceBytes));
     if constexpr (kWide) {
         return slots == 3 ? launchFilterPieces<kKind, 3>(scan, args, phase, emit, workgroups, stream)
                           : launchFilterPieces<kKind, 4>(scan, args, phase, emit, workgroups, stream);

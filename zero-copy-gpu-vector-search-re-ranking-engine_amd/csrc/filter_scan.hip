@@ -24,7 +24,7 @@ constexpr int kListRowsPerThread = 16;
 constexpr int kListThreads = 256;
 constexpr int kListRows = kListThreads * kListRowsPerThread;  // mask bytes per workgroup
 
-int stepsPerPiece(int dtype) { return dtype == ZCGVS_DTYPE_F32 ? 2 : dtype == ZCGVS_DTYPE_F16 ? 4 : 8; }
+int stepsPerPiece(int kind) { return kind == ZCGVS_DTYPE_F32 ? 2 : kind == ZCGVS_DTYPE_I8 ? 8 : 4; }
 
 // Component that element e of lane group h holds in step s of a row, -1 for none: the scan's
 // reading order (filter_kernel.hpp).
@@ -260,6 +260,39 @@ __global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(const
     }
 }
 
+// Per-vector int8: the operands are the queries' codes as they lie, chunk 16 piece + 4 j + h (step 4
+// piece + j) of a row's reading order at lane group h; the constants are the query scales.
+__global__ __launch_bounds__(kPrepareThreads) void filterPrepareCodesKernel(ScanArgs scan, FilterArgs args) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    const int t = threadIdx.x;
+    const int group = blockIdx.x;
+    const int chunks = scan.dim / 16;
+    if (group == 0 && blockIdx.y == 0 && t == 0 && args.list_count != nullptr) {
+        *args.list_count = 0u;
+    }
+    if (blockIdx.y == 0 && t < kFilterGroup) {
+        const int q = group * kFilterGroup + t;
+        FilterQuery out = {};
+        out.scale = q < scan.batch ? scan.query_scales[q] : 0.0f;
+        out.usable = 1.0f;
+        args.queries[q] = out;
+    }
+    u32x4* dst = reinterpret_cast<u32x4*>(args.operands) + static_cast<std::size_t>(group) * args.steps * kWave;
+    for (int item = static_cast<int>(blockIdx.y) * kPrepareThreads + t; item < args.steps * kWave;
+         item += kPrepareSplit * kPrepareThreads) {
+        const int step = item / kWave;
+        const int lane = item & (kWave - 1);
+        const int q = group * kFilterGroup + (lane & 15);
+        const int chunk = 4 * step + (lane >> 4);
+        u32x4 codes = {0u, 0u, 0u, 0u};
+        if (q < scan.batch && chunk < chunks) {
+            codes = *reinterpret_cast<const u32x4*>(static_cast<const std::uint8_t*>(scan.queries) +
+                                                    static_cast<std::size_t>(q) * scan.dim + 16 * chunk);
+        }
+        dst[item] = codes;
+    }
+}
+
 // The rows an allow-mask lets through, in no order across workgroups, 4096 mask bytes each. A
 // search with fewer such rows than it selects also returns masked rows, the lowest ones; all of
 // those lie among the first 2 * width rows (fewer than width of them are allowed), whose masked
@@ -316,8 +349,8 @@ __global__ __launch_bounds__(kListThreads) void filterListKernel(const std::uint
 
 FilterShape filterShape(const ScanArgs& scan, int width) {
     FilterShape shape;
-    if (scan.dtype != ZCGVS_DTYPE_F32 && scan.dtype != ZCGVS_DTYPE_F16 &&
-        !(scan.dtype == ZCGVS_DTYPE_I8 && scan.row_scales == nullptr)) {
+    const int kind = filterKind(scan);
+    if (kind == ZCGVS_DTYPE_BINARY) {
         return shape;
     }
     const std::size_t bytes = rowBytes(scan.dtype, scan.dim);
@@ -326,13 +359,16 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
     if (bytes < 16 || bytes > 4096 || !aligned16(scan.corpus) || scan.lexical != nullptr || scan.batch < 1) {
         return shape;
     }
-    if (scan.dtype == ZCGVS_DTYPE_I8 && !(scan.scale > 1e-15f && scan.scale < 1e15f)) {
+    if (kind == kFilterPerVector && (bytes % 16 != 0 || bytes > 1024)) {
+        return shape;
+    }
+    if (kind == ZCGVS_DTYPE_I8 && !(scan.scale > 1e-15f && scan.scale < 1e15f)) {
         return shape;
     }
     if (width > 8 * deviceComputeUnits() / 4) {
         return shape;  // too few sketch slots for this many keys
     }
-    shape.steps = static_cast<int>((bytes + 255) / 256) * stepsPerPiece(scan.dtype);
+    shape.steps = static_cast<int>((bytes + 255) / 256) * stepsPerPiece(kind);
     const int most = std::min<int>(kFilterMaxGroups, static_cast<int>(kFilterOperandBytes / 1024) / shape.steps);
     if (most < 1) {
         return shape;
@@ -362,7 +398,11 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
 int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_t stream) {
     const bool f32 = scan.dtype == ZCGVS_DTYPE_F32;
     const dim3 grid(static_cast<unsigned>(args.groups + (f32 ? 1 : 0)), kPrepareSplit);
-    filterPrepareKernel<<<grid, kPrepareThreads, 0, stream>>>(scan, args);
+    if (filterKind(scan) == kFilterPerVector) {
+        filterPrepareCodesKernel<<<grid, kPrepareThreads, 0, stream>>>(scan, args);
+    } else {
+        filterPrepareKernel<<<grid, kPrepareThreads, 0, stream>>>(scan, args);
+    }
     ZCGVS_LAUNCH_CHECK("filter prepare");
     if (args.list != nullptr) {
         const unsigned blocks = static_cast<unsigned>((scan.doc_count + kListRows - 1) / kListRows);
@@ -386,7 +426,10 @@ int launchFilterThreshold(const float* sketch, int slots, int batch, int width, 
 int launchFilterScan(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,
                      int workgroups, hipStream_t stream) {
     const bool wide = rowBytes(scan.dtype, scan.dim) > 2 * 256;
-    switch (scan.dtype) {
+    switch (filterKind(scan)) {
+        case kFilterPerVector:
+            return wide ? launchFilterKind<kFilterPerVector, true>(scan, args, phase, emit, workgroups, stream)
+                        : launchFilterKind<kFilterPerVector, false>(scan, args, phase, emit, workgroups, stream);
         case ZCGVS_DTYPE_F32:
             return wide ? launchFilterKind<ZCGVS_DTYPE_F32, true>(scan, args, phase, emit, workgroups, stream)
                         : launchFilterKind<ZCGVS_DTYPE_F32, false>(scan, args, phase, emit, workgroups, stream);

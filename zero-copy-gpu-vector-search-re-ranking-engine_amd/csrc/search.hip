@@ -382,6 +382,13 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
     if (singlePassShape(scan, plan.width).supported) {
         return false;  // a few queries: one launch that HBM bounds
     }
+    if (plan.use_mfma) {
+        // The int8 matrix-core scan serves 256 queries a launch and reads masked rows as well. 1M x 768:
+        // 16 queries 187 / 164, 64 queries 251 / 200, 128 queries 299 / 291; 30% allowed, 16 queries
+        // 202 / 80, 128 queries 300 / 141, 256 queries 273 / 250; 90% allowed, 256 queries 278 / 555.
+        // 5,000 x 384, 64 queries 24 / 38, 20,000 rows 46 / 39.
+        return n >= 8192 && scan.batch <= (scan.mask != nullptr ? 128 : 32);
+    }
     const long long tiles = (scan.batch + 7) / 8;  // of the queries the VALU kernels take at a time
     if (rowBytes(scan.dtype, scan.dim) % 16 != 0) {
         // The materialized pipeline's scalar scan: 20,000 x 100 int8, 2 queries 26 against 33;
@@ -443,17 +450,22 @@ Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
                     "zcgvs: per-vector int8 mode needs dim % 16 == 0 and a 16-byte aligned corpus");
     }
 
-    if (!forced && allow_filter && !plan.hybrid && !plan.binary && !plan.per_vector) {
+    if (!forced && allow_filter && !plan.hybrid && !plan.binary) {
         ScanArgs exact = probe;
         exact.mask = d.mask;
+        exact.row_scales = plan.per_vector ? d.corpus.row_scales : nullptr;
         plan.filter = filterShape(exact, plan.width);
         plan.use_filter = plan.filter.supported && recoverSupported(exact) && filterPays(exact, plan);
     }
     if (plan.use_filter) {
         Layout layout;
+        if (plan.per_vector) {
+            plan.qi8 = layout.add(static_cast<std::size_t>(batch) * dim);
+            plan.qscale = layout.add(static_cast<std::size_t>(batch) * 4);
+        }
         plan.overflow = layout.add(static_cast<std::size_t>(batch) * 4);
         planFilter(d, plan, layout);
-        plan.materialized = plan.use_mfma_float = false;
+        plan.materialized = plan.use_mfma_float = plan.use_mfma = false;
         // (a search that fits the no-allocation entry's scratch on another plan still does)
         return plan.total <= kStaticScratchBytes ? plan : makePlan(d, false);
     }
