@@ -179,3 +179,38 @@ def test_per_vector_int8_bit_exact(gpu, n, dim, batch, k, share):
     ref_idx, ref_val = oracle.topk(oracle.scores_i8i8(codes, scales, qcodes, qscales, mask), k)
     assert not flags.any()
     assert np.array_equal(idx, ref_idx) and np.array_equal(val, ref_val)
+
+
+# hybrid searches: the bounds go through the fusion; both ends of the weight
+@pytest.mark.parametrize("kind,n,dim,batch,k,metric,weight", [
+    ("f16", 20_011, 768, 9, 10, 0, 0.7),
+    ("f16", 20_011, 301, 33, 10, 0, 0.3),   # rows of no whole chunks, two launches
+    ("f32", 20_011, 100, 20, 50, 2, 0.5),
+    ("f32", 9_001, 1024, 16, 10, 1, 0.0),   # only the lexical scores decide (most tie at zero)
+    ("f16", 9_001, 100, 5, 10, 0, 1.0),
+])
+def test_hybrid(gpu, kind, n, dim, batch, k, metric, weight):
+    capi = gpu
+    stored, dtype, decoded = encode(capi, normalized(n, dim, 600 + dim), kind)
+    queries = normalized(batch, dim, 601)
+    rng = np.random.default_rng(602)
+    vocab, stride = 50, 4
+    counts = rng.integers(0, n // 10, vocab)
+    docs = np.concatenate([np.sort(rng.choice(n, c, replace=False)) for c in counts]).astype(np.int32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    weights = rng.random(docs.size).astype(np.float32)
+    terms = np.stack([rng.choice(vocab, stride, replace=False) for _ in range(batch)]).astype(np.int32)
+    terms[0] = -1  # a query without terms: no lexical part
+    d = [capi.DeviceArray.from_host(a) for a in (stored, queries, offsets, docs, weights, terms)]
+    desc = capi.search_desc(capi.store_desc(d[0], n, dim, dtype), d[1], batch, k, metric, lex_offsets=d[2], lex_docs=d[3],
+                            lex_weights=d[4], lex_doc_count=n, lex_vocab_size=vocab, query_terms=d[5],
+                            lexical_stride=stride, dense_weight=weight)
+    idx, val, flags = capi.search(desc)
+    dense = oracle.scores_f32(decoded, queries, metric)
+    fused = np.empty_like(dense)
+    for b in range(batch):
+        lex = oracle.bm25(offsets, docs, weights, terms[b], n)
+        fused[b] = oracle.fuse(dense[b], lex, oracle.max_positive(lex), weight)
+    # the dense part's rounding, and that of the fusion's three operations on values of at most 1
+    tol = np.float32(weight) * float_tolerance(queries, decoded, metric) + 3e-7
+    assert_topk_equivalent(idx, val, fused, k, tol)

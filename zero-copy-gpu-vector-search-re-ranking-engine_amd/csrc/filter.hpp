@@ -34,9 +34,11 @@ constexpr int filterSlots(int pieces) {
     return pieces <= 4 ? pieces : pieces == 5 || pieces == 6 || pieces == 9 ? 3 : 4;
 }
 
-// 16-row blocks of a wavefront's tile, which make it 8 to 16 KB in flight.
-constexpr int filterBlocks(int slots, int groups) {
-    return slots == 1 ? (groups <= 2 ? 4 : 2) : slots == 2 && groups <= 2 ? 2 : 1;
+// 16-row blocks of a wavefront's tile, which make it 8 to 16 KB in flight. (Fewer where the sums, or
+// a hybrid search's lexical scores, would take the registers.)
+constexpr int filterBlocks(int slots, int groups, bool lexical = false) {
+    const bool few = groups <= 2 && !lexical;
+    return slots == 1 ? (few ? 4 : 2) : slots == 2 && few ? 2 : 1;
 }
 
 struct FilterQuery {

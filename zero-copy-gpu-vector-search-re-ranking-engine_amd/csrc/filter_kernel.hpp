@@ -230,7 +230,9 @@ __device__ __forceinline__ float exactScore(const ScanArgs& scan, std::uint32_t 
 
 // A sketch phase (phase.sketch) scores one block of 16 rows per tile and keeps the best lower
 // bound of each query per wavefront.
-template <int kKind, int kPieces, int kBlocks, int kGroups>
+// With kLex, a hybrid search: the bounds go through the fusion with the lexical scores, which is
+// monotone in the dense score, rounding included.
+template <int kKind, int kPieces, int kBlocks, int kGroups, bool kLex>
 __global__ __launch_bounds__(kFilterThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs emit, int q_offset, int q_count,
                       int lanes_per_row) {
@@ -246,6 +248,8 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     __shared__ __attribute__((aligned(16))) float lds_slope[kQueries];  // threshold = slope * row term + base
     __shared__ __attribute__((aligned(16))) float lds_base[kQueries];
     __shared__ __attribute__((aligned(16))) float lds_gain[kQueries];   // sketch: bound = gain * acc + that
+    __shared__ __attribute__((aligned(16))) float lds_floor[kLex ? kQueries : 4];    // hybrid: the threshold,
+    __shared__ __attribute__((aligned(16))) float lds_inverse[kLex ? kQueries : 4];  // 1 / largest lexical score
     __shared__ std::uint64_t lds_tau[kQueries];
     __shared__ std::uint32_t lds_count[kQueries];
     __shared__ std::uint64_t lds_lowest[kQueries];  // the lowest of the first `width` keys appended
@@ -390,19 +394,34 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             lds_count[i] = 0u;
             lds_lowest[i] = ~0ull;
             lds_placed[i] = 0u;
-        } else if (sketch) {
-            // lower bound = gain * acc + slope * row term + base
+        } else if (kLex || sketch) {
+            // a bound of the score (hybrid: of its dense part; an upper one in a threshold phase) =
+            // gain * acc + slope * row term + base
+            const float side = sketch ? -1.0f : 1.0f;
             float gain = unit / query.scale;
-            float slope = -relative * qnorm * unit;
-            float base = -qnorm * unit * floor_abs;
+            float slope = side * relative * qnorm * unit;
+            float base = side * qnorm * unit * floor_abs;
             if (l2) {
                 gain *= 2.0f;
-                slope = -(1.0f + 2.0f * relative) * unit * unit;
-                base = 2.0f * (base - norm_abs) - (1.0f + 2.0f * relative) * query.norm2;
+                slope = -(1.0f - side * 2.0f * relative) * unit * unit;
+                base = 2.0f * (base + side * norm_abs) - (1.0f - side * 2.0f * relative) * query.norm2;
             }
-            lds_gain[i] = valid && query.usable != 0.0f ? gain : __uint_as_float(0x7FC00000u);  // NaN: no bound
+            // (NaN: no bound, which drops a sketch's row and keeps a threshold phase's)
+            lds_gain[i] = (valid || !sketch) && query.usable != 0.0f ? gain : __uint_as_float(0x7FC00000u);
             lds_slope[i] = slope;
             lds_base[i] = base;
+            if constexpr (kLex) {
+                bool gated = false;
+                const std::uint64_t tau = valid && !sketch ? emit.tau[q_offset + i] : ~0ull;
+                const float floor_score = keyFloor(tau, &gated);
+                lds_floor[i] = !valid ? INFINITY : gated ? floor_score : -INFINITY;
+                const float peak = valid ? scan.lexical_max[q_offset + i] : 0.0f;
+                lds_inverse[i] = peak > 0.0f ? 1.0f / peak : 0.0f;
+                lds_tau[i] = tau;
+                lds_count[i] = 0u;
+                lds_lowest[i] = ~0ull;
+                lds_placed[i] = 0u;
+            }
         } else {
             // a pair survives unless acc < slope * row term + base
             bool gated = false;
@@ -567,6 +586,10 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         const std::uint32_t row = listed & ~kMaskedRow;
         const int query = min(q_offset + q, scan.batch - 1);  // (a query past the batch parks NaN pairs only)
         float score = exactScore<kKind>(scan, row, query, lane, lanes_per_row);
+        if constexpr (kLex) {
+            score = fuseHybrid(score, scan.lexical[static_cast<std::size_t>(query) * scan.doc_count + row], scan.dense_weight,
+                               lds_inverse[q]);
+        }
         if (args.infinite_as_nan != 0 && scan.batch - query / 128 * 128 >= 32 && fabsf(score) == INFINITY) {
             score = __uint_as_float(0x7FC00000u);
         }
@@ -604,11 +627,24 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             const long long next = tile + waves;
             std::uint32_t id[kBlocks];  // this lane's rows in the results
             float row_scale[kBlocks];
+            v4f lexical[kLex ? kBlocks : 1][kLex ? kGroups : 1];
             std::uint32_t next_row[kBlocks][2];
             readRows(next, next_row);
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) {
                 id[b] = entryOf(tile, kFilterBlockRows * b + r16);
+                if constexpr (kLex) {
+                    // (a row or query that does not exist re-reads the first row's, the last query's)
+                    const std::size_t at = id[b] == kNoRow ? 0u : id[b];
+#pragma unroll
+                    for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int q = min(q_offset + kFilterGroup * g + 4 * h + i, scan.batch - 1);
+                            lexical[b][g][i] = scan.lexical[static_cast<std::size_t>(q) * scan.doc_count + at];
+                        }
+                    }
+                }
                 row_scale[b] = kInteger ? scan.row_scales[id[b] == kNoRow ? 0u : id[b] & ~kMaskedRow] : 0.0f;
                 norm[b] = 0.0f;
                 norm_codes[b] = 0;
@@ -653,7 +689,11 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             // Whether the pair of block b's row and query 16 g + 4 h + i can reach the query's threshold.
             // (A masked row does where every row does; a NaN survives.)
             auto survives = [&](int b, int g, int i, const v4f& slope, const v4f& offset) __attribute__((always_inline)) -> bool {
-                if constexpr (kInteger) {
+                if constexpr (kLex) {
+                    const int q = kFilterGroup * g + 4 * h + i;
+                    const float bound = fmaf(lds_gain[q], acc[b][g][i], fmaf(slope[i], term[b], offset[i]));
+                    return !(fuseHybrid(bound, lexical[b][g][i], scan.dense_weight, lds_inverse[q]) < lds_floor[q]);
+                } else if constexpr (kInteger) {
                     const float score = static_cast<float>(acc[b][g][i]) * (slope[i] * term[b]);
                     return masked[b] ? offset[i] == -INFINITY : !(score < offset[i]);
                 } else {
@@ -674,6 +714,10 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                             bound = static_cast<float>(acc[0][g][i]) * (gain[i] * term[0]);
                         } else {
                             bound = fmaf(gain[i], acc[0][g][i], fmaf(slope[i], term[0], offset[i]));
+                        }
+                        if constexpr (kLex) {
+                            bound = fuseHybrid(bound, lexical[0][g][i], scan.dense_weight,
+                                               lds_inverse[kFilterGroup * g + 4 * h + i]);
                         }
                         // (an infinite or NaN bound is none)
                         best[4 * g + i] = live[0] && !masked[0] && bound < 3.0e38f ? fmaxf(best[4 * g + i], bound) : best[4 * g + i];
@@ -823,11 +867,36 @@ int launchFilterPieces(const ScanArgs& scan, const FilterArgs& args, const Phase
     const int per_launch = args.groups_per_launch * kFilterGroup;
     for (int q0 = 0; q0 < scan.batch; q0 += per_launch) {
         const int count = scan.batch - q0 < per_launch ? scan.batch - q0 : per_launch;
+        if constexpr (kKind == ZCGVS_DTYPE_F32 || kKind == ZCGVS_DTYPE_F16) {
+            if (scan.lexical != nullptr) {
+                if (args.groups_per_launch == 1) {
+                    filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 1, true), 1, true>
+                    <<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes);
+                } else {
+                    filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 2, true), 2, true>
+                    <<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes);
+                }
+                ZCGVS_LAUNCH_CHECK("filter scan");
+                continue;
+            }
+        }
         switch (args.groups_per_launch) {
-            case 1: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 1), 1><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
-            case 2: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 2), 2><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
-            case 4: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 4), 4><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
-            default: filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 8), 8><<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes); break;
+            case 1:
+                filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 1), 1, false>
+                    <<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes);
+                break;
+            case 2:
+                filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 2), 2, false>
+                    <<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes);
+                break;
+            case 4:
+                filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 4), 4, false>
+                    <<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes);
+                break;
+            default:
+                filterScanKernel<kKind, kPieces, filterBlocks(kPieces, 8), 8, false>
+                    <<<grid, kFilterThreads, 0, stream>>>(scan, args, phase, emit, q0, count, lanes);
+                break;
         }
         ZCGVS_LAUNCH_CHECK("filter scan");
     }

@@ -356,10 +356,16 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
     const std::size_t bytes = rowBytes(scan.dtype, scan.dim);
     // rows of one chunk to 4 KB (the exact scores' lane groups), the corpus 16-byte aligned as the
     // other scans need it; an int8 scale whose products stay in range
-    if (bytes < 16 || bytes > 4096 || !aligned16(scan.corpus) || scan.lexical != nullptr || scan.batch < 1) {
+    if (bytes < 16 || bytes > 4096 || !aligned16(scan.corpus) || scan.batch < 1) {
         return shape;
     }
     if (kind == kFilterPerVector && (bytes % 16 != 0 || bytes > 1024)) {
+        return shape;
+    }
+    // Hybrid searches: float rows, a weight under which a higher dense score never lowers the fused
+    // one, and no mask (a masked row's fused score depends on its lexical one).
+    if (scan.lexical != nullptr && ((kind != ZCGVS_DTYPE_F32 && kind != ZCGVS_DTYPE_F16) || scan.mask != nullptr ||
+                                    !(scan.dense_weight >= 0.0f && scan.dense_weight <= 1.0f))) {
         return shape;
     }
     if (kind == ZCGVS_DTYPE_I8 && !(scan.scale > 1e-15f && scan.scale < 1e15f)) {
@@ -378,7 +384,7 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
     constexpr int kCounts[] = {1, 2, 4, 8};
     int largest = 1;
     for (const int c : kCounts) {
-        largest = c <= most ? c : largest;
+        largest = c <= (scan.lexical != nullptr ? std::min(most, 2) : most) ? c : largest;
     }
     int launches = (groups + largest - 1) / largest;
     const int even = (groups + launches - 1) / launches;  // as even a split as the counts allow
@@ -388,7 +394,8 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
         }
     }
     shape.tile_rows =
-        kFilterBlockRows * filterBlocks(filterSlots(static_cast<int>((bytes + 255) / 256)), shape.groups_per_launch);
+        kFilterBlockRows * filterBlocks(filterSlots(static_cast<int>((bytes + 255) / 256)), shape.groups_per_launch,
+                                        scan.lexical != nullptr);
     launches = (groups + shape.groups_per_launch - 1) / shape.groups_per_launch;
     shape.groups = launches * shape.groups_per_launch;
     shape.supported = true;

@@ -450,10 +450,11 @@ Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
                     "zcgvs: per-vector int8 mode needs dim % 16 == 0 and a 16-byte aligned corpus");
     }
 
-    if (!forced && allow_filter && !plan.hybrid && !plan.binary) {
+    if (!forced && allow_filter && !plan.binary && !(plan.hybrid && plan.use_mfma_float)) {
         ScanArgs exact = probe;
         exact.mask = d.mask;
         exact.row_scales = plan.per_vector ? d.corpus.row_scales : nullptr;
+        exact.dense_weight = d.dense_weight;
         plan.filter = filterShape(exact, plan.width);
         plan.use_filter = plan.filter.supported && recoverSupported(exact) && filterPays(exact, plan);
     }
@@ -464,10 +465,22 @@ Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
             plan.qscale = layout.add(static_cast<std::size_t>(batch) * 4);
         }
         plan.overflow = layout.add(static_cast<std::size_t>(batch) * 4);
+        if (plan.hybrid) {
+            plan.lex_sorted = (d.flags & ZCGVS_SEARCH_SORTED_POSTINGS) != 0;
+            if (plan.lex_sorted) {
+                plan.lexbounds = layout.add(lexicalBoundsBytes(batch, d.lexical_stride, static_cast<int>(n)));
+            }
+            plan.lex = layout.add(static_cast<std::size_t>(batch) * n * 4);
+            plan.lexmax = layout.add(static_cast<std::size_t>(batch) * 4);
+        }
         planFilter(d, plan, layout);
         plan.materialized = plan.use_mfma_float = plan.use_mfma = false;
+        if (plan.total <= kStaticScratchBytes) {
+            return plan;
+        }
         // (a search that fits the no-allocation entry's scratch on another plan still does)
-        return plan.total <= kStaticScratchBytes ? plan : makePlan(d, false);
+        const Plan other = makePlan(d, false);
+        return other.total <= kStaticScratchBytes ? other : plan;
     }
 
     Layout layout;
