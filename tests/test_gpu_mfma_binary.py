@@ -58,3 +58,34 @@ def test_batched_hamming_extreme_queries_and_duplicates(gpu):
     idx, val = search(capi, words, dim, queries, k)
     ref = oracle.scores_hamming(words, oracle.pack_binary(queries), dim)
     assert_topk_equivalent(idx, val, ref, k)
+
+
+# rows of 32, 48 and 96 bytes: words read past chunk boundaries, a last copy of half a kilobyte (384
+# bits); the dense, threshold and (2,000,003 rows) sketch phases, streamed and on the tile kernel
+@pytest.mark.parametrize("n,dim,batch,k", [
+    (3_001, 256, 4, 10),
+    (70_001, 256, 17, 100),
+    (70_001, 256, 100, 10),
+    (70_001, 384, 4, 10),
+    (120_007, 384, 33, 100),
+    (60_013, 768, 32, 1000),
+    (120_007, 768, 130, 10),
+    (2_000_003, 768, 20, 100),
+    (8_000_003, 384, 5, 10),
+])
+def test_short_rows_bit_exact(gpu, n, dim, batch, k):
+    capi = gpu
+    rng = np.random.default_rng(dim + batch)
+    words = rng.integers(0, 2**32, (n, dim // 32), dtype=np.uint32)
+    words[n // 3] = words[7]  # a tie across the corpus
+    queries = normalized(batch, dim, 900 + dim)
+    qbits = oracle.pack_binary(queries)
+    words[n - 1] = qbits[0]  # the best row is the last one
+    d_words, d_queries = capi.DeviceArray.from_host(words), capi.DeviceArray.from_host(queries)
+    desc = capi.search_desc(capi.store_desc(d_words, n, dim, capi.BINARY), d_queries, batch, k, capi.COSINE)
+    idx, val, flags = capi.search(desc)
+    assert not flags.any()
+    for first in range(0, batch, 16):  # (the oracle's scores of 8M rows a few queries at a time)
+        part = slice(first, first + 16)
+        ref_idx, ref_val = oracle.topk(oracle.scores_hamming(words, qbits[part], dim), k)
+        assert np.array_equal(idx[part], ref_idx) and np.array_equal(val[part], ref_val)

@@ -173,7 +173,7 @@ int launchMfmaSplitScan(const ScanArgs& scan, const PhaseArgs& phase, const Emit
                         int q0, int count, hipStream_t stream);
 
 // The binary (Hamming) MFMA scan (batches of at least 4 queries, no mask or lexical scores,
-// dim 512 or 1024).
+// dim 256, 384, 512, 768 or 1024).
 bool mfmaBinarySupported(const ScanArgs& scan);
 int mfmaBinaryBlockRows(const ScanArgs& scan);
 // Whether the binary scan can take the sketch plan (its streaming kernel has the sketch and rerun

@@ -32,7 +32,11 @@
 // MFMA layout (16x16x128, fp4 operands). Lane l supplies row (A) / query (B) l % 16 and 32 dims
 // of lane group h = l / 16 per step: 16-byte chunk h + 4j of the row covers steps 4j .. 4j + 3,
 // one word each; A and B use the same assignment, so every dim is counted once. D: lane l holds
-// query l % 16 and rows 4h + i, i < 4.
+// query l % 16 and rows 4h + i, i < 4. Rows of 256, 384 or 768 bits, which are no four chunks,
+// give lane group h a run of 2, 3 or 6 consecutive words instead (BinaryTile::wordOf) and lie in
+// LDS unswizzled. On the VALU scan they were bound by its popcounts: 4M rows, 32 queries, 500
+// candidates rescored took 506, 797 and 1397 us at 256, 384 and 768 bits against 116, 119 and 153
+// here (1024 bits: 173), 120 queries at 768 bits 4830 against 393.
 //
 // Corpus streaming as in the other MFMA scans (lds_copy.hpp): 48 KB tiles HBM -> LDS by
 // global_load_lds_dwordx4 in a 3-deep ring (smaller tiles in deeper rings measured slower: the
@@ -68,18 +72,55 @@ template <int kWords>
 struct BinaryTile {
     static constexpr int kRowBytes = kWords * 4;
     static constexpr int kChunks = kRowBytes / 16;
-    static constexpr int kLaneChunks = kChunks / 4;  // chunks per lane group
-    static constexpr int kRows = kTileBytesTarget / kRowBytes;
+    // The words a lane group holds of every row, one per product step (4 lane groups): whole chunks
+    // h, h + 4, ... of rows of 64 or 128 bytes, a run of consecutive words of others.
+    static constexpr int kLaneWords = kWords / 4;
+    static constexpr bool kWholeChunks = kChunks % 4 == 0;
+    // (at most 768 rows: short rows would make so few items of a small phase)
+    static constexpr int kRows = kTileBytesTarget / kRowBytes < 768 ? kTileBytesTarget / kRowBytes : 768;
     static constexpr int kRowBlocks = kRows / 16;
     static constexpr int kTileBytes = kRows * kRowBytes;
     static constexpr int kDepth = 3;
     static constexpr int kCopies = kTileBytes / 16 / kThreads;
-    static constexpr int kRowsPerBankPeriod = 256 / kRowBytes;
-    static_assert(kChunks % 4 == 0 && kChunks <= 8, "rows of 64 or 128 bytes (queries in registers)");
+    static_assert(kWords % 4 == 0 && kChunks <= 8, "rows of up to 128 bytes (queries in registers)");
     static_assert(kTileBytes % (16 * kThreads) == 0, "tile must split over the lanes");
     static_assert((kDepth - 1) * kCopies < 63, "copies in flight fit the vmcnt counter");
+    // Chunk position s of row r holds chunk s ^ swizzle(r), which spreads the 16 rows of a read over
+    // the LDS banks; rows of other sizes lie as they are (their 16 rows meet at most twice per bank).
     __host__ __device__ static constexpr int swizzle(int row) {
-        return (row / kRowsPerBankPeriod) & (kChunks - 1);
+        return kWholeChunks ? (row / (256 / kRowBytes)) & (kChunks - 1) : 0;
+    }
+    // Word of the row that lane group h holds at step t.
+    __host__ __device__ static constexpr int wordOf(int h, int t) {
+        return kWholeChunks ? 4 * (h + 4 * (t / 4)) + t % 4 : h * kLaneWords + t;
+    }
+    // Lane group h's words of the row staged at `row` (row number `r` of its tile or pair).
+    __device__ static __forceinline__ void read(const std::uint8_t* row, int r, int h, std::uint32_t (&dst)[kLaneWords]) {
+        if constexpr (kWholeChunks) {
+#pragma unroll
+            for (int jc = 0; jc < kLaneWords / 4; ++jc) {
+                const u32x4 chunk = *reinterpret_cast<const u32x4*>(row + ((h + 4 * jc) ^ swizzle(r)) * 16);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    dst[4 * jc + w] = chunk[w];
+                }
+            }
+        } else {
+            const std::uint32_t* words = reinterpret_cast<const std::uint32_t*>(row) + h * kLaneWords;
+            if constexpr (kLaneWords % 2 == 0) {
+#pragma unroll
+                for (int t = 0; t < kLaneWords; t += 2) {
+                    const uint2 pair = *reinterpret_cast<const uint2*>(words + t);
+                    dst[t] = pair.x;
+                    dst[t + 1] = pair.y;
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < kLaneWords; ++t) {
+                    dst[t] = words[t];
+                }
+            }
+        }
     }
 };
 
@@ -149,8 +190,7 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
     constexpr int kRows = Tile::kRows;
     constexpr int kRowBytes = Tile::kRowBytes;
     constexpr int kChunks = Tile::kChunks;
-    constexpr int kLaneChunks = Tile::kLaneChunks;
-    constexpr int kSteps = kLaneChunks * 4;  // one word (32 dims) per lane and step, 128 per step
+    constexpr int kSteps = Tile::kLaneWords;  // one word (32 dims) per lane and step, 128 per step
     constexpr int kDepth = Tile::kDepth;
     constexpr int kCopies = Tile::kCopies;
     constexpr int kRowBlocks = Tile::kRowBlocks;
@@ -195,18 +235,12 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
         const int q = q_offset + min(qlocal, q_count - 1);
         q_of[g] = q;
         const std::uint32_t* qrow = qwords + static_cast<std::size_t>(q) * kWords;
-        u32x4 chunk[kLaneChunks];
-#pragma unroll
-        for (int jc = 0; jc < kLaneChunks; ++jc) {
-            chunk[jc] = *reinterpret_cast<const u32x4*>(qrow + 4 * (h + 4 * jc));
-        }
+        std::uint32_t word[kSteps];
         int pop = 0;
 #pragma unroll
-        for (int jc = 0; jc < kLaneChunks; ++jc) {
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                pop += __popc(chunk[jc][w]);
-            }
+        for (int t = 0; t < kSteps; ++t) {
+            word[t] = qrow[Tile::wordOf(h, t)];
+            pop += __popc(word[t]);
         }
         // the four lane groups hold disjoint chunks of the query
         pop += waveXor(pop, 16);
@@ -214,7 +248,7 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
         popq[g] = pop;
 #pragma unroll
         for (int t = 0; t < kSteps; ++t) {
-            qb[g][t] = valid_of[g] ? signNibbles(chunk[t / 4][t % 4]) : v4i{0, 0, 0, 0};
+            qb[g][t] = valid_of[g] ? signNibbles(word[t]) : v4i{0, 0, 0, 0};
         }
         h_limit[g] = kDim + 1;  // no threshold: every h passes
         row_limit[g] = 0xFFFFFFFFu;
@@ -283,13 +317,6 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
         asm volatile("" ::: "memory");  // no LDS access moves above the barrier
     };
 
-    // chunk h + 4 jc of row r16 of a block
-    std::uint32_t a_off[kLaneChunks];
-#pragma unroll
-    for (int jc = 0; jc < kLaneChunks; ++jc) {
-        a_off[jc] = static_cast<std::uint32_t>(r16 * kRowBytes + ((h + 4 * jc) ^ Tile::swizzle(r16)) * 16);
-    }
-
     auto emitKeys = [&](const v4f& acc, int g, long long row0, int block, long long item_) {
         if (!valid_of[g]) {
             return;
@@ -331,11 +358,9 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
             const long long row0 = phaseBlock(item, phase.stride, phase.skip) * kRows;
             for (int block = first_block; block < kRowBlocks; block += waves_per_set) {
                 const std::uint8_t* rows = ring[slot] + block * 16 * kRowBytes;
-                u32x4 chunk[kLaneChunks];
-#pragma unroll
-                for (int jc = 0; jc < kLaneChunks; ++jc) {
-                    chunk[jc] = *reinterpret_cast<const u32x4*>(rows + a_off[jc]);
-                }
+                // (a block starts at a multiple of the swizzle's period)
+                std::uint32_t word[kSteps];
+                Tile::read(rows + r16 * kRowBytes, r16, h, word);
                 v4f acc[kGroups];
 #pragma unroll
                 for (int g = 0; g < kGroups; ++g) {
@@ -349,7 +374,7 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
                 // instead of waiting for them to read their operands; a sched_barrier per step pins
                 // that order.
                 v4i a[2];
-                a[0] = spreadNibbles(chunk[0][0]);
+                a[0] = spreadNibbles(word[0]);
 #pragma unroll
                 for (int t = 0; t < kSteps; ++t) {
 #pragma unroll
@@ -357,7 +382,7 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
                         acc[g] = mfmaNibbles(a[t % 2], qb[g][t], acc[g]);
                     }
                     if (t + 1 < kSteps) {
-                        a[(t + 1) % 2] = spreadNibbles(chunk[(t + 1) / 4][(t + 1) % 4]);
+                        a[(t + 1) % 2] = spreadNibbles(word[t + 1]);
                         // keeps step t's operand allocated until the expansion is written, so
                         // the two buffers never share registers
                         asm volatile("" ::"v"(a[t % 2]));
@@ -403,7 +428,8 @@ void mfmaBinaryScanKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q_o
 
 constexpr int kStreamThreads = 768;
 constexpr int kStreamWaves = kStreamThreads / kWave;
-constexpr int kStreamSlots = 3;  // LDS pair slots per wavefront
+// LDS pair slots per wavefront (108 to 144 KB per workgroup, 72 at 512 bits)
+constexpr int streamSlots(int words) { return words == 8 ? 9 : words == 12 ? 6 : 3; }
 
 // One query set (<= 32 queries): each of the workgroup's 12 wavefronts (three per SIMD) holds the
 // set's B operands in registers and streams its own rows, 32 rows (two 16-row blocks) at a time,
@@ -436,18 +462,17 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
     using Tile = BinaryTile<kWords>;
     constexpr int kRows = Tile::kRows;
     constexpr int kRowBytes = Tile::kRowBytes;
-    constexpr int kLaneChunks = Tile::kLaneChunks;
-    constexpr int kSteps = kLaneChunks * 4;  // one word (32 dims) per lane and step, 128 per step
+    constexpr int kSteps = Tile::kLaneWords;  // one word (32 dims) per lane and step, 128 per step
     constexpr int kPairs = Tile::kRowBlocks / 2;
     constexpr int kDim = kWords * 32;
     static_assert(Tile::kRowBlocks % 2 == 0, "an item splits into 32-row pairs");
 
     constexpr int kChunks = Tile::kChunks;
     constexpr int kPairBytes = 32 * kRowBytes;
-    constexpr int kPairCopies = kPairBytes / 1024;  // one 1 KB global_load_lds_dwordx4 per 1024 / kRowBytes rows
-    constexpr int kRowsPerCopy = 1024 / kRowBytes;
-    // each wavefront's two pair slots; slot position s of pair row r holds chunk s ^ swizzle(r)
-    __shared__ __attribute__((aligned(16))) std::uint8_t pair_lds[kStreamWaves][kStreamSlots][kPairBytes];
+    constexpr int kPairCopies = (kPairBytes + 1023) / 1024;  // global_load_lds_dwordx4 copies of 1 KB
+    constexpr int kSlots = streamSlots(kWords);
+    // each wavefront's pair slots; slot position s of pair row r holds chunk s ^ swizzle(r)
+    __shared__ __attribute__((aligned(16))) std::uint8_t pair_lds[kStreamWaves][kSlots][kPairCopies * 1024];
     __shared__ std::uint32_t lds_count[kSetQueries];
     __shared__ int lds_sketch[kSketch ? kStreamWaves : 1][kSetQueries];
 
@@ -493,8 +518,7 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
         for (int t = 0; t < kSteps; ++t) {
             v4i value = {0, 0, 0, 0};
             if (qlocal < q_count) {
-                const std::uint32_t word = qwords[static_cast<std::size_t>(queryOf(qlocal)) * kWords +
-                                                  4 * (h + 4 * (t / 4)) + t % 4];
+                const std::uint32_t word = qwords[static_cast<std::size_t>(queryOf(qlocal)) * kWords + Tile::wordOf(h, t)];
                 value = signNibbles(word);
             }
             qreg[t][g] = value;
@@ -517,12 +541,11 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
         const int q = queryOf(min(qlocal, q_count - 1));
         q_of[g] = q;
         const std::uint32_t* qrow = qwords + static_cast<std::size_t>(q) * kWords;
-        // the four lane groups hold disjoint chunks h + 4 jc of the query
+        // the four lane groups hold disjoint words of the query
         int pop = 0;
 #pragma unroll
-        for (int jc = 0; jc < kLaneChunks; ++jc) {
-            const u32x4 words = *reinterpret_cast<const u32x4*>(qrow + 4 * (h + 4 * jc));
-            pop += __popc(words[0]) + __popc(words[1]) + __popc(words[2]) + __popc(words[3]);
+        for (int t = 0; t < kSteps; ++t) {
+            pop += __popc(qrow[Tile::wordOf(h, t)]);
         }
         pop += waveXor(pop, 16);
         pop += waveXor(pop, 32);
@@ -572,17 +595,18 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
             }
         }
     };
-    // Pair p's rows into LDS slot `slot` of this wavefront: copy k moves pair rows
-    // k * kRowsPerCopy .. + kRowsPerCopy - 1, lane l the 16 bytes of row k * kRowsPerCopy + l / kChunks
-    // that land at slot position l % kChunks, so every copy reads 1 KB of consecutive rows (whole
-    // cache lines per quarter-wave). Rows past the corpus re-read its last row (their keys are never
-    // emitted). Pair indices stay below 2^31: 32-bit division by the constant kPairs.
+    // Pair p's rows into LDS slot `slot` of this wavefront: lane l of copy k moves the 16 bytes that
+    // land at chunk position 64 k + l of the pair, so every copy reads 1 KB of consecutive rows (whole
+    // cache lines per quarter-wave). The lanes past the pair's end (a last copy of half a kilobyte at
+    // 384 bits) repeat its last row into the slot's padding. Rows past the corpus re-read its last
+    // row (their keys are never emitted). Pair indices stay below 2^31: 32-bit division by the
+    // constant kPairs.
     // copy_offset[k]: this lane's source byte offset within the pair for copy k
     std::uint32_t copy_offset[kPairCopies];
 #pragma unroll
     for (int k = 0; k < kPairCopies; ++k) {
-        const int r = k * kRowsPerCopy + lane / kChunks;
-        copy_offset[k] = static_cast<std::uint32_t>(r * kRowBytes + ((lane % kChunks) ^ Tile::swizzle(r)) * 16);
+        const int r = min((k * kWave + lane) / kChunks, 31);
+        copy_offset[k] = static_cast<std::uint32_t>(r * kRowBytes + (((k * kWave + lane) % kChunks) ^ Tile::swizzle(r)) * 16);
     }
     auto copyPair = [&](long long p, int slot) {
         const std::uint32_t p32 = static_cast<std::uint32_t>(p);
@@ -599,27 +623,22 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
         } else {
 #pragma unroll
             for (int k = 0; k < kPairCopies; ++k) {
-                const int r = k * kRowsPerCopy + lane / kChunks;
+                const int r = min((k * kWave + lane) / kChunks, 31);
                 const long long row = min(row0 + r, doc_count - 1);
                 copyToLds(corpus + static_cast<std::size_t>(row) * kRowBytes + (copy_offset[k] - r * kRowBytes),
                           base + k * 1024);
             }
         }
     };
-    // The lane's A chunks of a staged pair: row 16 b + r16, chunk h + 4 jc (the 16 rows of one
-    // ds_read_b128 quarter-wave hit 16 distinct 16-byte bank groups through the swizzle).
-    auto readPair = [&](int slot, u32x4 (&dst)[2][kLaneChunks]) {
+    // The lane's words of a staged pair's rows 16 b + r16.
+    auto readPair = [&](int slot, std::uint32_t (&dst)[2][kSteps]) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             const int r = 16 * b + r16;
-#pragma unroll
-            for (int jc = 0; jc < kLaneChunks; ++jc) {
-                const int position = (h + 4 * jc) ^ Tile::swizzle(r);
-                dst[b][jc] = *reinterpret_cast<const u32x4*>(&pair_lds[wave][slot][r * kRowBytes + position * 16]);
-            }
+            Tile::read(&pair_lds[wave][slot][r * kRowBytes], r, h, dst[b]);
         }
     };
-    auto processPair = [&](const u32x4 (&cur)[2][kLaneChunks], long long p) {
+    auto processPair = [&](const std::uint32_t (&cur)[2][kSteps], long long p) {
         // the pair's rows first: phaseBlock branches, and products computed before a branch whose
         // far side uses them would be sunk past it, out of the step-by-step schedule below
         const std::uint32_t p32 = static_cast<std::uint32_t>(p);
@@ -628,8 +647,8 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
         const int pair_row = 32 * static_cast<int>(p32 - it * kPairs);
         v4f acc[2][2] = {};
         v4i a[2];
-        a[0] = spreadNibbles(cur[0][0][0]);
-        a[1] = spreadNibbles(cur[1][0][0]);
+        a[0] = spreadNibbles(cur[0][0]);
+        a[1] = spreadNibbles(cur[1][0]);
         // The B operands of step t + 1 are read from LDS during step t. The lane's index is
         // opaque to the compiler, which would otherwise keep every step's B operands in registers
         // across pairs (64 more registers, and spills).
@@ -642,8 +661,8 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
             acc[1][0] = mfmaNibbles(a[1], b0, acc[1][0]);
             acc[1][1] = mfmaNibbles(a[1], b1, acc[1][1]);
             if (t + 1 < kSteps) {
-                a[0] = spreadNibbles(cur[0][(t + 1) / 4][(t + 1) % 4]);
-                a[1] = spreadNibbles(cur[1][(t + 1) / 4][(t + 1) % 4]);
+                a[0] = spreadNibbles(cur[0][t + 1]);
+                a[1] = spreadNibbles(cur[1][t + 1]);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -690,26 +709,27 @@ void mfmaBinaryStreamKernel(ScanArgs scan, PhaseArgs phase, EmitArgs emit, int q
     const long long stride = static_cast<long long>(gridDim.x) * kStreamWaves;
     // workgroup-first: with few pairs every workgroup (candidate segment) still gets its share
     long long p = static_cast<long long>(wave) * gridDim.x + blockIdx.x;
-    // Three pairs in flight while one is multiplied, with no registers held for them: pair i waits
-    // in slot i % 3 of the wavefront's LDS, copied there three pairs ahead. Every iteration issues
+    // kSlots pairs in flight while one is multiplied, with no registers held for them: pair i waits
+    // in slot i % kSlots of the wavefront's LDS, copied there kSlots pairs ahead. Every iteration issues
     // one pair's copies (past the phase's end, its last pair again), so before pair i is read only
-    // pairs i + 1 and i + 2 may still be pending (later global stores of the emission only make
+    // the kSlots - 1 after it may still be pending (later global stores of the emission only make
     // the wait stricter). The copies are inline assembly the compiler does not count, hence the
     // explicit waits; the memory clobbers keep the LDS reads between them.
     const long long mine = p < pairs ? (pairs - p + stride - 1) / stride : 0;  // this wave's pairs
     if (mine > 0) {
-        copyPair(p, 0);
-        copyPair(min(p + stride, pairs - 1), 1);
-        copyPair(min(p + 2 * stride, pairs - 1), 2);
+#pragma unroll
+        for (int slot = 0; slot < kSlots; ++slot) {
+            copyPair(min(p + slot * stride, pairs - 1), slot);
+        }
     }
     for (long long i = 0; i < mine; ++i) {
-        const int slot = static_cast<int>(i % 3);
-        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * kPairCopies) : "memory");
-        u32x4 cur[2][kLaneChunks];
+        const int slot = static_cast<int>(i % kSlots);
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kSlots - 1) * kPairCopies) : "memory");
+        std::uint32_t cur[2][kSteps];
         readPair(slot, cur);
         // the slot's reads are done before its next copy is issued
         asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-        copyPair(min(p + 3 * stride, pairs - 1), slot);
+        copyPair(min(p + kSlots * stride, pairs - 1), slot);
         processPair(cur, p);
         p += stride;
     }
@@ -797,7 +817,7 @@ bool mfmaBinarySupported(const ScanArgs& scan) {
     if (!aligned16(scan.corpus) || !aligned16(scan.queries)) {
         return false;
     }
-    return scan.dim == 512 || scan.dim == 1024;
+    return scan.dim == 256 || scan.dim == 384 || scan.dim == 512 || scan.dim == 768 || scan.dim == 1024;
 }
 
 bool mfmaBinaryStreams(const ScanArgs& scan) { return scan.dtype == ZCGVS_DTYPE_BINARY; }
@@ -805,7 +825,13 @@ bool mfmaBinaryStreams(const ScanArgs& scan) { return scan.dtype == ZCGVS_DTYPE_
 int mfmaBinarySketchSlotsPerWorkgroup() { return kStreamSketchSlots; }
 
 int mfmaBinaryBlockRows(const ScanArgs& scan) {
-    return scan.dim == 512 ? BinaryTile<16>::kRows : BinaryTile<32>::kRows;
+    switch (scan.dim) {
+        case 256: return BinaryTile<8>::kRows;
+        case 384: return BinaryTile<12>::kRows;
+        case 512: return BinaryTile<16>::kRows;
+        case 768: return BinaryTile<24>::kRows;
+        default: return BinaryTile<32>::kRows;
+    }
 }
 
 int launchMfmaBinaryScan(const ScanArgs& scan, const PhaseArgs& phase, const EmitArgs& emit,
@@ -814,6 +840,9 @@ int launchMfmaBinaryScan(const ScanArgs& scan, const PhaseArgs& phase, const Emi
         return ZCGVS_OK;
     }
     switch (scan.dim) {
+        case 256: return launchShape<8>(scan, phase, emit, workgroups, stream);
+        case 384: return launchShape<12>(scan, phase, emit, workgroups, stream);
+        case 768: return launchShape<24>(scan, phase, emit, workgroups, stream);
         case 512: return launchShape<16>(scan, phase, emit, workgroups, stream);
         case 1024: return launchShape<32>(scan, phase, emit, workgroups, stream);
         default:
