@@ -140,7 +140,7 @@ def test_non_finite(gpu):
 @pytest.mark.parametrize("kind,dim,metric", [("f16", 768, 0), ("f16", 301, 2), ("i8", 100, 0), ("f32", 333, 1)])
 def test_overflowing_segments_fall_back(gpu, kind, dim, metric):
     capi = gpu
-    n, batch, k = 20_011, 11, 150
+    n, batch, k = 40_011, 11, 150
     stored, dtype, decoded = encode(capi, normalized(n, dim, 91), kind)
     queries = normalized(batch, dim, 92)
     mask = np.ones(n, np.uint8)

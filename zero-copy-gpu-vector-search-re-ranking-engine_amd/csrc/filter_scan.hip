@@ -371,8 +371,9 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
     if (kind == ZCGVS_DTYPE_I8 && !(scan.scale > 1e-15f && scan.scale < 1e15f)) {
         return shape;
     }
-    if (width > 8 * deviceComputeUnits() / 4) {
-        return shape;  // too few sketch slots for this many keys
+    const int slots = kFilterSketchSlots * deviceComputeUnits();
+    if (slots > kMaxSketchSlots || width > slots / 4) {
+        return shape;  // (too few sketch slots for this many keys)
     }
     shape.steps = static_cast<int>((bytes + 255) / 256) * stepsPerPiece(kind);
     const int most = std::min<int>(kFilterMaxGroups, static_cast<int>(kFilterOperandBytes / 1024) / shape.steps);

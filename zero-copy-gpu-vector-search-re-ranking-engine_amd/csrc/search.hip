@@ -29,6 +29,7 @@
 #include "filter.hpp"
 #include "fused.hpp"
 #include "rescore.hpp"
+#include "scan_core.hpp"
 #include "select.hpp"
 
 namespace zcgvs_hip {
@@ -387,13 +388,35 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
         // 16 queries 187 / 164, 64 queries 251 / 200, 128 queries 299 / 291; 30% allowed, 16 queries
         // 202 / 80, 128 queries 300 / 141, 256 queries 273 / 250; 90% allowed, 256 queries 278 / 555.
         // 5,000 x 384, 64 queries 24 / 38, 20,000 rows 46 / 39.
-        return n >= 8192 && scan.batch <= (scan.mask != nullptr ? 128 : 32);
+        // (A mask that lets a thousand rows through leaves every pair of theirs to score exactly, on
+        // few wavefronts: no large batches of wide selections.)
+        return n >= 8192 && (scan.mask != nullptr ? scan.batch <= 128 && scan.batch * plan.width <= 2048
+                                                  : scan.batch <= 32);
     }
+    // Pairs to score exactly, about 2 per key: over the wavefront tiles that share them, more than
+    // about 160 a tile would make the scan score those tiles whole (3,000 x 256 int8, 128 queries, k 90:
+    // 202 / 690), and a round of them (64 / lanes-per-row pairs a wavefront) takes about 1 us.
+    const long long pairs = 2LL * scan.batch * plan.width;
+    // (A mask may let few rows through, and fewer than the sketch needs leave all of them to score
+    // exactly: 20,000 x 300 float16, 5% allowed, 128 queries, k 200 144 / 2431; a sixteenth of the
+    // rows is taken for masked searches.)
+    const long long listed = scan.mask != nullptr ? n / 16 : n;
+    if (pairs * plan.filter.tile_rows > 160 * listed) {
+        return false;
+    }
+    const std::size_t row_bytes = rowBytes(scan.dtype, scan.dim);
+    const bool whole_chunks = row_bytes % 16 == 0;
+    const int per_round =
+        whole_chunks ? kWave / std::max(8, lanesPerRow(static_cast<int>(row_bytes / 16), 8, 8)) : 1;
+    const long long waves = std::min<long long>((n + plan.filter.tile_rows - 1) / plan.filter.tile_rows,
+                                                static_cast<long long>(deviceComputeUnits()) * kFilterWaves);
+    const long long rounds = pairs / (waves * per_round);
     const long long tiles = (scan.batch + 7) / 8;  // of the queries the VALU kernels take at a time
-    if (rowBytes(scan.dtype, scan.dim) % 16 != 0) {
-        // The materialized pipeline's scalar scan: 20,000 x 100 int8, 2 queries 26 against 33;
-        // 5,000 x 300 float16, 16 queries 31 / 31; 100,000 x 100 float16, 1 query 47 / 35.
-        return n * tiles * ((scan.dim + 63) / 64) >= 50'000;
+    if (!whole_chunks) {
+        // The materialized pipeline's scalar scan, about 0.2 ns per row, query tile and 64 components:
+        // 20,000 x 100 int8, 2 queries 26 / 33; 5,000 x 300 float16, 16 queries 31 / 31; 3,000 x 300,
+        // 128 queries 71 / 63, with k 90 73 / 171; 100,000 x 100, 1 query 47 / 35.
+        return n * tiles * ((scan.dim + 63) / 64) >= 50'000 + 5'000 * rounds;
     }
     if (plan.use_mfma_float) {
         // Up to 8191 rows that scan is one dense phase (5,000 x 384 float32, 64 queries 26 against 42;
@@ -401,11 +424,14 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
         // float16, 16 queries 155 / 160, 64 queries 169 / 176; float32, 16 queries 278 / 282); float32
         // batches, which that scan splits into six products, do not (64 queries 381 / 299, 128
         // queries 575 / 329).
-        return n >= 8192 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32;
+        // (8,200 x 384, 128 queries, k 200: 54 / 137 with that many pairs to score exactly)
+        return n >= 8192 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32 && rounds <= n / 8192;
     }
-    // The same line for the VALU scan's plan, or where its dense phase alone takes longer: float16
-    // 2,000 x 768, 5 queries 37 / 34, 16 queries 82 / 38; int8 2,000 x 384, 8 queries 30 / 35.
-    return n >= 8192 || tiles * scan.dim >= 640;
+    // The same line for the VALU scan's plan, or where its dense phase alone, about 0.033 us per query
+    // tile and component (per-vector int8 0.02), takes longer: float16 2,000 x 768, 5 queries 37 / 34,
+    // 16 queries 82 / 38; int8 2,000 x 384, 8 queries 30 / 35; per-vector 3,000 x 320, 16 queries 31 / 33.
+    const long long components = plan.per_vector ? scan.dim * 3LL / 5 : scan.dim;
+    return n >= 8192 || tiles * components >= 640 + 30 * rounds;
 }
 
 Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
