@@ -425,7 +425,9 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
         // batches, which that scan splits into six products, do not (64 queries 381 / 299, 128
         // queries 575 / 329).
         // (8,200 x 384, 128 queries, k 200: 54 / 137 with that many pairs to score exactly)
-        return n >= 8192 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32 && rounds <= n / 8192;
+        // Two phases and their merges cost 22 us more, which the gain of about 0.08 us per 1000 rows
+        // covers from some 300,000 rows on (one search of fewer measured 56 / 72).
+        return n >= 400'000 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32 && rounds <= n / 8192;
     }
     // The same line for the VALU scan's plan, or where its dense phase alone, about 0.033 us per query
     // tile and component (per-vector int8 0.02), takes longer: float16 2,000 x 768, 5 queries 37 / 34,
