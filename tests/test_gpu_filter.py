@@ -93,15 +93,99 @@ def test_magnitudes(gpu, kind, dim, scale):
                            float_tolerance(queries, decoded, 1) - np.float64(1e-7) * (scale < 1e-3))
 
 
-def test_mixed_magnitudes(gpu):
-    # rows whose scales span forty binary orders: most approximate to zero or overflow float16
+@pytest.mark.parametrize("metric", [1, 2])
+@pytest.mark.parametrize("sampled", [0, -20])
+def test_mixed_magnitudes(gpu, metric, sampled):
+    # rows whose scales span forty binary orders: most approximate to zero, and with the sampled rows (the
+    # multiples of n / 16) at the bottom the largest overflow float16
     capi = gpu
     n, dim, batch, k = 9_001, 640, 5, 10
     rng = np.random.default_rng(63)
-    rows = normalized(n, dim, 64) * np.exp2(rng.integers(-20, 21, (n, 1))).astype(np.float32)
+    exponents = rng.integers(-20, 21, (n, 1))
+    if sampled:
+        exponents[np.arange(16) * (n // 16)] = sampled
+    rows = normalized(n, dim, 64) * np.exp2(exponents).astype(np.float32)
     queries = normalized(batch, dim, 65)
+    if metric == 2:  # distances on every scale
+        queries *= np.exp2(np.array([[-20], [-10], [0], [10], [20]])).astype(np.float32)
+    idx, val, _ = run(capi, rows, capi.F32, queries, k, metric)
+    assert_topk_equivalent(idx, val, oracle.scores_f32(rows, queries, metric), k, float_tolerance(queries, rows, metric))
+
+
+# Rows thousands (and, with `scale`, hundreds of thousands) of times longer than the ones the row unit is
+# sampled from, which are the multiples of n / 16: their float16 operands overflow or are far from the
+# unit, and the approximate scores of an overflowing row say nothing.
+def _unsampled(n, rng, count):
+    return rng.permutation(np.setdiff1d(np.arange(n), np.arange(16) * (n // 16)))[:count]
+
+
+@pytest.mark.parametrize("dim", [640, 300, 333])  # whole pieces, a partial chunk half, 4-byte alignment
+@pytest.mark.parametrize("lexical", [False, True])
+@pytest.mark.parametrize("scale", [1, 200])
+def test_outlier_rows_dot(gpu, dim, lexical, scale):
+    # every query has 3 rows of length 5000 that score 400, 12 of length 300 that score 300, and ordinary
+    # rows (all but those times `scale`); clamped, the longest would score about 100 to 200
+    capi = gpu
+    n, batch, k = 20_000, 8, 10
+    rng = np.random.default_rng(66 + dim)
+    rows, queries = normalized(n, dim, 67), normalized(batch, dim, 68)
+    places = _unsampled(n, rng, batch * 15).reshape(batch, 15)
+    for b in range(batch):
+        away = rng.standard_normal((3, dim))
+        away -= (away @ queries[b])[:, None] * queries[b]
+        away /= np.linalg.norm(away, axis=1, keepdims=True)
+        rows[places[b, :3]] = scale * 5000.0 * (0.08 * queries[b] + np.sqrt(1 - 0.08 ** 2) * away)
+        rows[places[b, 3:]] = scale * (300.0 - 0.01 * np.arange(12)[:, None]) * queries[b]
+    if not lexical:
+        idx, val, _ = run(capi, rows, capi.F32, queries, k, 1)
+        ref = oracle.scores_f32(rows, queries, 1)
+        assert all(set(places[b, :3]) <= set(idx[b]) for b in range(batch))
+    else:  # a posting list over a few rows
+        docs, terms = np.sort(rng.choice(n, 500, replace=False)).astype(np.int32), np.zeros((batch, 1), np.int32)
+        offsets, weights = np.array([0, docs.size], np.int64), rng.random(docs.size).astype(np.float32)
+        d = [capi.DeviceArray.from_host(a) for a in (rows, queries, offsets, docs, weights, terms)]
+        desc = capi.search_desc(capi.store_desc(d[0], n, dim, capi.F32), d[1], batch, k, 1, lex_offsets=d[2], lex_docs=d[3],
+                                lex_weights=d[4], lex_doc_count=n, lex_vocab_size=1, query_terms=d[5], lexical_stride=1,
+                                dense_weight=0.5)
+        idx, val, _ = capi.search(desc)
+        lex = oracle.bm25(offsets, docs, weights, terms[0], n)
+        ref = oracle.scores_f32(rows, queries, 1)
+        ref = np.stack([oracle.fuse(ref[b], lex, oracle.max_positive(lex), 0.5) for b in range(batch)])
+    assert_topk_equivalent(idx, val, ref, k, float_tolerance(queries, rows, 1) + 3e-7)
+
+
+def test_sums_that_overflow_on_the_way(gpu):
+    # a row whose float32 sum becomes infinite and would be zero: it ranks first, as the sum says
+    capi = gpu
+    n, dim, batch, k = 9_001, 640, 5, 10
+    rows = normalized(n, dim, 74) * np.float32(1e37)
+    places = 100 + 160 * np.arange(50)
+    rows[places] = 0.0
+    rows[places, 0] = np.float32(1e38)
+    rows[4_321] = 0.0
+    rows[4_321, :4] = np.float32(3e38) * np.array([1, 1, -1, -1], np.float32)
+    queries = np.ones((batch, dim), np.float32) + np.arange(batch, dtype=np.float32)[:, None]
     idx, val, _ = run(capi, rows, capi.F32, queries, k, 1)
-    assert_topk_equivalent(idx, val, oracle.scores_f32(rows, queries, 1), k, float_tolerance(queries, rows, 1))
+    assert (idx[0] == [4_321, *places[:9]]).all() and np.isinf(val[0, 0])
+    exact = run(capi, rows, capi.F32, queries, k, 1, flags=capi.SEARCH_FORCE_EXACT_PASS)
+    assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("dim", [640, 300, 333])
+@pytest.mark.parametrize("length", [5e3, 1e6])
+def test_outlier_rows_l2(gpu, dim, length):
+    # twenty long rows, queries near some of them, between them and the rest, and near the rest
+    capi = gpu
+    n, batch, k = 20_000, 9, 10
+    rng = np.random.default_rng(69 + dim)
+    rows, queries = normalized(n, dim, 70), normalized(batch, dim, 73)
+    places = _unsampled(n, rng, 20)
+    rows[places] *= np.float32(length)
+    queries[:4] = rows[places[:4]] + np.float32(50.0) * queries[:4]
+    queries[4:7] = np.float32(0.5) * rows[places[4:7]] + queries[4:7]
+    idx, val, _ = run(capi, rows, capi.F32, queries, k, 2)
+    assert np.array_equal(idx[:4, 0], places[:4])
+    assert_topk_equivalent(idx, val, oracle.scores_f32(rows, queries, 2), k, float_tolerance(queries, rows, 2))
 
 
 @pytest.mark.parametrize("kind,dim,metric", [("f16", 768, 0), ("f32", 300, 2), ("i8", 333, 0)])

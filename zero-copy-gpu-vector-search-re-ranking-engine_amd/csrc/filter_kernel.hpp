@@ -74,10 +74,16 @@ struct FilterSums<true> {
     typedef v4i type;
 };
 
+// Square of float16's largest value. The conversion of a float32 row rounds toward zero, so a
+// component beyond that value becomes it, not infinity, and the row's approximate scores say
+// nothing. Its squared norm in operand units (a float32 sum of non-negative terms, at least any one
+// of them) then reaches this: such a row is unbounded.
+constexpr float kOperandNorm2 = 65504.0f * 65504.0f;
+
 // Relative error of an approximate dot product, in units of |q| |x|: operand rounding (float16
 // queries to nearest, 2^-11; float32 rows toward zero, another 2^-10), float32 accumulation over
 // `steps` products of 32 (each taken at 2^-21, four times a rounding of every addition inside),
-// and the exact score's own rounding.
+// and the exact score's own rounding. For rows that are not unbounded.
 __host__ __device__ inline float filterRelative(int kind, int steps) {
     const float operands = kind == ZCGVS_DTYPE_F32 ? 1.48e-3f : 4.95e-4f;
     return operands + 4.8e-7f * static_cast<float>(steps) + 3.1e-5f;
@@ -382,6 +388,10 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         const bool valid = i < q_count;
         const FilterQuery query = args.queries[q_offset + i];
         const float qnorm = sqrtf(query.norm2) * 1.00001f;
+        // (a score, and every partial sum of one, is bounded by the norms: where that is beyond float32,
+        // an exact sum may overflow on its way to a value the approximation has in range)
+        const float reach = kF32 ? 65504.0f * unit : 0.0f;  // of a row that is not unbounded
+        const bool usable = query.usable != 0.0f && (l2 ? (qnorm + reach) * (qnorm + reach) : qnorm * reach) < 1e38f;
         if constexpr (kInteger) {
             // score = acc * (query scale * row scale), compared with the threshold's itself
             bool gated = false;
@@ -407,7 +417,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 base = 2.0f * (base + side * norm_abs) - (1.0f - side * 2.0f * relative) * query.norm2;
             }
             // (NaN: no bound, which drops a sketch's row and keeps a threshold phase's)
-            lds_gain[i] = (valid || !sketch) && query.usable != 0.0f ? gain : __uint_as_float(0x7FC00000u);
+            lds_gain[i] = (valid || !sketch) && usable ? gain : __uint_as_float(0x7FC00000u);
             lds_slope[i] = slope;
             lds_base[i] = base;
             if constexpr (kLex) {
@@ -435,7 +445,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 base = to_acc * (0.5f * (floor_score + (1.0f - 2.0f * relative) * query.norm2) - qnorm * unit * floor_abs -
                                  norm_abs);
             }
-            const bool filter = gated && query.usable != 0.0f && fabsf(base) < 3.0e38f && fabsf(slope) < 3.0e38f &&
+            const bool filter = gated && usable && fabsf(base) < 3.0e38f && fabsf(slope) < 3.0e38f &&
                                 floor_score > kMaskedScore;
             lds_slope[i] = valid && filter ? slope : 0.0f;
             // (a query past the batch takes no pair: nothing but NaN fails acc < inf, and those
@@ -682,6 +692,11 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                     n2 += waveXor(n2, 16);
                     n2 += waveXor(n2, 32);
                     term[b] = l2 ? n2 : sqrtf(n2) * 1.00001f;
+                    if constexpr (kF32) {
+                        // an unbounded row: every bound is NaN, which no sketch takes and every
+                        // threshold lets through
+                        term[b] = n2 < kOperandNorm2 ? term[b] : __uint_as_float(0x7FC00000u);
+                    }
                 }
                 live[b] = id[b] != kNoRow;
                 masked[b] = list != nullptr && (id[b] & kMaskedRow) != 0u;

@@ -55,7 +55,7 @@ __device__ __forceinline__ int componentOf(int dtype, int dim, int s, int h, int
     return chunk == whole && at >= elems - rest ? dim - elems + at : -1;
 }
 
-// Largest power of two exponent that keeps `peak` * 2^e at or below 2^15 (0 for a peak that is
+// Exponent e of the power of two that brings `peak` into [2^(top - 1), 2^top) (0 for a peak that is
 // zero or not finite).
 __device__ __forceinline__ int exponentBelow(float peak, int top) {
     if (!(peak > 0.0f) || !(peak <= 3.402823466e+38f)) {
@@ -69,9 +69,11 @@ __device__ __forceinline__ int exponentBelow(float peak, int top) {
 // Block (g, part): query group g's constants (part 0 writes them) and its share of the group's
 // operands. Block (0, 0) also clears the row list's count; with float32 rows, the blocks past the
 // groups find the row unit: the power of two that brings the largest component of a sample of rows
-// near 2^7, which leaves a factor of 2^9 to float16's largest value and 2^21 to its smallest
-// normal one. (A row outside that range only loses precision, or overflows, in its approximate
-// score, whose bound says so.)
+// to [1, 2), which leaves a factor of 2^15 to float16's largest value, 2^14 to its smallest normal
+// one and 2^24 to its smallest. (A smaller component loses up to that last one, which the bound's
+// absolute part counts. A row that leaves the range at the top has no bound and is scored exactly
+// for every query, kOperandNorm2, hence the middle: components 2^9 times the sample's, all that a
+// peak near 2^7 allows, are met where rows' lengths vary.)
 __global__ __launch_bounds__(kPrepareThreads) void filterPrepareKernel(ScanArgs scan, FilterArgs args) {
     const int t = threadIdx.x;
     const int dim = scan.dim;
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(kPrepareThreads) void filterPrepareKernel(ScanArgs 
             for (int w = 1; w < kPrepareThreads / kWave; ++w) {
                 peak = fmaxf(peak, lds_peak[w]);
             }
-            *args.row_unit = ldexpf(1.0f, -exponentBelow(peak, 7));
+            *args.row_unit = ldexpf(1.0f, -exponentBelow(peak, 1));
         }
         return;
     }
