@@ -221,6 +221,33 @@ def test_non_finite(gpu):
     assert not (np.delete(idx, 2, axis=0) == 900).any()
 
 
+@pytest.mark.parametrize("kind,dim,metric,batch,n,masked", [
+    ("f16", 768, 0, 9, 20_011, 0.05),
+    ("i8", 333, 1, 17, 20_011, 0.5),
+    ("f32", 300, 2, 5, 60_017, 0.0003),  # masked rows sought over several steps, about as many as are selected
+    ("f16", 100, 0, 5, 60_017, 0.0),     # a single masked row, the last one
+])
+def test_masked_rows_outrank_nan_and_minus_infinity(gpu, kind, dim, metric, batch, n, masked):
+    # a query for which every allowed row scores NaN (cosine, dot) or -inf (L2): the masked rows, lowest
+    # first and wherever they lie, come before those
+    capi = gpu
+    k = 10
+    stored, dtype, decoded = encode(capi, normalized(n, dim, 83), kind)
+    queries = normalized(batch, dim, 84)
+    bad = batch // 2
+    queries[bad, 7] = np.float32(1e30) if metric == 2 else np.nan
+    mask = (np.random.default_rng(85).random(n) >= masked).astype(np.uint8)
+    mask[:3 * k], mask[n - 1] = 1, 0
+    idx, val, _ = run(capi, stored, dtype, queries, k, metric, mask)
+    hidden, allowed = np.flatnonzero(mask == 0)[:k], np.flatnonzero(mask)
+    assert np.array_equal(idx[bad], np.concatenate([hidden, allowed])[:k])
+    assert (val[bad, :hidden.size] == -np.finfo(np.float32).max).all()
+    assert not np.isfinite(val[bad, hidden.size:]).any()
+    good = np.arange(batch) != bad
+    assert_topk_equivalent(idx[good], val[good], oracle.scores_f32(decoded, queries[good], metric, mask), k,
+                           float_tolerance(queries[good], decoded, metric))
+
+
 @pytest.mark.parametrize("kind,dim,metric", [("f16", 768, 0), ("f16", 301, 2), ("i8", 100, 0), ("f32", 333, 1)])
 def test_overflowing_segments_fall_back(gpu, kind, dim, metric):
     capi = gpu

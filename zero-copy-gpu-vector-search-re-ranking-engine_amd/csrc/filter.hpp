@@ -78,6 +78,12 @@ inline std::size_t filterOperandBytes(const FilterShape& shape) {
 // Entries of the row list: every row, and room for a whole tile.
 inline std::size_t filterListEntries(long long rows) { return static_cast<std::size_t>(rows) + 64; }
 
+// A search with fewer allowed rows than it selects also returns masked rows, the lowest ones. All of
+// those lie among the first 2 * width rows (fewer than width of them are allowed), whose masked ones
+// the row list holds too. (Masked rows past these can be selected only in the place of allowed rows
+// that score -inf or NaN, which the last merge sees to: MergeInputs::masked_from.)
+inline long long filterMaskedRows(long long rows, int width) { return rows < 2LL * width ? rows : 2LL * width; }
+
 // The query operands, the row unit and, with a mask, the row list.
 int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_t stream);
 // After a sketch phase: tau[q] (and tau_safe[q]), a key below the width-th best of query q's rows.

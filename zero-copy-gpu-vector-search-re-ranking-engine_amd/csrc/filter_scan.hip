@@ -295,10 +295,8 @@ __global__ __launch_bounds__(kPrepareThreads) void filterPrepareCodesKernel(Scan
     }
 }
 
-// The rows an allow-mask lets through, in no order across workgroups, 4096 mask bytes each. A
-// search with fewer such rows than it selects also returns masked rows, the lowest ones; all of
-// those lie among the first 2 * width rows (fewer than width of them are allowed), whose masked
-// ones are listed too, with kMaskedRow set.
+// The rows an allow-mask lets through, in no order across workgroups, 4096 mask bytes each, and the
+// masked ones of the first keep_masked rows (filterMaskedRows) with kMaskedRow set.
 __global__ __launch_bounds__(kListThreads) void filterListKernel(const std::uint8_t* __restrict__ mask, long long rows,
                                                                  long long keep_masked, std::uint32_t* __restrict__ list,
                                                                  std::uint32_t* __restrict__ count) {
@@ -416,7 +414,7 @@ int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_
     ZCGVS_LAUNCH_CHECK("filter prepare");
     if (args.list != nullptr) {
         const unsigned blocks = static_cast<unsigned>((scan.doc_count + kListRows - 1) / kListRows);
-        const long long keep = std::min<long long>(scan.doc_count, 2LL * args.width);
+        const long long keep = filterMaskedRows(scan.doc_count, args.width);
         filterListKernel<<<blocks, kListThreads, 0, stream>>>(scan.mask, scan.doc_count, keep, args.list, args.list_count);
         ZCGVS_LAUNCH_CHECK("filter row list");
     }

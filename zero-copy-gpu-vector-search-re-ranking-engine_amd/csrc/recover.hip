@@ -458,6 +458,49 @@ __global__ __launch_bounds__(kRecoverThreads) void recoverKernel(ScanArgs scan, 
                                           &lds_state, &lds_fill, &lds_tau});
 }
 
+// Joins the `k` keys the merge of query q selected (in lds.keys) with the lowest masked rows from
+// in.masked_from on, for a selection that ends below their keys; written like the merge's. By the
+// whole block, 16 mask bytes a thread and step until k masked rows are found.
+__device__ __forceinline__ void joinMaskedTail(const MergeInputs& in, const ScanArgs& scan, int k, int q,
+                                               std::uint64_t* __restrict__ out_keys, int* __restrict__ out_index,
+                                               float* __restrict__ out_score, MergeLds& lds) {
+    constexpr int kPer = 16;
+    const int t = threadIdx.x;
+    const long long rows = scan.doc_count;
+    for (int i = t; i < k; i += kRecoverThreads) {
+        lds.cand[i] = lds.keys[i];
+    }
+    std::uint32_t found = 0u;  // (uniform)
+    for (long long base = in.masked_from; base < rows && found < static_cast<std::uint32_t>(k);
+         base += kRecoverThreads * kPer) {
+        const long long first = base + t * kPer;
+        std::uint32_t masked = 0u;  // bit i: row first + i is masked
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            masked |= first + i < rows && scan.mask[min(first + i, rows - 1)] == 0 ? 1u << i : 0u;
+        }
+        std::uint32_t total = 0u;
+        const std::uint32_t own = static_cast<std::uint32_t>(__popc(masked));
+        std::uint32_t at = found + blockInclusiveSum<kRecoverThreads>(own, lds.scan, &total) - own;
+        for (; masked != 0u && at < static_cast<std::uint32_t>(k); ++at) {
+            lds.cand[k + at] = makeKey(kMaskedScore, static_cast<std::uint32_t>(first + __ffs(masked) - 1));
+            masked &= masked - 1u;
+        }
+        found += total;
+    }
+    __syncthreads();
+    const std::uint32_t joined = static_cast<std::uint32_t>(k) + min(found, static_cast<std::uint32_t>(k));
+    forEachRanked(lds.cand, joined, [&](std::uint32_t rank, std::uint64_t key) {
+        if (rank < static_cast<std::uint32_t>(k)) {
+            const std::size_t o = static_cast<std::size_t>(q) * k + rank;
+            out_keys[o] = key;
+            if (out_index != nullptr) {
+                writeHit(key, &out_index[o], &out_score[o]);
+            }
+        }
+    });
+}
+
 // The final merge of a phased search and its exact fallback in one launch: block q merges query
 // q's candidates (merge.hpp) and, when that merge flags the query (or with `force`), recomputes
 // its selection in the merge's LDS. No separate fallback launch runs for a search without flags.
@@ -472,6 +515,10 @@ __global__ __launch_bounds__(kRecoverThreads) void mergeRecoverKernel(MergeInput
     const int q = static_cast<int>(blockIdx.x);
     const bool flagged = mergeQuery(in, k, batch, out_keys, nullptr, overflow, out_index, out_score, q, lds);
     if (!flagged && !args.force) {
+        // (an unflagged query of a search that gives masked_from has k keys, require_full)
+        if (in.masked_from > 0 && lds.kth < makeKey(kMaskedScore, static_cast<std::uint32_t>(in.masked_from - 1))) {
+            joinMaskedTail(in, scan, k, q, out_keys, out_index, out_score, lds);
+        }
         return;  // uniform
     }
     // the staged query at the end of the candidate LDS, the running list before it
@@ -579,7 +626,7 @@ int launchMergeRecover(const MergeInputs& in, int k, int batch, std::uint64_t* o
                        int* out_index, float* out_score, const ScanArgs& scan, const RecoverArgs& args,
                        hipStream_t stream) {
     if (args.width != k || k <= 0 || k > kMaxK || batch != scan.batch || batch <= 0 || in.n_seg > kMaxSegments ||
-        args.flag_list != nullptr || args.seg != nullptr) {
+        args.flag_list != nullptr || args.seg != nullptr || (in.masked_from > 0 && (scan.mask == nullptr || !in.require_full))) {
         return setError(ZCGVS_ERR_RUNTIME, "zcgvs merge and recovery: arguments out of range");
     }
     if (!recoverSupported(scan)) {

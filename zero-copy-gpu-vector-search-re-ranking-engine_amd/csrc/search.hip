@@ -1225,6 +1225,9 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
                 in.reset_overflow = first_scan;
                 in.require_full = last;
                 in.fallback_tau = at<std::uint64_t>(ws, plan.tau_safe);
+                if (last && plan.use_filter && d.mask != nullptr) {
+                    in.masked_from = filterMaskedRows(d.corpus.doc_count, plan.width);
+                }
             } else if (p == 0) {
                 in.dense = emit.dense;
                 in.n_dense = phase.items * phase.block_rows;

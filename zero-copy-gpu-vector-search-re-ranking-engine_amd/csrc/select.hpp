@@ -175,6 +175,10 @@ struct MergeInputs {
     std::uint32_t* flag_list = nullptr;
     std::uint32_t* flag_count = nullptr;
     std::uint64_t* rerun_tau = nullptr;
+    // When not 0 (launchMergeRecover with a mask): no candidate is a masked row of this number or a
+    // higher one. They rank above rows that score -inf or NaN, so a selection that reaches below
+    // their keys takes the lowest of them in their place.
+    long long masked_from = 0;
 };
 
 // Selects the best k keys of each query's candidate set; writes them to out_keys[q][0..k)
