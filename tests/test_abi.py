@@ -215,6 +215,22 @@ def test_phase_rows_cover_the_corpus_once(capi, n, dtype, int8_mode, batch, k):
     assert all(r > 0 for r in rows)
 
 
+@pytest.mark.parametrize("n,dim,dtype,batch,masked", [
+    (16_000_000, 384, 1, 16, True),  # row lists of 64 and 80 MB
+    (20_000_000, 384, 1, 16, True),
+    (16_500_000, 384, 2, 16, True),
+    (20_000, 300, 1, 470, False),    # segments around 64 MB
+    (20_000, 300, 1, 520, False),
+    (20_000, 300, 1, 600, False),
+])
+def test_workspace_size_does_not_end_the_filter_scan(capi, n, dim, dtype, batch, masked):
+    # only the no-allocation entry's workspace is fixed; every other search keeps its plan (a sample,
+    # then every row) whatever it needs
+    desc = _desc(capi, n=n, dim=dim, dtype=dtype, batch=batch, mask=1 << 22 if masked else None)
+    rows = capi.search_phase_rows(desc)
+    assert len(rows) == 2 and rows[1] == n
+
+
 @pytest.mark.parametrize("n,dtype,int8_mode,batch,k", [
     (123_457, 1, 0, 3, 10),         # float16, three queries
     (1_000_000, 0, 0, 1, 32),       # float32

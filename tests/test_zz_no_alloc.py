@@ -68,6 +68,25 @@ def test_noalloc_matches_the_workspace_entry_point(gpu, case):
             assert np.array_equal(got_idx, ref[0]) and np.array_equal(got_val, ref[1])
 
 
+@pytest.mark.parametrize("dim,batch,masked", [(300, 520, False), (96, 5, True)])
+def test_noalloc_takes_a_smaller_plan_where_the_filter_scan_needs_more(gpu, dim, batch, masked):
+    # the filter scan's segments, or its row list, beyond the static array: another plan with the same scores
+    capi = gpu
+    n, k = (18_000_000, 10) if masked else (20_000, 10)
+    if masked:  # codes of any value do
+        codes = np.random.default_rng(61).integers(-127, 128, (n, dim), dtype=np.int8)
+        store = capi.store_desc(capi.DeviceArray.from_host(codes), n, dim, capi.I8, 1.0 / 127.0)
+    else:
+        store = capi.store_desc(capi.DeviceArray.from_host(oracle.f32_to_f16(normalized(n, dim, 61))), n, dim, capi.F16)
+    mask = (np.random.default_rng(62).random(n) < 0.1).astype(np.uint8) if masked else None
+    desc = capi.search_desc(store, capi.DeviceArray.from_host(normalized(batch, dim, 63)), batch, k,
+                            mask=None if mask is None else capi.DeviceArray.from_host(mask))
+    assert capi.search_workspace_bytes(desc) > 64 << 20
+    (exp_idx, exp_val, _), (got_idx, got_val) = _pair(capi, desc)
+    assert np.array_equal(got_idx, exp_idx)
+    assert np.array_equal(got_val.view(np.uint32), exp_val.view(np.uint32))
+
+
 def test_noalloc_rejects_a_search_beyond_the_static_scratch(gpu):
     capi = gpu
     n, dim, batch = 2_000_000, 128, 64

@@ -276,10 +276,6 @@ ScanArgs recoverArgsOf(const zcgvs_search_desc& d, const Plan& plan, std::uint8_
     return scan;
 }
 
-// Workspace of zcgvs_search_topk_noalloc: one library-owned array per device, so a caller that
-// cannot allocate still runs the pipeline. Its size caps the searches that entry point accepts.
-constexpr std::size_t kStaticScratchBytes = std::size_t(64) << 20;
-
 FilterArgs filterArgsOf(const zcgvs_search_desc& d, const Plan& plan, std::uint8_t* ws) {
     FilterArgs args;
     args.operands = ws + plan.filter_operands;
@@ -436,7 +432,9 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
     return n >= 8192 || tiles * components >= 640 + 30 * rounds;
 }
 
-Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
+// The plan of a search. One whose workspace has a fixed size (`limit` bytes) gives up the filter scan
+// where that needs more (its row list, its segments), and the other plans may not.
+Plan makePlan(const zcgvs_search_desc& d, std::size_t limit = ~std::size_t(0), bool allow_filter = true) {
     Plan plan = validate(d);
     if (plan.status != ZCGVS_OK) {
         return plan;
@@ -503,12 +501,7 @@ Plan makePlan(const zcgvs_search_desc& d, bool allow_filter = true) {
         }
         planFilter(d, plan, layout);
         plan.materialized = plan.use_mfma_float = plan.use_mfma = false;
-        if (plan.total <= kStaticScratchBytes) {
-            return plan;
-        }
-        // (a search that fits the no-allocation entry's scratch on another plan still does)
-        const Plan other = makePlan(d, false);
-        return other.total <= kStaticScratchBytes ? other : plan;
+        return plan.total <= limit ? plan : makePlan(d, limit, false);
     }
 
     Layout layout;
@@ -856,6 +849,10 @@ __global__ void zeroWordsKernel(std::uint32_t* __restrict__ dst, std::size_t cou
     }
 }
 
+// Workspace of zcgvs_search_topk_noalloc: one library-owned array per device, so a caller that
+// cannot allocate still runs the pipeline. Its size caps the searches that entry point accepts.
+constexpr std::size_t kStaticScratchBytes = std::size_t(64) << 20;
+
 }  // namespace
 
 }  // namespace zcgvs_hip
@@ -955,14 +952,15 @@ int zcgvs_search_sketch_state(const zcgvs_search_desc* desc, void* d_workspace, 
 
 namespace {
 
+// (limit: makePlan's)
 int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t workspace_bytes,
                int* d_out_indices, float* d_out_values, zcgvs_stream_t stream,
-               zcgvs_event_t* events, int max_phases, int* phases_out) {
+               zcgvs_event_t* events, int max_phases, int* phases_out, std::size_t limit = ~std::size_t(0)) {
     if (desc == nullptr) {
         return setError(ZCGVS_ERR_INVALID_ARGUMENT, "zcgvs: descriptor must not be null");
     }
     const zcgvs_search_desc& d = *desc;
-    const Plan plan = makePlan(d);
+    const Plan plan = makePlan(d, limit);
     if (plan.status != ZCGVS_OK) {
         return setError(plan.status, plan.error);
     }
@@ -1376,7 +1374,7 @@ int zcgvs_search_topk_noalloc(const zcgvs_search_desc* desc, int* d_out_indices,
     if (desc == nullptr) {
         return setError(ZCGVS_ERR_INVALID_ARGUMENT, "zcgvs: descriptor must not be null");
     }
-    const Plan plan = makePlan(*desc);
+    const Plan plan = makePlan(*desc, kStaticScratchBytes);
     if (plan.status != ZCGVS_OK) {
         return setError(plan.status, plan.error);
     }
@@ -1393,7 +1391,7 @@ int zcgvs_search_topk_noalloc(const zcgvs_search_desc* desc, int* d_out_indices,
         return status;
     }
     return searchTopk(desc, address, kStaticScratchBytes, d_out_indices, d_out_values, stream, nullptr, 0,
-                      nullptr);
+                      nullptr, kStaticScratchBytes);
 }
 
 }  // extern "C"
