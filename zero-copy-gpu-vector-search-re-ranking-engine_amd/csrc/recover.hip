@@ -392,7 +392,8 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
         if (++step == check_every) {
             step = 0;
             __syncthreads();
-            const std::uint32_t count = lds_fill;  // uniform: read after the barrier
+            const std::uint32_t count = lds_fill;
+            __syncthreads();  // (before a faster wavefront's next step appends: count is uniform)
             if (count > check_limit) {
                 cutList(count);
                 tau = lds_tau;
