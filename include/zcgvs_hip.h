@@ -406,7 +406,10 @@ int zcgvs_search_overflow_flags(const zcgvs_search_desc* desc, void* d_workspace
  * saw none) and two [batch] threshold keys (a key is kept when it is at least the threshold):
  * the speculative one, ordered32(the *rank-th best slot score) << 32 (for a flagged query the
  * merge replaces it by its rerun's threshold), and the certain one, of the *width-th best slot
- * score. A search that is not sketch-planned sets *slots and *rank to 0 and the addresses to
+ * score. In a filter scan the slot scores are lower bounds of the rows' scores, and both thresholds are
+ * the certain one; where it
+ * runs in two phases the speculative one is the first phase's. A search that is not sketch-planned sets
+ * *slots and *rank to 0 and the addresses to
  * null. For monitoring and tests; no reference counterpart. */
 int zcgvs_search_sketch_state(const zcgvs_search_desc* desc, void* d_workspace, float** d_slot_scores,
                               int* slots, int* rank, int* width, uint64_t** d_tau, uint64_t** d_tau_safe);

@@ -202,6 +202,61 @@ def test_ties_take_the_lowest_rows(gpu, kind, dim, metric):
     assert (val == val[:, :1]).all()
 
 
+def _desc(capi, kind, rows, queries, k, metric, mask=None):
+    """(descriptor, decoded rows, queries as the scan sees them) of a search over `rows`."""
+    n, dim = rows.shape
+    options = dict(mask=None if mask is None else capi.DeviceArray.from_host(mask))
+    d_queries = capi.DeviceArray.from_host(queries)
+    if kind == "i8row":
+        codes, scales = oracle.quantize_rows_i8(rows)
+        store = capi.store_desc(capi.DeviceArray.from_host(codes), n, dim, capi.I8, 1.0, capi.DeviceArray.from_host(scales))
+        options["int8_mode"] = capi.INT8_PER_VECTOR
+        qcodes, qscales = oracle.quantize_rows_i8(queries)
+        return (capi.search_desc(store, d_queries, queries.shape[0], k, metric, **options),
+                oracle.scores_i8i8(codes, scales, qcodes, qscales, mask))
+    stored, dtype, decoded = encode(capi, rows, kind)
+    store = capi.store_desc(capi.DeviceArray.from_host(stored), n, dim, dtype, float(INT8_SCALE) if kind == "i8" else 1.0)
+    return (capi.search_desc(store, d_queries, queries.shape[0], k, metric, **options),
+            oracle.scores_f32(decoded, queries, metric, mask))
+
+
+# Rows that reach a query's threshold by the thousand: a segment that fills is cut to its best keys, so that
+# none overflows, and rows that tie with the threshold are dropped by their numbers.
+@pytest.mark.parametrize("kind,n,dim,batch,k,metric,masked", [
+    ("f16", 100_003, 768, 9, 10, 0, False),
+    ("f16", 60_011, 301, 5, 100, 2, True),
+    ("f32", 100_003, 333, 6, 30, 1, False),
+    ("i8", 100_003, 384, 17, 10, 0, False),
+    ("i8", 50_021, 1024, 5, 200, 1, True),
+    ("i8row", 100_003, 640, 20, 40, 0, False),
+    ("f16", 60_011, 768, 20, 512, 0, False),  # the widest selections: segments of 1024 keys
+])
+@pytest.mark.parametrize("equal", [True, False])
+def test_crowded_thresholds(gpu, kind, n, dim, batch, k, metric, masked, equal):
+    # 40% of the rows are copies of one row, or within the bound's error of it, and half of the queries
+    # are near it
+    capi = gpu
+    rng = np.random.default_rng(75 + dim)
+    rows, queries = normalized(n, dim, 76), normalized(batch, dim, 77)
+    crowd = np.flatnonzero(rng.random(n) < 0.4)
+    noise = np.float32(0.0 if equal else 1e-4 / np.sqrt(dim)) * rng.standard_normal((crowd.size, dim), dtype=np.float32)
+    rows[crowd] = rows[crowd[0]] + noise
+    queries[:batch // 2] = rows[crowd[0]] + np.float32(0.05) * queries[:batch // 2]
+    mask = (rng.random(n) < 0.5).astype(np.uint8) if masked else None
+    desc, ref = _desc(capi, kind, rows, queries, k, metric, mask)
+    idx, val, flags = capi.search(desc)
+    assert not flags.any()
+    if equal and kind != "i8row":  # (the oracle's ties are the scan's)
+        best = crowd if mask is None else crowd[mask[crowd] != 0]
+        assert (idx[:batch // 2] == best[:k]).all()
+    if kind == "i8row":
+        assert_topk_equivalent(idx, val, ref, k)
+    else:
+        desc.flags = capi.SEARCH_FORCE_EXACT_PASS
+        exact = capi.search(desc)
+        assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
+
+
 def test_non_finite(gpu):
     # infinite and NaN components follow the float32 sum: +inf ranks first, NaN last; a query with a
     # NaN scores NaN everywhere and takes the lowest rows

@@ -1,9 +1,9 @@
-// The filter scan's kernel (filter.hpp); filter_f32.hip, filter_f16.hip and filter_i8.hip
-// instantiate it for their row type.
+// The filter scan's kernel (filter.hpp); filter_{f32,f16,i8,i8i8}_{narrow,wide}.hip instantiate it for
+// their row type and width.
 //
 // Work split. One workgroup of 8 wavefronts per compute unit. The launch's query operands (up to
 // 8 groups of 16 queries) lie in LDS for the whole launch; every wavefront streams rows of its own
-// straight into registers, in the layout the matrix core wants, so no barrier runs in the loop. A
+// straight into registers, so no barrier runs in the loop (but for the cuts of a crowded search). A
 // wavefront's tile is kBlocks blocks of 16 rows, of which it keeps kPieces pieces of 256 bytes of
 // every row in flight (whole rows up to 1 KB), four 16-byte loads a lane, block and piece: as it
 // consumes a load it starts the same one of the next tile. That is 8 to 16 KB of consecutive
@@ -18,8 +18,8 @@
 // the whole search, the bf16 split scan 1.3): 1M x 768 float16, 32 queries, k = 100 272 us (5.6 of
 // the 7.07 TB/s a streaming read reaches), 1M x 384 float32, 64 queries 263 us (5.8), 500,009 x 256
 // float32 L2 87 us, 400,009 x 300 float16 49 us (4.9), 300,000 allowed rows of 1M x 384 float16 42 us
-// (5.5), 1M x 384 int8, 8 queries 94 us (4.1: it also converts its codes
-// to halves). A ring of more registers (6 and 8 pieces) made the compiler spill: 297-310 us for the
+// (5.5), 1M x 384 int8, 8 queries 77 us (5.0: it also converts its codes to halves; 94 while the
+// exact scores held all of a query's chunks and spilled registers). A ring of more registers (6 and 8 pieces) made the compiler spill: 297-310 us for the
 // first; tiles of 64 rows a piece at a time 577 us.
 //
 // MFMA layout (16x16x32 f16): the queries are the first operand (lane l supplies query l % 16 and 8
@@ -125,42 +125,47 @@ __device__ __forceinline__ float exactScoreLanes(const ScanArgs& scan, std::uint
     const std::uint8_t* base = static_cast<const std::uint8_t*>(scan.corpus) + static_cast<std::size_t>(row) * row_bytes;
     const float* query = static_cast<const float*>(scan.queries) + static_cast<std::size_t>(q) * dim;
     const bool l2 = scan.metric == ZCGVS_METRIC_L2;
-    // (every load without a branch, so that all are in flight together; the opaque copy keeps their
-    // addresses from being computed, and kept in memory, outside the caller's loop)
-    v4u raw[kPer];
+    // (every load of a turn without a branch, so that all are in flight together; the opaque copy keeps
+    // their addresses from being computed, and kept in memory, outside the caller's loop. int8 takes two
+    // turns: a chunk's 16 query values fill the registers)
+    constexpr int kTurn = kKind == ZCGVS_DTYPE_I8 ? kPer / 2 : kPer;
     int group = lane % L;
     asm volatile("" : "+v"(group));
+    float acc = 0.0f;
+#pragma unroll 1
+    for (int first = 0; first < kPer && first * L < chunks; first += kTurn) {
+        v4u raw[kTurn];
 #pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-        if (t * L < chunks) {  // (uniform)
-            raw[t] = loadRowChunk<false>(base + min(group + t * L, chunks - 1) * 16);
+        for (int t = 0; t < kTurn; ++t) {
+            if ((first + t) * L < chunks) {  // (uniform)
+                raw[t] = loadRowChunk<false>(base + min(group + (first + t) * L, chunks - 1) * 16);
+            }
         }
-    }
-    float qe[kPer][E];
+        float qe[kTurn][E];
 #pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-        if (t * L < chunks) {  // (uniform)
-            const float* qv = query + min((group + t * L) * E, dim - E);
+        for (int t = 0; t < kTurn; ++t) {
+            if ((first + t) * L < chunks) {  // (uniform)
+                const float* qv = query + min((group + (first + t) * L) * E, dim - E);
 #pragma unroll
-            for (int e = 0; e < E; e += 4) {
-                const v4f part = *reinterpret_cast<const v4fAny*>(qv + e);
+                for (int e = 0; e < E; e += 4) {
+                    const v4f part = *reinterpret_cast<const v4fAny*>(qv + e);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    qe[t][e + i] = part[i];
+                    for (int i = 0; i < 4; ++i) {
+                        qe[t][e + i] = part[i];
+                    }
                 }
             }
         }
-    }
-    float acc = 0.0f;
 #pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-        if (group + t * L < chunks) {
-            float v[E];
-            Traits::decode(make_uint4(raw[t][0], raw[t][1], raw[t][2], raw[t][3]), scan.scale, v);
+        for (int t = 0; t < kTurn; ++t) {
+            if (group + (first + t) * L < chunks) {
+                float v[E];
+                Traits::decode(make_uint4(raw[t][0], raw[t][1], raw[t][2], raw[t][3]), scan.scale, v);
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const float d = l2 ? qe[t][e] - v[e] : v[e];
-                acc = fmaf(l2 ? d : qe[t][e], d, acc);
+                for (int e = 0; e < E; ++e) {
+                    const float d = l2 ? qe[t][e] - v[e] : v[e];
+                    acc = fmaf(l2 ? d : qe[t][e], d, acc);
+                }
             }
         }
     }
@@ -258,8 +263,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     __shared__ __attribute__((aligned(16))) float lds_inverse[kLex ? kQueries : 4];  // 1 / largest lexical score
     __shared__ std::uint64_t lds_tau[kQueries];
     __shared__ std::uint32_t lds_count[kQueries];
-    __shared__ std::uint64_t lds_lowest[kQueries];  // the lowest of the first `width` keys appended
-    __shared__ std::uint32_t lds_placed[kQueries];  // how many of those it covers
+    __shared__ std::uint32_t lds_asked[2];  // a wavefront asks for a cut of the segments (in turns)
     __shared__ __attribute__((aligned(16))) std::uint8_t lds_stage[kFilterWaves][kFilterBlockRows * kPieceBytes / 2];
     __shared__ uint2 lds_park[kFilterWaves][kParkSlots];
 
@@ -384,7 +388,9 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     const float root_dim = sqrtf(static_cast<float>(dim));
     const float floor_abs = kF32 ? root_dim * 5.97e-8f : kF16 ? root_dim * 6.2e-5f * relative : 0.0f;
     const float norm_abs = unit * unit * static_cast<float>(dim) * 3.8e-9f;
-    for (int i = tid; i < kQueries; i += kFilterThreads) {
+    // The constants of query i and, in a threshold phase, its threshold `tau` (those are written again
+    // when a cut raises it).
+    auto setQuery = [&](int i, std::uint64_t tau) __attribute__((always_inline)) {
         const bool valid = i < q_count;
         const FilterQuery query = args.queries[q_offset + i];
         const float qnorm = sqrtf(query.norm2) * 1.00001f;
@@ -392,18 +398,14 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         // an exact sum may overflow on its way to a value the approximation has in range)
         const float reach = kF32 ? 65504.0f * unit : 0.0f;  // of a row that is not unbounded
         const bool usable = query.usable != 0.0f && (l2 ? (qnorm + reach) * (qnorm + reach) : qnorm * reach) < 1e38f;
+        bool gated = false;
+        const float floor_score = keyFloor(tau, &gated);
+        lds_tau[i] = tau;
         if constexpr (kInteger) {
             // score = acc * (query scale * row scale), compared with the threshold's itself
-            bool gated = false;
-            const std::uint64_t tau = valid && !sketch ? emit.tau[q_offset + i] : ~0ull;
-            const float floor_score = keyFloor(tau, &gated);
             lds_gain[i] = valid ? query.scale : __uint_as_float(0x7FC00000u);
             lds_slope[i] = query.scale;
             lds_base[i] = !valid ? INFINITY : gated && floor_score > kMaskedScore ? floor_score : -INFINITY;
-            lds_tau[i] = tau;
-            lds_count[i] = 0u;
-            lds_lowest[i] = ~0ull;
-            lds_placed[i] = 0u;
         } else if (kLex || sketch) {
             // a bound of the score (hybrid: of its dense part; an upper one in a threshold phase) =
             // gain * acc + slope * row term + base
@@ -421,22 +423,12 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             lds_slope[i] = slope;
             lds_base[i] = base;
             if constexpr (kLex) {
-                bool gated = false;
-                const std::uint64_t tau = valid && !sketch ? emit.tau[q_offset + i] : ~0ull;
-                const float floor_score = keyFloor(tau, &gated);
                 lds_floor[i] = !valid ? INFINITY : gated ? floor_score : -INFINITY;
                 const float peak = valid ? scan.lexical_max[q_offset + i] : 0.0f;
                 lds_inverse[i] = peak > 0.0f ? 1.0f / peak : 0.0f;
-                lds_tau[i] = tau;
-                lds_count[i] = 0u;
-                lds_lowest[i] = ~0ull;
-                lds_placed[i] = 0u;
             }
         } else {
             // a pair survives unless acc < slope * row term + base
-            bool gated = false;
-            const std::uint64_t tau = valid ? emit.tau[q_offset + i] : ~0ull;
-            const float floor_score = keyFloor(tau, &gated);
             const float to_acc = query.scale / unit;  // dot product -> accumulator
             float slope = -relative * qnorm * query.scale;
             float base = to_acc * floor_score - qnorm * query.scale * floor_abs;
@@ -451,11 +443,14 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             // (a query past the batch takes no pair: nothing but NaN fails acc < inf, and those
             // pairs are dropped by its threshold key)
             lds_base[i] = !valid ? INFINITY : filter ? base : -INFINITY;
-            lds_tau[i] = tau;
-            lds_count[i] = 0u;
-            lds_lowest[i] = ~0ull;
-            lds_placed[i] = 0u;
         }
+    };
+    for (int i = tid; i < kQueries; i += kFilterThreads) {
+        lds_count[i] = 0u;
+        setQuery(i, i < q_count && !sketch ? emit.tau[q_offset + i] : ~0ull);
+    }
+    if (tid < 2) {
+        lds_asked[tid] = 0u;
     }
     __syncthreads();
 
@@ -590,9 +585,98 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         }
     };
 
+    // ---- cuts ----
+    // A workgroup's segment of a query holds more keys than are selected, and a full one is cut to its
+    // `width` best, the last of which becomes the workgroup's threshold: no row whose key is lower can
+    // be selected any more. So rows that tie, or come close, by the thousand do not overflow the segments,
+    // after which the exact fallback would sweep the corpus at one compute unit's rate (1M rows, 30% of
+    // them copies of the row that 4 queries seek: float16 x 768, 32 queries 41.9 ms, now 0.83; per-vector
+    // int8, 16 queries 14.5, now 0.26; rows within 2% of 16 topics, float16 42.3, now 1.98).
+    // A cut is made by all wavefronts together, each for queries of its own: one that finds a segment
+    // full asks for it and waits; the others look once a tile (and between the exact scores) and, when
+    // done with their rows, wait until all are.
+    const std::uint32_t capacity = 1u << emit.seg_log2;
+    const std::uint32_t width = static_cast<std::uint32_t>(args.width);
+    const bool cuts = capacity > width;  // (not with the segments that a test makes too small)
+    std::uint32_t turn = 0u;             // cuts made: the same in all wavefronts between two barriers
+    auto askedForCut = [&]() __attribute__((always_inline)) -> std::uint32_t {
+        return __hip_atomic_load(&lds_asked[turn & 1u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    auto segmentOf = [&](int q) __attribute__((always_inline)) -> std::uint64_t* {
+        return emit.seg + ((static_cast<std::size_t>(blockIdx.x) * scan.batch + q_offset + q) << emit.seg_log2);
+    };
+    // Query q's full segment, by one wavefront, which holds its keys in registers and finds the width-th
+    // best of them bit by bit.
+    auto cutSegment = [&](int q) __attribute__((always_inline)) {
+        std::uint64_t* seg = segmentOf(q);
+        std::uint64_t key[kFilterSegmentKeys / kWave];
+#pragma unroll
+        for (int r = 0; r < kFilterSegmentKeys / kWave; ++r) {
+            // (past the compute unit's cache: the other wavefronts' stores have reached the next one)
+            key[r] = static_cast<std::uint32_t>(r * kWave) < capacity
+                         ? __hip_atomic_load(seg + r * kWave + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                         : 0ull;
+        }
+        std::uint64_t cut = 0ull;
+#pragma unroll 1
+        for (int bit = 63; bit >= 0; --bit) {
+            const std::uint64_t candidate = cut | 1ull << bit;
+            std::uint32_t above = 0u;
+#pragma unroll
+            for (int r = 0; r < kFilterSegmentKeys / kWave; ++r) {
+                if (static_cast<std::uint32_t>(r * kWave) < capacity) {  // (uniform)
+                    above += static_cast<std::uint32_t>(__popcll(__ballot(key[r] >= candidate)));
+                }
+            }
+            cut = above >= width ? candidate : cut;
+        }
+        std::uint32_t kept = 0u;
+#pragma unroll
+        for (int r = 0; r < kFilterSegmentKeys / kWave; ++r) {
+            if (static_cast<std::uint32_t>(r * kWave) < capacity) {
+                const unsigned long long take = __ballot(key[r] >= cut);
+                const std::uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                    static_cast<std::uint32_t>(take >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<std::uint32_t>(take), 0u));
+                if (key[r] >= cut) {
+                    seg[kept + below] = key[r];
+                }
+                kept += static_cast<std::uint32_t>(__popcll(take));
+            }
+        }
+        if (lane == 0) {
+            lds_count[q] = width;
+            setQuery(q, cut);
+        }
+    };
+    // By every wavefront: waits for all of them and, if one asked, cuts the full segments. False: none
+    // asked, so all are done with their rows.
+    auto waitForCut = [&](bool ask) __attribute__((always_inline)) -> bool {
+        if (ask) {
+            __hip_atomic_store(&lds_asked[turn & 1u], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's keys have left the compute unit
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(askedForCut()) == 0u) {
+            return false;
+        }
+#pragma unroll 1
+        for (int q = wave; q < q_count; q += kFilterWaves) {
+            if (__builtin_amdgcn_readfirstlane(lds_count[q]) >= capacity) {
+                cutSegment(q);
+            }
+        }
+        // (nobody reads the other turn's word between these two barriers)
+        if (tid == 0) {
+            __hip_atomic_store(&lds_asked[(turn + 1u) & 1u], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        ++turn;
+        __syncthreads();
+        return true;
+    };
+
     // ---- exact scores, a row per group of lanes_per_row lanes ----
-    // The pair (row as listed, query of the launch) of this lane's group; `take` clear: no pair.
-    auto scorePair = [&](std::uint32_t listed, int q, bool take) __attribute__((always_inline)) {
+    // The key of a pair (row as listed, query of the launch), on every lane of the group.
+    auto keyOfPair = [&](std::uint32_t listed, int q) __attribute__((always_inline)) -> std::uint64_t {
         const std::uint32_t row = listed & ~kMaskedRow;
         const int query = min(q_offset + q, scan.batch - 1);  // (a query past the batch parks NaN pairs only)
         float score = exactScore<kKind>(scan, row, query, lane, lanes_per_row);
@@ -603,22 +687,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         if (args.infinite_as_nan != 0 && scan.batch - query / 128 * 128 >= 32 && fabsf(score) == INFINITY) {
             score = __uint_as_float(0x7FC00000u);
         }
-        const std::uint64_t key = makeKey((listed & kMaskedRow) != 0u ? kMaskedScore : score, row);
-        if (take && lane % lanes_per_row == 0 && key > lds_tau[q]) {
-            const std::uint32_t slot = atomicAdd(&lds_count[q], 1u);
-            if (slot < (1u << emit.seg_log2)) {
-                emit.seg[((static_cast<std::size_t>(blockIdx.x) * scan.batch + q_offset + q) << emit.seg_log2) + slot] = key;
-            }
-            // Once the workgroup holds `width` keys of a query, no key below the lowest of them can be
-            // selected any more: rows that tie by the thousand (copies of one row) stop filling the
-            // segment.
-            if (slot < static_cast<std::uint32_t>(args.width)) {
-                atomicMin(&lds_lowest[q], key);
-                if (atomicAdd(&lds_placed[q], 1u) + 1u == static_cast<std::uint32_t>(args.width)) {
-                    lds_tau[q] = max(lds_tau[q], lds_lowest[q]);
-                }
-            }
-        }
+        return makeKey((listed & kMaskedRow) != 0u ? kMaskedScore : score, row);
     };
     const int per_round = kWave / lanes_per_row;
 
@@ -632,7 +701,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     // the stream's registers free; a tile whose pairs do not fit (or would not even an empty park) is
     // streamed again (scored whole) after it.
     bool crowded = false;
-    while (tile < tiles) {
+    while (true) {
         while (tile < tiles) {
             const long long next = tile + waves;
             std::uint32_t id[kBlocks];  // this lane's rows in the results
@@ -681,6 +750,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             // ---- the tile's scores (the thresholds are read again for every tile: kept, they would
             //      take the accumulators' registers) ----
             asm volatile("" ::: "memory");
+            const std::uint32_t asked = askedForCut();
             float term[kBlocks];
             bool live[kBlocks], masked[kBlocks];
 #pragma unroll
@@ -702,18 +772,25 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 masked[b] = list != nullptr && (id[b] & kMaskedRow) != 0u;
             }
             // Whether the pair of block b's row and query 16 g + 4 h + i can reach the query's threshold.
-            // (A masked row does where every row does; a NaN survives.)
-            auto survives = [&](int b, int g, int i, const v4f& slope, const v4f& offset) __attribute__((always_inline)) -> bool {
+            // (A masked row does where every row does; a NaN survives.) `tie`: its score is no better than
+            // the threshold's, so that the row numbers decide.
+            auto survives = [&](int b, int g, int i, const v4f& slope, const v4f& offset,
+                                bool& tie) __attribute__((always_inline)) -> bool {
                 if constexpr (kLex) {
                     const int q = kFilterGroup * g + 4 * h + i;
                     const float bound = fmaf(lds_gain[q], acc[b][g][i], fmaf(slope[i], term[b], offset[i]));
-                    return !(fuseHybrid(bound, lexical[b][g][i], scan.dense_weight, lds_inverse[q]) < lds_floor[q]);
+                    const float fused = fuseHybrid(bound, lexical[b][g][i], scan.dense_weight, lds_inverse[q]);
+                    tie = fused == lds_floor[q] && fused > -INFINITY;
+                    return !(fused < lds_floor[q]);
                 } else if constexpr (kInteger) {
                     const float score = static_cast<float>(acc[b][g][i]) * (slope[i] * term[b]);
+                    tie = !masked[b] && score == offset[i] && score > -INFINITY;
                     return masked[b] ? offset[i] == -INFINITY : !(score < offset[i]);
                 } else {
                     const float sum = masked[b] ? -INFINITY : acc[b][g][i];
-                    return !(sum < fmaf(slope[i], masked[b] ? 0.0f : term[b], offset[i]));
+                    const float edge = fmaf(slope[i], masked[b] ? 0.0f : term[b], offset[i]);
+                    tie = false;
+                    return !(sum < edge);
                 }
             };
             if (sketch) {
@@ -749,7 +826,8 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                         bool here = false;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            here |= survives(b, g, i, slope, offset);
+                            bool tie;
+                            here |= survives(b, g, i, slope, offset, tie);
                         }
                         any |= here && live[b];
                     }
@@ -767,12 +845,30 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                         const v4f slope = *reinterpret_cast<const v4f*>(&lds_slope[kFilterGroup * g + 4 * h]);
                         const v4f offset = *reinterpret_cast<const v4f*>(&lds_base[kFilterGroup * g + 4 * h]);
                         survivors[g] = 0u;
+                        std::uint32_t ties = 0u;
 #pragma unroll
                         for (int b = 0; b < kBlocks; ++b) {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
-                                if (live[b] && survives(b, g, i, slope, offset)) {
+                                bool tie;
+                                if (live[b] && survives(b, g, i, slope, offset, tie)) {
                                     survivors[g] |= 1u << (4 * b + i);
+                                    ties |= tie ? 1u << (4 * b + i) : 0u;
+                                }
+                            }
+                        }
+                        while ((kLex || kInteger) && __any(ties != 0u)) {
+                            if (ties != 0u) {
+                                const int bit = __ffs(ties) - 1;
+                                ties &= ties - 1u;
+                                std::uint32_t tied = id[0];
+#pragma unroll
+                                for (int b = 1; b < kBlocks; ++b) {
+                                    tied = (bit >> 2) == b ? id[b] : tied;
+                                }
+                                const std::uint64_t tau = lds_tau[kFilterGroup * g + 4 * h + (bit & 3)];
+                                if (makeKey(keyScore(tau), tied) <= tau) {
+                                    survivors[g] &= ~(1u << bit);
                                 }
                             }
                         }
@@ -822,27 +918,68 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 row[b][0] = next_row[b][0];
                 row[b][1] = next_row[b][1];
             }
-        }
-        if (crowded) {
-            // every pair of the tile, its rows from the list or the tile's place
-            const int tile_rows = kBlocks * kFilterBlockRows;
-            for (int first = 0; first < tile_rows * q_count; first += per_round) {
-                const int pair = first + lane / lanes_per_row;
-                const long long at = tileAt(tile) * tile_rows + pair % tile_rows;
-                const bool take = pair < tile_rows * q_count && at < rows;
-                const long long place = min(at, rows - 1);
-                scorePair(list != nullptr ? list[place] : static_cast<std::uint32_t>(place),
-                          min(pair / tile_rows, q_count - 1), take);
+            if (__builtin_amdgcn_readfirstlane(asked) != 0u) {
+                break;
             }
-            crowded = false;
-            tile += waves;
         }
-        for (std::uint32_t first = 0; first < parked; first += static_cast<std::uint32_t>(per_round)) {
-            const std::uint32_t e = first + static_cast<std::uint32_t>(lane / lanes_per_row);
-            const uint2 pair = lds_park[wave][min(e, parked - 1u)];
-            scorePair(pair.x, static_cast<int>(pair.y), e < parked);
+        // The exact scores of the parked pairs and, of a crowded tile, of every pair (its rows from the list
+        // or the tile's place). A key that finds its segment full waits for a cut.
+        constexpr int kTileRows = kBlocks * kFilterBlockRows;
+        const std::uint32_t total = parked + (crowded ? static_cast<std::uint32_t>(kTileRows * q_count) : 0u);
+        const long long tile_row = tileAt(tile) * kTileRows;  // (not used past the last tile)
+        tile += crowded ? waves : 0;
+        const bool done = tile >= tiles;
+        std::uint32_t first = 0u;
+        std::uint64_t key = 0ull;
+        int q = 0;
+        bool waits = false;
+        bool over = false;
+#pragma unroll 1
+        while (true) {
+            if (first < total && !__any(waits)) {
+                const std::uint32_t e = first + static_cast<std::uint32_t>(lane / lanes_per_row);
+                const uint2 pair = lds_park[wave][min(e, max(parked, 1u) - 1u)];  // (the last one's again past them)
+                std::uint32_t listed = pair.x;
+                q = static_cast<int>(pair.y);
+                waits = e < total;
+                if (crowded && e >= parked) {
+                    const std::uint32_t at = min(e, total - 1u) - parked;
+                    const long long place = tile_row + at % kTileRows;
+                    waits = waits && place < rows;
+                    listed = static_cast<std::uint32_t>(min(place, rows - 1));
+                    listed = list != nullptr ? list[listed] : listed;
+                    q = static_cast<int>(at / kTileRows);
+                }
+                key = keyOfPair(listed, q);
+                waits = waits && lane % lanes_per_row == 0;
+                first += static_cast<std::uint32_t>(per_round);
+            }
+            waits = waits && key > lds_tau[q];
+            if (waits) {
+                const std::uint32_t slot = atomicAdd(&lds_count[q], 1u);
+                if (slot < capacity) {
+                    segmentOf(q)[slot] = key;
+                }
+                waits = slot >= capacity && cuts;
+            }
+            const bool ask = __any(waits);
+            if (!ask && first < total) {
+                continue;
+            }
+            if (!ask && !done && __builtin_amdgcn_readfirstlane(askedForCut()) == 0u) {
+                break;
+            }
+            // (a cut leaves room for capacity - width keys, or a threshold above the ones that wait)
+            if (!waitForCut(ask)) {
+                over = true;
+                break;
+            }
         }
         parked = 0u;
+        crowded = false;
+        if (over) {
+            break;
+        }
         readRows(tile, row);  // (past the last tile too: with a branch the ring would be kept across all this)
         issueTile(row);
     }
@@ -861,7 +998,6 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
             }
         }
     } else {
-        __syncthreads();
         for (int i = tid; i < q_count; i += kFilterThreads) {
             emit.seg_count[static_cast<std::size_t>(blockIdx.x) * scan.batch + q_offset + i] = lds_count[i];
         }

@@ -341,8 +341,10 @@ void planFilter(const zcgvs_search_desc& d, Plan& plan, Layout& layout) {
         plan.phases = {sketch, scan};
     }
     plan.recover = true;
+    // A segment holds four times the keys that the sample's threshold lets through on average, if that
+    // is no more than kFilterSegmentKeys, and some more than are selected, so that a full one can be cut.
     const long long expected = plan.width * sketch.stride / plan.segments;
-    plan.seg_log2 = std::max(6, ceilLog2(4 * expected + 16));
+    plan.seg_log2 = std::min(ceilLog2(kFilterSegmentKeys), std::max({6, ceilLog2(4 * expected + 16), ceilLog2(plan.width + 24)}));
     if ((d.flags & ZCGVS_SEARCH_TEST_TINY_SEGMENTS) != 0) {
         plan.seg_log2 = 1;
     }
