@@ -407,7 +407,7 @@ int zcgvs_search_overflow_flags(const zcgvs_search_desc* desc, void* d_workspace
  * the speculative one, ordered32(the *rank-th best slot score) << 32 (for a flagged query the
  * merge replaces it by its rerun's threshold), and the certain one, of the *width-th best slot
  * score. In a filter scan the slot scores are lower bounds of the rows' scores, and both thresholds are
- * the certain one; where it
+ * the certain one (of all ones for a query of zeros, which that scan leaves to the last merge); where it
  * runs in two phases the speculative one is the first phase's. A search that is not sketch-planned sets
  * *slots and *rank to 0 and the addresses to
  * null. For monitoring and tests; no reference counterpart. */

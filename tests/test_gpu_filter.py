@@ -4,6 +4,8 @@ does. Sizes at its edges: rows of one chunk to 4 KB, whole and partial 256-byte 
 halves and 16-byte chunks, one and several rounds of pieces; one query to several launches; row
 counts that end in a partial block; masks that let through everything, some, and fewer rows than k."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -202,6 +204,20 @@ def test_ties_take_the_lowest_rows(gpu, kind, dim, metric):
     assert (val == val[:, :1]).all()
 
 
+def _seconds(capi, desc):
+    """Best of four passes over a workspace that is there."""
+    size = capi.search_workspace_bytes(desc)
+    workspace = capi.DeviceArray(size, np.uint8)
+    idx, val = capi.DeviceArray((desc.batch, desc.k), np.int32), capi.DeviceArray((desc.batch, desc.k), np.float32)
+    best = np.inf
+    for _ in range(5):
+        begin = time.perf_counter()
+        capi.search_topk(desc, workspace, size, idx, val)
+        capi.synchronize()
+        best = min(best, time.perf_counter() - begin)
+    return best
+
+
 def _desc(capi, kind, rows, queries, k, metric, mask=None):
     """(descriptor, decoded rows, queries as the scan sees them) of a search over `rows`."""
     n, dim = rows.shape
@@ -255,6 +271,34 @@ def test_crowded_thresholds(gpu, kind, n, dim, batch, k, metric, masked, equal):
         desc.flags = capi.SEARCH_FORCE_EXACT_PASS
         exact = capi.search(desc)
         assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
+
+
+# A query of zeros scores every row 0 and takes the lowest ones: a batch padded with such queries costs
+# about what the others do.
+@pytest.mark.parametrize("kind,dim,batch,zeros,metric,share", [
+    ("f16", 768, 16, 7, 0, None), ("f16", 300, 5, 5, 1, 0.3), ("f32", 333, 6, 1, 0, None), ("f32", 640, 64, 32, 1, 0.02),
+    ("i8", 384, 8, 4, 0, None), ("i8row", 768, 16, 8, 0, None), ("i8row", 640, 100, 64, 0, 0.0), ("f16", 768, 9, 3, 2, None),
+])
+def test_queries_of_zeros(gpu, kind, dim, batch, zeros, metric, share):
+    capi = gpu
+    n, k = 100_003, 10
+    rows, queries = normalized(n, dim, 78), normalized(batch, dim, 79)
+    mask = None
+    if share is not None:
+        mask = (np.random.default_rng(80).random(n) < share).astype(np.uint8)
+        mask[[70_000, n - 1]] = 1
+    plain, _ = _desc(capi, kind, rows, queries, k, metric, mask)
+    queries[::batch // zeros][:zeros] = 0.0
+    if kind != "i8row":
+        rows[2, 1] = np.nan if kind == "f32" else 0.0  # a row whose score is no zero
+    desc, ref = _desc(capi, kind, rows, queries, k, metric, mask)
+    idx, val, _ = capi.search(desc)
+    if kind == "i8row":
+        assert_topk_equivalent(idx, val, ref, k)
+    else:
+        decoded = encode(capi, rows, kind)[2]
+        assert_topk_equivalent(idx, val, ref, k, np.nan_to_num(float_tolerance(queries, decoded, metric)))
+    assert _seconds(capi, desc) < 10 * _seconds(capi, plain)
 
 
 def test_non_finite(gpu):

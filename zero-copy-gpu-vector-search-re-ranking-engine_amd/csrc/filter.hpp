@@ -49,8 +49,15 @@ struct FilterQuery {
     float scale;  // the power of two the operands were multiplied by; per-vector int8: the query's scale
     float norm2;  // sum q_j^2
     float usable; // 0: not finite or out of range, every pair is scored exactly
-    float pad;
+    // 1: all zero, under a metric by which every finite row then scores 0, so that the row numbers decide
+    // (a batch padded to its size, say). The scan takes no pair of such a query; the last merge, which
+    // finds too few keys, sweeps the rows from the first on until enough score 0 (recover.hip). In the
+    // scan every row would reach its threshold: 1M x 384 float32, 64 queries, 32 of them zero 14.0 ms,
+    // now 0.34; with one 25.9, now 0.35.
+    float zero;
 };
+// Threshold of a query that the scan leaves out.
+constexpr std::uint64_t kFilterNoKey = ~0ull;
 
 struct FilterArgs {
     std::uint8_t* operands = nullptr;  // [groups][steps][64 lanes][16 bytes]
@@ -91,7 +98,7 @@ inline long long filterMaskedRows(long long rows, int width) { return rows < 2LL
 // The query operands, the row unit and, with a mask, the row list.
 int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_t stream);
 // After a sketch phase: tau[q] (and tau_safe[q]), a key below the width-th best of query q's rows.
-int launchFilterThreshold(const float* sketch, int slots, int batch, int width, std::uint64_t* tau,
+int launchFilterThreshold(const FilterArgs& args, const float* sketch, int slots, int batch, std::uint64_t* tau,
                           std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream);
 // A sketch phase (emit.sketch: the best certain lower bound of every slot's rows; items of 16 rows)
 // or a threshold phase (items of tile_rows rows; over every listed row when there is a row list).

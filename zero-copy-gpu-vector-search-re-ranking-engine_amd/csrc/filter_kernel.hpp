@@ -391,7 +391,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     // The constants of query i and, in a threshold phase, its threshold `tau` (those are written again
     // when a cut raises it).
     auto setQuery = [&](int i, std::uint64_t tau) __attribute__((always_inline)) {
-        const bool valid = i < q_count;
+        const bool valid = i < q_count && (sketch || tau != kFilterNoKey);
         const FilterQuery query = args.queries[q_offset + i];
         const float qnorm = sqrtf(query.norm2) * 1.00001f;
         // (a score, and every partial sum of one, is bounded by the norms: where that is beyond float32,
@@ -447,7 +447,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     };
     for (int i = tid; i < kQueries; i += kFilterThreads) {
         lds_count[i] = 0u;
-        setQuery(i, i < q_count && !sketch ? emit.tau[q_offset + i] : ~0ull);
+        setQuery(i, i < q_count && !sketch ? emit.tau[q_offset + i] : kFilterNoKey);
     }
     if (tid < 2) {
         lds_asked[tid] = 0u;

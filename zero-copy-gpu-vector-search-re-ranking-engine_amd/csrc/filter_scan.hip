@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kPrepareThreads) void filterPrepareKernel(ScanArgs 
                 // (within these bounds no square, product or scaled threshold leaves float32's range
                 // unnoticed; an all-zero query is in them)
                 out.usable = finite && (peak == 0.0f || (peak > 1e-17f && peak < 1e17f)) ? 1.0f : 0.0f;
-                out.pad = 0.0f;
+                out.zero = finite && peak == 0.0f && scan.metric != ZCGVS_METRIC_L2 && scan.lexical == nullptr ? 1.0f : 0.0f;
                 args.queries[group * kFilterGroup + t / 16] = out;
             }
         }
@@ -180,7 +180,8 @@ constexpr int kThresholdThreads = 512;
 constexpr int kThresholdBins = 2048;
 constexpr int kThresholdSlots = kMaxSketchSlots / kThresholdThreads;
 
-__global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(const float* __restrict__ sketch, int slots,
+__global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(const FilterQuery* __restrict__ queries,
+                                                                           const float* __restrict__ sketch, int slots,
                                                                            int batch, int width,
                                                                            std::uint64_t* __restrict__ tau,
                                                                            std::uint64_t* __restrict__ tau_safe,
@@ -208,6 +209,13 @@ __global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(const
     }
     if (q == 0 && t == 0) {
         *flag_count = 0u;
+    }
+    if (queries[q].zero != 0.0f) {  // (uniform)
+        if (t == 0) {
+            tau[q] = kFilterNoKey;
+            tau_safe[q] = kFilterNoKey;
+        }
+        return;
     }
 #pragma unroll
     for (int m = kWave / 2; m > 0; m >>= 1) {
@@ -272,12 +280,27 @@ __global__ __launch_bounds__(kPrepareThreads) void filterPrepareCodesKernel(Scan
     if (group == 0 && blockIdx.y == 0 && t == 0 && args.list_count != nullptr) {
         *args.list_count = 0u;
     }
-    if (blockIdx.y == 0 && t < kFilterGroup) {
-        const int q = group * kFilterGroup + t;
-        FilterQuery out = {};
-        out.scale = q < scan.batch ? scan.query_scales[q] : 0.0f;
-        out.usable = 1.0f;
-        args.queries[q] = out;
+    if (blockIdx.y == 0) {
+        // 16 threads per query
+        const int q = group * kFilterGroup + t / 16;
+        const std::uint8_t* src = static_cast<const std::uint8_t*>(scan.queries) + static_cast<std::size_t>(min(q, scan.batch - 1)) * scan.dim;
+        std::uint32_t any = 0u;
+#pragma unroll 4
+        for (int c = t & 15; c < chunks; c += 16) {
+            const u32x4 codes = *reinterpret_cast<const u32x4*>(src + 16 * c);
+            any |= codes[0] | codes[1] | codes[2] | codes[3];
+        }
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1) {
+            any |= waveXor(any, m);
+        }
+        if ((t & 15) == 0) {
+            FilterQuery out = {};
+            out.scale = q < scan.batch ? scan.query_scales[q] : 0.0f;
+            out.usable = 1.0f;
+            out.zero = any == 0u ? 1.0f : 0.0f;
+            args.queries[q] = out;
+        }
     }
     u32x4* dst = reinterpret_cast<u32x4*>(args.operands) + static_cast<std::size_t>(group) * args.steps * kWave;
     for (int item = static_cast<int>(blockIdx.y) * kPrepareThreads + t; item < args.steps * kWave;
@@ -421,12 +444,13 @@ int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_
     return ZCGVS_OK;
 }
 
-int launchFilterThreshold(const float* sketch, int slots, int batch, int width, std::uint64_t* tau,
+int launchFilterThreshold(const FilterArgs& args, const float* sketch, int slots, int batch, std::uint64_t* tau,
                           std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream) {
-    if (slots < 1 || slots > kMaxSketchSlots || width < 1) {
+    if (slots < 1 || slots > kMaxSketchSlots || args.width < 1) {
         return setError(ZCGVS_ERR_RUNTIME, "zcgvs filter: sketch shape out of range");
     }
-    filterThresholdKernel<<<batch, kThresholdThreads, 0, stream>>>(sketch, slots, batch, width, tau, tau_safe, flag_count);
+    filterThresholdKernel<<<batch, kThresholdThreads, 0, stream>>>(args.queries, sketch, slots, batch, args.width, tau,
+                                                                   tau_safe, flag_count);
     ZCGVS_LAUNCH_CHECK("filter threshold");
     return ZCGVS_OK;
 }

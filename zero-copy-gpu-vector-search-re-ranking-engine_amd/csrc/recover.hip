@@ -218,6 +218,18 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
         lds_fill = 0u;
         lds_tau = 0ull;
     }
+    // A query of zeros (no L2, no lexical scores): 0 is the best score there is, so the sweep ends once
+    // `width` rows have it.
+    bool zero = false;
+    if constexpr (kKind != ZCGVS_DTYPE_BINARY) {
+        if (scan.metric != ZCGVS_METRIC_L2 && scan.lexical == nullptr) {
+            int any = 0;
+            for (int i = t; i < words; i += kRecoverThreads) {  // (this thread's own words)
+                any |= kKind == kKindI8I8 ? lds_query[i] != 0u : !(__uint_as_float(lds_query[i]) == 0.0f);
+            }
+            zero = __syncthreads_or(any) == 0;
+        }
+    }
     float inverse = 0.0f;
     if (scan.lexical != nullptr) {
         const float peak = scan.lexical_max[q];
@@ -375,7 +387,7 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
     // ---- one sweep in index order, kRowsPerPass rows per step ----
     // A step appends at most kRowsPerPass keys, so a list at most cap - check_every * kRowsPerPass
     // long takes check_every steps before the next check.
-    const int check_every = max(1, (static_cast<int>(lds.cap) - width) / kRowsPerPass);
+    const int check_every = zero ? 1 : max(1, (static_cast<int>(lds.cap) - width) / kRowsPerPass);
     const std::uint32_t check_limit = lds.cap - static_cast<std::uint32_t>(check_every * kRowsPerPass);
     std::uint64_t tau = 0ull;  // lds_tau, read after each barrier that follows a change
     int step = 0;
@@ -394,9 +406,12 @@ __device__ __forceinline__ void recomputeQuery(const ScanArgs& scan, const Recov
             __syncthreads();
             const std::uint32_t count = lds_fill;
             __syncthreads();  // (before a faster wavefront's next step appends: count is uniform)
-            if (count > check_limit) {
+            if (count > check_limit || (zero && count > static_cast<std::uint32_t>(width))) {
                 cutList(count);
                 tau = lds_tau;
+                if (zero && tau >= makeKey(0.0f, 0xFFFFFFFFu)) {
+                    break;  // uniform
+                }
             }
         }
     }

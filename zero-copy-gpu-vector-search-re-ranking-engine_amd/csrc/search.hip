@@ -1171,7 +1171,7 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
             if (sketch_first) {
                 status = launchFilterScan(scan, filter, plan.filter_sketch, emit, plan.workgroups, s);
                 if (status == ZCGVS_OK) {
-                    status = launchFilterThreshold(emit.sketch, plan.sketch_slots, batch, plan.width, tau,
+                    status = launchFilterThreshold(filter, emit.sketch, plan.sketch_slots, batch, tau,
                                                    at<std::uint64_t>(ws, plan.tau_safe), flag_count, s);
                 }
                 if (status != ZCGVS_OK) {
@@ -1200,8 +1200,7 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
                 // the speculative threshold and the guaranteed one; clears the flagged list
                 std::uint64_t* tau_safe = at<std::uint64_t>(ws, plan.tau_safe);
                 status = plan.use_filter
-                             ? launchFilterThreshold(emit.sketch, plan.sketch_slots, batch, plan.width, tau, tau_safe,
-                                                     flag_count, s)
+                             ? launchFilterThreshold(filter, emit.sketch, plan.sketch_slots, batch, tau, tau_safe, flag_count, s)
                              : launchSketchThreshold(emit.sketch, plan.sketch_slots, batch, plan.sketch_rank, plan.width,
                                                      tau, tau_safe, flag_count, s);
                 if (status != ZCGVS_OK) {
