@@ -1,8 +1,9 @@
 """The filter scan: approximate float16 scores with an error bound decide which pairs are scored
 exactly, so every result must be the oracle's (within float32 rounding) whatever the approximation
-does. Sizes at its edges: rows of one chunk to 4 KB, whole and partial 256-byte pieces, 128-byte
-halves and 16-byte chunks, one and several rounds of pieces; one query to several launches; row
-counts that end in a partial block; masks that let through everything, some, and fewer rows than k."""
+does, and the exact fallback's bit for bit. Sizes at its edges: rows of one chunk to 4 KB, whole and
+partial 256-byte pieces, 128-byte halves and 16-byte chunks, one and several rounds of pieces; one query
+to several launches; row counts that end in a partial block; masks that let through everything, some,
+and fewer rows than k."""
 
 import time
 
@@ -79,6 +80,9 @@ def test_filter_scan(gpu, kind, n, dim, batch, k, metric, share):
     assert not flags.any()
     assert_topk_equivalent(idx, val, oracle.scores_f32(decoded, queries, metric, mask), k,
                            float_tolerance(queries, decoded, metric))
+    # and bit for bit what the exact fallback, which sums as the VALU and scalar scans do, computes
+    exact = run(capi, stored, dtype, queries, k, metric, mask, capi.SEARCH_FORCE_EXACT_PASS)
+    assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
 
 
 @pytest.mark.parametrize("kind,dim,scale", [("f32", 768, 1e6), ("f32", 768, 1e-6), ("f32", 1024, 3e18), ("f16", 768, 1e-5),
@@ -243,7 +247,7 @@ def _desc(capi, kind, rows, queries, k, metric, mask=None):
     ("f16", 60_011, 301, 5, 100, 2, True),
     ("f32", 100_003, 333, 6, 30, 1, False),
     ("i8", 100_003, 384, 17, 10, 0, False),
-    ("i8", 50_021, 1024, 5, 200, 1, True),
+    ("i8", 50_021, 1024, 5, 200, 2, True),
     ("i8row", 100_003, 640, 20, 40, 0, False),
     ("f16", 60_011, 768, 20, 512, 0, False),  # the widest selections: segments of 1024 keys
 ])
@@ -424,3 +428,6 @@ def test_hybrid(gpu, kind, n, dim, batch, k, metric, weight):
     # the dense part's rounding, and that of the fusion's three operations on values of at most 1
     tol = np.float32(weight) * float_tolerance(queries, decoded, metric) + 3e-7
     assert_topk_equivalent(idx, val, fused, k, tol)
+    desc.flags = capi.SEARCH_FORCE_EXACT_PASS
+    exact = capi.search(desc)
+    assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))

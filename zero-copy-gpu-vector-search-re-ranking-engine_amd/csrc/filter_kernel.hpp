@@ -112,6 +112,13 @@ __device__ __forceinline__ v4u keepFrom(v4u v, int skip) {
     return v;
 }
 
+// A term of an L2 distance: the decoded value is rounded before the difference is, as in the VALU scan
+// (a compiler left to itself subtracts the int8 product unrounded here).
+__device__ __forceinline__ float l2Difference(float q, float x) {
+#pragma clang fp contract(off)
+    return q - x;
+}
+
 // The exact score of `row` (allowed) for query q, by the L lanes of a group, as the VALU scan
 // computes it: lane g of the group takes chunks g, g + L, ... in turn, groupSum adds the lanes.
 template <int kKind, int L>
@@ -163,7 +170,7 @@ __device__ __forceinline__ float exactScoreLanes(const ScanArgs& scan, std::uint
                 Traits::decode(make_uint4(raw[t][0], raw[t][1], raw[t][2], raw[t][3]), scan.scale, v);
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
-                    const float d = l2 ? qe[t][e] - v[e] : v[e];
+                    const float d = l2 ? l2Difference(qe[t][e], v[e]) : v[e];
                     acc = fmaf(l2 ? d : qe[t][e], d, acc);
                 }
             }
@@ -185,7 +192,7 @@ __device__ __forceinline__ float exactScoreStrided(const ScanArgs& scan, std::ui
 #pragma unroll 4
     for (int j = lane; j < dim; j += kWave) {
         const float x = loadScalar<kKind>(values, j, scan.scale);
-        const float d = l2 ? query[j] - x : x;
+        const float d = l2 ? l2Difference(query[j], x) : x;
         acc = fmaf(l2 ? d : query[j], d, acc);
     }
     const float total = groupSum<kWave>(acc);
