@@ -277,6 +277,44 @@ def test_crowded_thresholds(gpu, kind, n, dim, batch, k, metric, masked, equal):
         assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
 
 
+# Few rows, in the corpus or let through by a mask: a wavefront's tile is then 1, 2, 4, ... rows, so that all
+# have some, and a block of the sketch has 16, 8, 4, ... slots.
+@pytest.mark.parametrize("kind,dim,batch,metric", [("f16", 768, 9, 0), ("f16", 64, 100, 2), ("f32", 640, 16, 1), ("i8", 301, 40, 0),
+                                                   ("i8row", 640, 30, 0)])
+@pytest.mark.parametrize("n,allowed", [(1_100, None), (2_049, None), (4_100, None), (33_001, None), (40_009, 3), (40_009, 70),
+                                       (40_009, 1_500), (40_009, 2_500), (100_003, 17_000)])
+def test_few_rows(gpu, kind, dim, batch, metric, n, allowed):
+    capi = gpu
+    k = 32
+    rows, queries = normalized(n, dim, 86), normalized(batch, dim, 87)
+    mask = None
+    if allowed is not None:
+        mask = np.zeros(n, np.uint8)
+        mask[np.random.default_rng(88).choice(n, allowed, replace=False)] = 1
+    desc, ref = _desc(capi, kind, rows, queries, k, metric, mask)
+    idx, val, flags = capi.search(desc)
+    assert not flags.any()
+    if kind == "i8row":
+        assert_topk_equivalent(idx, val, ref, k)
+        return
+    assert_topk_equivalent(idx, val, ref, k, float_tolerance(queries, encode(capi, rows, kind)[2], metric))
+    desc.flags = capi.SEARCH_FORCE_EXACT_PASS
+    exact = capi.search(desc)
+    assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind,dim,batch,k,n,share", [("f16", 100, 16, 170, 60_000, 0.03), ("i8", 922, 5, 170, 40_000, 0.05)])
+def test_masks_that_let_few_rows_through_cost_no_more(gpu, kind, dim, batch, k, n, share):
+    # fewer rows than 16 per selected key, of rows that take a wavefront each to score
+    capi = gpu
+    mask = (np.random.default_rng(89).random(n) < share).astype(np.uint8)
+    desc, _ = _desc(capi, kind, normalized(n, dim, 90), normalized(batch, dim, 91), k, 0, mask)
+    assert len(capi.search_phase_rows(desc)) == 2  # the filter scan
+    filtered = _seconds(capi, desc)
+    desc.flags = capi.SEARCH_MATERIALIZE
+    assert filtered < 3 * _seconds(capi, desc)
+
+
 # A query of zeros scores every row 0 and takes the lowest ones: a batch padded with such queries costs
 # about what the others do.
 @pytest.mark.parametrize("kind,dim,batch,zeros,metric,share", [

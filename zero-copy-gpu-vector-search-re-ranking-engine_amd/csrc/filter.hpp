@@ -50,7 +50,8 @@ struct FilterQuery {
     float norm2;  // sum q_j^2
     float usable; // 0: not finite or out of range, every pair is scored exactly
     // 1: all zero, under a metric by which every finite row then scores 0, so that the row numbers decide
-    // (a batch padded to its size, say). The scan takes no pair of such a query; the last merge, which
+    // (a batch padded to its size, say). The scan takes no pair of such a query (unless a mask lets few
+    // rows through); the last merge, which
     // finds too few keys, sweeps the rows from the first on until enough score 0 (recover.hip). In the
     // scan every row would reach its threshold: 1M x 384 float32, 64 queries, 32 of them zero 14.0 ms,
     // now 0.34; with one 25.9, now 0.35.
@@ -69,6 +70,7 @@ struct FilterArgs {
     int groups = 0;                    // query groups prepared (launches * groups per launch)
     int groups_per_launch = 0;
     int width = 0;                     // keys selected per query
+    int tile_log2 = 0;                 // log2 of FilterShape::tile_rows
     // Launches of 32 to 128 queries over float32 rows of 256 or 384 components take NaN for an
     // infinite score, as the split scan (fused_mfma_split.hip) does.
     int infinite_as_nan = 0;
@@ -82,6 +84,16 @@ struct FilterShape {
     int groups_per_launch = 0;
     int tile_rows = 0;  // rows of a threshold phase's work item
 };
+// log2 of the rows of a wavefront's tile: `most` (the kernel's blocks), or with fewer rows than those
+// fill of `waves` wavefronts the smallest number that covers them, so that the pairs to score exactly are
+// shared by all.
+__host__ __device__ inline int filterTileLog2(long long rows, int most, int waves) {
+    int log2 = 0;
+    while (1 << log2 < most && static_cast<long long>(waves) << log2 < rows) {
+        ++log2;
+    }
+    return log2;
+}
 FilterShape filterShape(const ScanArgs& scan, int width);
 inline std::size_t filterOperandBytes(const FilterShape& shape) {
     return static_cast<std::size_t>(shape.groups) * shape.steps * 1024;
@@ -98,8 +110,8 @@ inline long long filterMaskedRows(long long rows, int width) { return rows < 2LL
 // The query operands, the row unit and, with a mask, the row list.
 int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_t stream);
 // After a sketch phase: tau[q] (and tau_safe[q]), a key below the width-th best of query q's rows.
-int launchFilterThreshold(const FilterArgs& args, const float* sketch, int slots, int batch, std::uint64_t* tau,
-                          std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream);
+int launchFilterThreshold(const FilterArgs& args, long long rows, const float* sketch, int slots, int batch,
+                          std::uint64_t* tau, std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream);
 // A sketch phase (emit.sketch: the best certain lower bound of every slot's rows; items of 16 rows)
 // or a threshold phase (items of tile_rows rows; over every listed row when there is a row list).
 int launchFilterScan(const ScanArgs& scan, const FilterArgs& args, const PhaseArgs& phase, const EmitArgs& emit,

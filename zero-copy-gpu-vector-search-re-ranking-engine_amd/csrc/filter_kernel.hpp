@@ -291,7 +291,10 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
 
     // ---- tiles ----
     const long long row_blocks = (rows + kFilterBlockRows - 1) / kFilterBlockRows;
-    long long tiles = list != nullptr ? (row_blocks + kBlocks - 1) / kBlocks : phase.items;
+    // (a short row list: smaller tiles, as filterTileLog2 makes them where the host knows the rows)
+    const int tile_log2 = list != nullptr ? filterTileLog2(rows, kBlocks * kFilterBlockRows, gridDim.x * kFilterWaves)
+                                          : args.tile_log2;
+    long long tiles = list != nullptr ? (rows + (1LL << tile_log2) - 1) >> tile_log2 : phase.items;
     long long stride = 1;  // sketch: one block of every `stride`
     if (sketch) {
         // (with a row list the host knows only an upper bound of the rows: the stride that visits
@@ -300,7 +303,8 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         tiles = (row_blocks + stride - 1) / stride;
     }
     const long long waves = static_cast<long long>(gridDim.x) * kFilterWaves;
-    long long tile = static_cast<long long>(wave) * gridDim.x + blockIdx.x;
+    const long long first_tile = static_cast<long long>(wave) * gridDim.x + blockIdx.x;
+    long long tile = first_tile;
 
     // Place of threshold tile t among the corpus's (the list's) tiles.
     auto tileAt = [&](long long t) __attribute__((always_inline)) -> long long {
@@ -308,9 +312,9 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     };
     // Entry (row number, kMaskedRow with it for a masked one) of place `local` of tile t.
     auto entryOf = [&](long long t, int local) __attribute__((always_inline)) -> std::uint32_t {
-        const long long at = (sketch ? t * stride : tileAt(t) * kBlocks) * kFilterBlockRows + local;
+        const long long at = (sketch ? t * stride * kFilterBlockRows : tileAt(t) << tile_log2) + local;
         std::uint32_t entry = kNoRow;
-        if (at < rows && !(sketch && local >= kFilterBlockRows)) {
+        if (at < rows && local < (sketch ? kFilterBlockRows : 1 << tile_log2)) {
             entry = list != nullptr ? list[at] : static_cast<std::uint32_t>(at);
         }
         return entry;
@@ -931,9 +935,8 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         }
         // The exact scores of the parked pairs and, of a crowded tile, of every pair (its rows from the list
         // or the tile's place). A key that finds its segment full waits for a cut.
-        constexpr int kTileRows = kBlocks * kFilterBlockRows;
-        const std::uint32_t total = parked + (crowded ? static_cast<std::uint32_t>(kTileRows * q_count) : 0u);
-        const long long tile_row = tileAt(tile) * kTileRows;  // (not used past the last tile)
+        const std::uint32_t total = parked + (crowded ? static_cast<std::uint32_t>(q_count) << tile_log2 : 0u);
+        const long long tile_row = tileAt(tile) << tile_log2;  // (not used past the last tile)
         tile += crowded ? waves : 0;
         const bool done = tile >= tiles;
         std::uint32_t first = 0u;
@@ -951,11 +954,11 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 waits = e < total;
                 if (crowded && e >= parked) {
                     const std::uint32_t at = min(e, total - 1u) - parked;
-                    const long long place = tile_row + at % kTileRows;
+                    const long long place = tile_row + (at & ((1u << tile_log2) - 1u));
                     waits = waits && place < rows;
                     listed = static_cast<std::uint32_t>(min(place, rows - 1));
                     listed = list != nullptr ? list[listed] : listed;
-                    q = static_cast<int>(at / kTileRows);
+                    q = static_cast<int>(at >> tile_log2);
                 }
                 key = keyOfPair(listed, q);
                 waits = waits && lane % lanes_per_row == 0;
@@ -991,17 +994,27 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         issueTile(row);
     }
     if (sketch) {
-        // one slot per wavefront: the best over its 16 row lanes
+        // One slot per wavefront, the best over its 16 row lanes; with fewer blocks than half the slots, as
+        // many slots per block (2, 4, 8 or 16, its rows dealt out to them) as there are.
+        int split = 0;
+        while (split < 4 && tiles << (split + 1) <= waves) {
+            ++split;
+        }
+        const int lanes = kFilterBlockRows >> split;
+        const bool has_block = first_tile < tiles;
+        const std::size_t slot = has_block ? (static_cast<std::size_t>(first_tile) << split) + r16 / lanes : first_tile;
+        const bool owns = has_block ? r16 % lanes == 0 : r16 == 0 && first_tile >= tiles << split;
 #pragma unroll
         for (int i = 0; i < kGroups * 4; ++i) {
             float v = best[i];
 #pragma unroll
-            for (int x = 1; x < 16; x <<= 1) {
-                v = fmaxf(v, waveXor(v, x));
+            for (int x = 1; x < kFilterBlockRows; x <<= 1) {
+                const float other = waveXor(v, x);
+                v = x < lanes ? fmaxf(v, other) : v;
             }
             const int q = kFilterGroup * (i / 4) + 4 * h + (i & 3);
-            if (r16 == 0 && q < q_count) {
-                emit.sketch[static_cast<std::size_t>(blockIdx.x * kFilterWaves + wave) * scan.batch + q_offset + q] = v;
+            if (owns && q < q_count) {
+                emit.sketch[slot * scan.batch + q_offset + q] = v;
             }
         }
     } else {

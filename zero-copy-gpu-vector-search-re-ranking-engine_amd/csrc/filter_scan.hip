@@ -180,7 +180,7 @@ constexpr int kThresholdThreads = 512;
 constexpr int kThresholdBins = 2048;
 constexpr int kThresholdSlots = kMaxSketchSlots / kThresholdThreads;
 
-__global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(const FilterQuery* __restrict__ queries,
+__global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(FilterArgs args, long long rows,
                                                                            const float* __restrict__ sketch, int slots,
                                                                            int batch, int width,
                                                                            std::uint64_t* __restrict__ tau,
@@ -210,7 +210,10 @@ __global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(const
     if (q == 0 && t == 0) {
         *flag_count = 0u;
     }
-    if (queries[q].zero != 0.0f) {  // (uniform)
+    // (with an allow-mask, only if the sweep finds its rows among the first 8192 or so, about 70 us: of a
+    // few rows let through, the scan scores every pair sooner)
+    if (args.queries[q].zero != 0.0f &&
+        (args.list_count == nullptr || rows * width <= 8192LL * static_cast<long long>(*args.list_count))) {  // (uniform)
         if (t == 0) {
             tau[q] = kFilterNoKey;
             tau_safe[q] = kFilterNoKey;
@@ -418,8 +421,10 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
         }
     }
     shape.tile_rows =
-        kFilterBlockRows * filterBlocks(filterSlots(static_cast<int>((bytes + 255) / 256)), shape.groups_per_launch,
-                                        scan.lexical != nullptr);
+        1 << filterTileLog2(scan.doc_count,
+                            kFilterBlockRows * filterBlocks(filterSlots(static_cast<int>((bytes + 255) / 256)),
+                                                            shape.groups_per_launch, scan.lexical != nullptr),
+                            deviceComputeUnits() * kFilterWaves);
     launches = (groups + shape.groups_per_launch - 1) / shape.groups_per_launch;
     shape.groups = launches * shape.groups_per_launch;
     shape.supported = true;
@@ -444,13 +449,13 @@ int launchFilterPrepare(const ScanArgs& scan, const FilterArgs& args, hipStream_
     return ZCGVS_OK;
 }
 
-int launchFilterThreshold(const FilterArgs& args, const float* sketch, int slots, int batch, std::uint64_t* tau,
-                          std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream) {
+int launchFilterThreshold(const FilterArgs& args, long long rows, const float* sketch, int slots, int batch,
+                          std::uint64_t* tau, std::uint64_t* tau_safe, std::uint32_t* flag_count, hipStream_t stream) {
     if (slots < 1 || slots > kMaxSketchSlots || args.width < 1) {
         return setError(ZCGVS_ERR_RUNTIME, "zcgvs filter: sketch shape out of range");
     }
-    filterThresholdKernel<<<batch, kThresholdThreads, 0, stream>>>(args.queries, sketch, slots, batch, args.width, tau,
-                                                                   tau_safe, flag_count);
+    filterThresholdKernel<<<batch, kThresholdThreads, 0, stream>>>(args, rows, sketch, slots, batch, args.width, tau, tau_safe,
+                                                                   flag_count);
     ZCGVS_LAUNCH_CHECK("filter threshold");
     return ZCGVS_OK;
 }

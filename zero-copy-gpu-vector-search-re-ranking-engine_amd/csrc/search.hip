@@ -289,6 +289,7 @@ FilterArgs filterArgsOf(const zcgvs_search_desc& d, const Plan& plan, std::uint8
     args.groups = plan.filter.groups;
     args.groups_per_launch = plan.filter.groups_per_launch;
     args.width = plan.width;
+    args.tile_log2 = ceilLog2(plan.filter.tile_rows);
     args.infinite_as_nan = d.corpus.dtype == ZCGVS_DTYPE_F32 && d.mask == nullptr && d.metric != ZCGVS_METRIC_L2 &&
                                    (d.corpus.dim == 256 || d.corpus.dim == 384)
                                ? 1
@@ -1171,7 +1172,7 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
             if (sketch_first) {
                 status = launchFilterScan(scan, filter, plan.filter_sketch, emit, plan.workgroups, s);
                 if (status == ZCGVS_OK) {
-                    status = launchFilterThreshold(filter, emit.sketch, plan.sketch_slots, batch, tau,
+                    status = launchFilterThreshold(filter, d.corpus.doc_count, emit.sketch, plan.sketch_slots, batch, tau,
                                                    at<std::uint64_t>(ws, plan.tau_safe), flag_count, s);
                 }
                 if (status != ZCGVS_OK) {
@@ -1200,7 +1201,7 @@ int searchTopk(const zcgvs_search_desc* desc, void* d_workspace, std::size_t wor
                 // the speculative threshold and the guaranteed one; clears the flagged list
                 std::uint64_t* tau_safe = at<std::uint64_t>(ws, plan.tau_safe);
                 status = plan.use_filter
-                             ? launchFilterThreshold(filter, emit.sketch, plan.sketch_slots, batch, tau, tau_safe, flag_count, s)
+                             ? launchFilterThreshold(filter, d.corpus.doc_count, emit.sketch, plan.sketch_slots, batch, tau, tau_safe, flag_count, s)
                              : launchSketchThreshold(emit.sketch, plan.sketch_slots, batch, plan.sketch_rank, plan.width,
                                                      tau, tau_safe, flag_count, s);
                 if (status != ZCGVS_OK) {
