@@ -270,6 +270,8 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     __shared__ __attribute__((aligned(16))) float lds_inverse[kLex ? kQueries : 4];  // 1 / largest lexical score
     __shared__ std::uint64_t lds_tau[kQueries];
     __shared__ std::uint32_t lds_count[kQueries];
+    __shared__ std::uint64_t lds_lowest[kQueries];  // the lowest of the first `width` keys appended
+    __shared__ std::uint32_t lds_placed[kQueries];  // how many of those it covers
     __shared__ std::uint32_t lds_asked[2];  // a wavefront asks for a cut of the segments (in turns)
     __shared__ __attribute__((aligned(16))) std::uint8_t lds_stage[kFilterWaves][kFilterBlockRows * kPieceBytes / 2];
     __shared__ uint2 lds_park[kFilterWaves][kParkSlots];
@@ -458,6 +460,8 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     };
     for (int i = tid; i < kQueries; i += kFilterThreads) {
         lds_count[i] = 0u;
+        lds_lowest[i] = ~0ull;
+        lds_placed[i] = 0u;
         setQuery(i, i < q_count && !sketch ? emit.tau[q_offset + i] : kFilterNoKey);
     }
     if (tid < 2) {
@@ -665,18 +669,19 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         if (ask) {
             __hip_atomic_store(&lds_asked[turn & 1u], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's keys have left the compute unit
         __syncthreads();
         if (__builtin_amdgcn_readfirstlane(askedForCut()) == 0u) {
-            return false;
+            return false;  // (without a wait for the rows read past the last tile: 1 us of every launch)
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's keys have left the compute unit
+        __syncthreads();
 #pragma unroll 1
         for (int q = wave; q < q_count; q += kFilterWaves) {
             if (__builtin_amdgcn_readfirstlane(lds_count[q]) >= capacity) {
                 cutSegment(q);
             }
         }
-        // (nobody reads the other turn's word between these two barriers)
+        // (nobody reads the other turn's word between the barriers before and after)
         if (tid == 0) {
             __hip_atomic_store(&lds_asked[(turn + 1u) & 1u], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
@@ -933,6 +938,9 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 break;
             }
         }
+        if (sketch) {
+            break;  // (no keys)
+        }
         // The exact scores of the parked pairs and, of a crowded tile, of every pair (its rows from the list
         // or the tile's place). A key that finds its segment full waits for a cut.
         const std::uint32_t total = parked + (crowded ? static_cast<std::uint32_t>(q_count) << tile_log2 : 0u);
@@ -970,6 +978,14 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
                 if (slot < capacity) {
                     segmentOf(q)[slot] = key;
                 }
+                // The workgroup's first `width` keys of a query are a threshold as a cut's are: the last of
+                // them to be covered raises it, which spares the merge keys.
+                if (slot < width) {
+                    atomicMin(&lds_lowest[q], key);
+                    if (atomicAdd(&lds_placed[q], 1u) + 1u == width) {
+                        lds_tau[q] = max(lds_tau[q], lds_lowest[q]);
+                    }
+                }
                 waits = slot >= capacity && cuts;
             }
             const bool ask = __any(waits);
@@ -1000,22 +1016,29 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
         while (split < 4 && tiles << (split + 1) <= waves) {
             ++split;
         }
-        const int lanes = kFilterBlockRows >> split;
-        const bool has_block = first_tile < tiles;
-        const std::size_t slot = has_block ? (static_cast<std::size_t>(first_tile) << split) + r16 / lanes : first_tile;
-        const bool owns = has_block ? r16 % lanes == 0 : r16 == 0 && first_tile >= tiles << split;
+        // (the usual single slot first: its shuffles, of all queries side by side, end every sketch)
+        auto storeBest = [&](int lanes, std::size_t slot, bool owns) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < kGroups * 4; ++i) {
-            float v = best[i];
+            for (int i = 0; i < kGroups * 4; ++i) {
+                float v = best[i];
 #pragma unroll
-            for (int x = 1; x < kFilterBlockRows; x <<= 1) {
-                const float other = waveXor(v, x);
-                v = x < lanes ? fmaxf(v, other) : v;
+                for (int x = 1; x < kFilterBlockRows; x <<= 1) {
+                    const float other = waveXor(v, x);
+                    v = x < lanes ? fmaxf(v, other) : v;
+                }
+                const int q = kFilterGroup * (i / 4) + 4 * h + (i & 3);
+                if (owns && q < q_count) {
+                    emit.sketch[slot * scan.batch + q_offset + q] = v;
+                }
             }
-            const int q = kFilterGroup * (i / 4) + 4 * h + (i & 3);
-            if (owns && q < q_count) {
-                emit.sketch[slot * scan.batch + q_offset + q] = v;
-            }
+        };
+        if (split == 0) {
+            storeBest(kFilterBlockRows, static_cast<std::size_t>(first_tile), r16 == 0);
+        } else {
+            const int lanes = kFilterBlockRows >> split;
+            const bool has_block = first_tile < tiles;
+            storeBest(lanes, static_cast<std::size_t>(has_block ? (first_tile << split) + r16 / lanes : first_tile),
+                      has_block ? r16 % lanes == 0 : r16 == 0 && first_tile >= tiles << split);
         }
     } else {
         for (int i = tid; i < q_count; i += kFilterThreads) {

@@ -192,6 +192,13 @@ __global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(Filte
     __shared__ std::uint32_t lds_low[kWaves], lds_high[kWaves], lds_sums[kWaves];
     const int q = blockIdx.x;
     const int t = threadIdx.x;
+    // (with an allow-mask, only if the merge's sweep finds its rows among the first 8192 or so, about 70 us: of
+    // a few rows let through, the scan scores every pair sooner)
+    const float zero = args.queries[q].zero;
+    auto leftOut = [&]() {
+        return zero != 0.0f &&
+               (args.list_count == nullptr || rows * width <= 8192LL * static_cast<long long>(*args.list_count));
+    };
     std::uint32_t v[kThresholdSlots];  // ordered bits; 0: no score
     std::uint32_t low = 0xFFFFFFFFu;
     std::uint32_t high = 0u;
@@ -209,16 +216,6 @@ __global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(Filte
     }
     if (q == 0 && t == 0) {
         *flag_count = 0u;
-    }
-    // (with an allow-mask, only if the sweep finds its rows among the first 8192 or so, about 70 us: of a
-    // few rows let through, the scan scores every pair sooner)
-    if (args.queries[q].zero != 0.0f &&
-        (args.list_count == nullptr || rows * width <= 8192LL * static_cast<long long>(*args.list_count))) {  // (uniform)
-        if (t == 0) {
-            tau[q] = kFilterNoKey;
-            tau_safe[q] = kFilterNoKey;
-        }
-        return;
     }
 #pragma unroll
     for (int m = kWave / 2; m > 0; m >>= 1) {
@@ -261,15 +258,17 @@ __global__ __launch_bounds__(kThresholdThreads) void filterThresholdKernel(Filte
         if (above < need && above + own[b] >= need) {
             const std::uint32_t edge =
                 low + (static_cast<std::uint32_t>(kThresholdBins - 1 - kBinsPerThread * t - b) << shift);
-            tau[q] = static_cast<std::uint64_t>(edge) << 32;
-            tau_safe[q] = tau[q];
+            const std::uint64_t key = leftOut() ? kFilterNoKey : static_cast<std::uint64_t>(edge) << 32;
+            tau[q] = key;
+            tau_safe[q] = key;
         }
         above += own[b];
     }
     if (t == 0 && total < need) {
         // rows 0 to width - 1 alone are width keys at or above this one
-        tau[q] = makeKey(__uint_as_float(0x7FC00000u), need - 1u) - 1ull;
-        tau_safe[q] = tau[q];
+        const std::uint64_t key = leftOut() ? kFilterNoKey : makeKey(__uint_as_float(0x7FC00000u), need - 1u) - 1ull;
+        tau[q] = key;
+        tau_safe[q] = key;
     }
 }
 
