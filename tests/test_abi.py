@@ -215,6 +215,21 @@ def test_phase_rows_cover_the_corpus_once(capi, n, dtype, int8_mode, batch, k):
     assert all(r > 0 for r in rows)
 
 
+@pytest.mark.parametrize("n,dim,dtype,batch,masked,filtered", [
+    (5_000, 922, 0, 1, False, False),    # odd rows: a few thousand take the score matrix
+    (10_000, 301, 2, 5, False, False),
+    (30_000, 301, 1, 16, False, True),
+    (80_000, 100, 1, 1, False, True),
+    (10_000, 301, 0, 128, True, False),  # a mask that lets a few rows through leaves all their pairs
+    (200_000, 301, 0, 128, True, True),
+    (2_000, 384, 2, 9, False, False),    # whole chunks
+    (2_000, 768, 1, 16, False, True),
+])
+def test_small_searches_filter_where_it_pays(capi, n, dim, dtype, batch, masked, filtered):
+    rows = capi.search_phase_rows(_desc(capi, n=n, dim=dim, dtype=dtype, batch=batch, mask=1 << 22 if masked else None))
+    assert (len(rows) == 2 and rows[1] == n) == filtered
+
+
 @pytest.mark.parametrize("n,dim,dtype,batch,masked", [
     (16_000_000, 384, 1, 16, True),  # row lists of 64 and 80 MB
     (20_000_000, 384, 1, 16, True),

@@ -370,12 +370,12 @@ void planFilter(const zcgvs_search_desc& d, Plan& plan, Layout& layout) {
     plan.total = layout.total;
 }
 
-// Whether the filter scan is the fastest plan for a shape it takes. Its five launches cost 31 us
-// (and 0.4 per query group) before any row, so small searches keep the plans they had; the lines lie
+// Whether the filter scan is the fastest plan for a shape it takes. Its five launches (six with a mask)
+// cost 31 us (and 0.4 per query group) before any row, so small searches keep the plans they had; the lines lie
 // where both measured the same (us, that plan against the filter scan).
 bool filterPays(const ScanArgs& scan, const Plan& plan) {
     const long long n = scan.doc_count;
-    // (few rows: the sketch has a slot per 16 of them, and needs more slots than keys)
+    // (fewer rows: a threshold leaves too large a part of them to score exactly)
     if (n < std::max<long long>(kFilterMinRows, 2LL * kFilterBlockRows * plan.width)) {
         return false;
     }
@@ -387,35 +387,25 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
         // 16 queries 187 / 164, 64 queries 251 / 200, 128 queries 299 / 291; 30% allowed, 16 queries
         // 202 / 80, 128 queries 300 / 141, 256 queries 273 / 250; 90% allowed, 256 queries 278 / 555.
         // 5,000 x 384, 64 queries 24 / 38, 20,000 rows 46 / 39.
-        // (A mask that lets a thousand rows through leaves every pair of theirs to score exactly, on
-        // few wavefronts: no large batches of wide selections.)
+        // (A mask that lets fewer rows through than are selected leaves every pair of theirs to score exactly:
+        // no large batches of wide selections. 10,000 x 768, 0.05% allowed, 128 queries 57 / 69.)
         return n >= 8192 && (scan.mask != nullptr ? scan.batch <= 128 && scan.batch * plan.width <= 2048
                                                   : scan.batch <= 32);
     }
-    // Pairs to score exactly, about 2 per key: over the wavefront tiles that share them, more than
-    // about 160 a tile would make the scan score those tiles whole (3,000 x 256 int8, 128 queries, k 90:
-    // 202 / 690), and a round of them (64 / lanes-per-row pairs a wavefront) takes about 1 us.
-    const long long pairs = 2LL * scan.batch * plan.width;
-    // (A mask may let few rows through, and fewer than the sketch needs leave all of them to score
-    // exactly: 20,000 x 300 float16, 5% allowed, 128 queries, k 200 144 / 2431; a sixteenth of the
-    // rows is taken for masked searches.)
-    const long long listed = scan.mask != nullptr ? n / 16 : n;
-    if (pairs * plan.filter.tile_rows > 160 * listed) {
-        return false;
-    }
     const std::size_t row_bytes = rowBytes(scan.dtype, scan.dim);
-    const bool whole_chunks = row_bytes % 16 == 0;
-    const int per_round =
-        whole_chunks ? kWave / std::max(8, lanesPerRow(static_cast<int>(row_bytes / 16), 8, 8)) : 1;
-    const long long waves = std::min<long long>((n + plan.filter.tile_rows - 1) / plan.filter.tile_rows,
-                                                static_cast<long long>(deviceComputeUnits()) * kFilterWaves);
-    const long long rounds = pairs / (waves * per_round);
     const long long tiles = (scan.batch + 7) / 8;  // of the queries the VALU kernels take at a time
-    if (!whole_chunks) {
-        // The materialized pipeline's scalar scan, about 0.2 ns per row, query tile and 64 components:
-        // 20,000 x 100 int8, 2 queries 26 / 33; 5,000 x 300 float16, 16 queries 31 / 31; 3,000 x 300,
-        // 128 queries 71 / 63, with k 90 73 / 171; 100,000 x 100, 1 query 47 / 35.
-        return n * tiles * ((scan.dim + 63) / 64) >= 50'000 + 5'000 * rounds;
+    if (row_bytes % 16 != 0) {
+        // The materialized pipeline's scalar scan takes about 0.22 ns per row, query tile and 64 components
+        // and its other launches 16 us, the filter scan 35 us (922 components 45) and the exact scores,
+        // against 2304 shapes: float16 x 100, 1 query, 40,000 rows 29 / 36, 80,000 39 / 37, 16 queries, 10,000
+        // rows 32 / 38, 40,000 56 / 40; float32 x 922, 1 query, 20,000 rows 49 / 59, 40,000 85 / 71; int8 x
+        // 301, 100 queries, 5,000 rows 77 / 56. With a mask the list takes 6 us, and where the mask lets through
+        // fewer rows than are selected a wavefront scores one row against every query, about 4 us each
+        // (3,000 x 922 int8, 5% allowed, 100 queries 73 / 129; 10,000 x 301 float32, 0.4%, 128 queries 86 / 214).
+        const long long pieces = (scan.dim + 63) / 64;
+        const long long cost = n * tiles * pieces;
+        return scan.mask != nullptr ? cost >= 80'000 + (24'000 + 1'200LL * scan.batch) * pieces
+                                    : cost >= 120'000 + 16'000 * pieces + 5LL * scan.batch * plan.width;
     }
     if (plan.use_mfma_float) {
         // Up to 8191 rows that scan is one dense phase (5,000 x 384 float32, 64 queries 26 against 42;
@@ -423,16 +413,22 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
         // float16, 16 queries 155 / 160, 64 queries 169 / 176; float32, 16 queries 278 / 282); float32
         // batches, which that scan splits into six products, do not (64 queries 381 / 299, 128
         // queries 575 / 329).
-        // (8,200 x 384, 128 queries, k 200: 54 / 137 with that many pairs to score exactly)
         // Two phases and their merges cost 22 us more, which the gain of about 0.08 us per 1000 rows
         // covers from some 300,000 rows on (one search of fewer measured 56 / 72).
-        return n >= 400'000 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32 && rounds <= n / 8192;
+        // (about two pairs per key are scored exactly, 4 or 8 a round of each wavefront, which takes about 1 us)
+        const long long round = static_cast<long long>(deviceComputeUnits()) * kFilterWaves * kWave /
+                                std::max(8, lanesPerRow(static_cast<int>(row_bytes / 16), 8, 8));
+        return n >= 400'000 && scan.dtype == ZCGVS_DTYPE_F32 && scan.batch >= 32 &&
+               2LL * scan.batch * plan.width / round <= n / 8192;
     }
-    // The same line for the VALU scan's plan, or where its dense phase alone, about 0.033 us per query
-    // tile and component (per-vector int8 0.02), takes longer: float16 2,000 x 768, 5 queries 37 / 34,
-    // 16 queries 82 / 38; int8 2,000 x 384, 8 queries 30 / 35; per-vector 3,000 x 320, 16 queries 31 / 33.
-    const long long components = plan.per_vector ? scan.dim * 3LL / 5 : scan.dim;
-    return n >= 8192 || tiles * components >= 640 + 30 * rounds;
+    // Up to 8191 rows the VALU scan is one dense phase, whose time grows with the queries and components:
+    // 2,000 to 4,000 rows of float16 x 768, 5 queries 37 / 38, 9 queries 55 / 39; float32 x 96, 16 queries 28 /
+    // 36, 40 queries 51 / 39; int8 x 384, 9 queries 32 / 38, 16 queries 45 / 38; int8 x 1024, 5 queries 37 / 42;
+    // per-vector x 320, 16 queries 30 / 36, 40 queries 51 / 42. Beyond, only the least work is level: 9,000
+    // rows of int8 x 64, 5 queries 34 / 36, 50,000 rows 40 / 37; float16 x 64, 16 queries 50 / 36.
+    const bool floats = scan.dtype == ZCGVS_DTYPE_F32 || scan.dtype == ZCGVS_DTYPE_F16;
+    const long long work = scan.batch * (plan.per_vector ? scan.dim * 3LL / 5 : scan.dim);
+    return n >= (work >= 512 ? 8192 : 32768) || work + 300 * tiles >= (floats ? 3900 : 5600);
 }
 
 // The plan of a search. One whose workspace has a fixed size (`limit` bytes) gives up the filter scan
