@@ -388,9 +388,11 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
         // 202 / 80, 128 queries 300 / 141, 256 queries 273 / 250; 90% allowed, 256 queries 278 / 555.
         // 5,000 x 384, 64 queries 24 / 38, 20,000 rows 46 / 39.
         // (A mask that lets fewer rows through than are selected leaves every pair of theirs to score exactly:
-        // no large batches of wide selections. 10,000 x 768, 0.05% allowed, 128 queries 57 / 69.)
-        return n >= 8192 && (scan.mask != nullptr ? scan.batch <= 128 && scan.batch * plan.width <= 2048
-                                                  : scan.batch <= 32);
+        // no large batches of wide selections. 10,000 x 768, 0.05% allowed, 128 queries 57 / 69; 20% allowed, 100
+        // queries 55 / 56, 50,000 rows 70 / 57.)
+        return scan.mask != nullptr ? n >= (scan.batch > 64 ? 32768 : 8192) && scan.batch <= 128 &&
+                                          scan.batch * plan.width <= 2048
+                                    : n >= 8192 && scan.batch <= 32;
     }
     const std::size_t row_bytes = rowBytes(scan.dtype, scan.dim);
     const long long tiles = (scan.batch + 7) / 8;  // of the queries the VALU kernels take at a time
