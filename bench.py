@@ -235,16 +235,28 @@ def measured_traffic(workload, kernel):
     return entry["traffic_bytes_per_launch"]
 
 
+def filter_kernel_name(kind, row_bytes, batch):
+    """The filter scan's kernel (csrc/filter_kernel.hpp) for one launch of up to 128 queries, no lexical
+    scores: scan kind, 256-byte pieces of a row in flight, 16-row blocks of a tile, groups of 16 queries."""
+    pieces = -(-row_bytes // 256)
+    slots = pieces if pieces <= 4 else 3 if pieces in (5, 6, 9) else 4
+    groups = next(g for g in (1, 2, 4, 8) if 16 * g >= batch)
+    blocks = {1: 4, 2: 2}.get(slots, 1) if groups <= 2 else 2 if slots == 1 else 1
+    return f"filterScanKernel<{kind}, {slots}, {blocks}, {groups}, false>"
+
+
 def scan_kernel_name(w):
     if w["kind"] == "i8i8" and w["batch"] >= 8:
         return f"mfmaScanKernel<{w['dim'] // 32}, 0>"
+    if w["kind"] == "f32" and 32 <= w["batch"] <= 128 and w["dim"] in (128, 256, 384, 512) and w["n"] >= 400_000:
+        return filter_kernel_name(0, 4 * w["dim"], w["batch"])
     if w["kind"] == "f32" and w["batch"] >= 32 and w["dim"] in (256, 384):
         return f"mfmaSplitScanKernel<{w['dim']}, false>"
     if w["kind"] in ("f32", "f16", "hybrid") and w["batch"] >= 4 and w["dim"] in (128, 256, 384, 512):
         kind = 0 if w["kind"] == "f32" else 1
         lexical = "true" if w["kind"] == "hybrid" else "false"
         return f"mfmaFloatScanKernel<{kind}, {w['dim']}, false, {lexical}>"
-    if w["kind"] == "binary" and w["batch"] >= 4 and w["dim"] in (512, 1024):
+    if w["kind"] == "binary" and w["batch"] >= 4 and w["dim"] in (256, 384, 512, 768, 1024):
         # one set of up to 32 queries: the streaming kernel (mode 0: threshold scan); more: the
         # shared-tile kernel
         if w["batch"] <= 32:
@@ -501,8 +513,9 @@ def scan_figures(w, m, keep):
     used = len(m["phase_rows"])
     # Dominant kernel: the scan launches of the threshold phases (the MFMA paths compile the dense
     # first phase and the sketch phase as separate kernels; the VALU path runs every phase with one
-    # kernel). A sketch plan's last phase is its one full scan.
-    first = 1 if scan_kernel_name(w).startswith("mfma") and used > 1 else 0
+    # kernel). A sketch plan's last phase is its one full scan; a filter scan's first phase holds its
+    # sketch's launches too, so its last one is taken.
+    first = 1 if scan_kernel_name(w).startswith(("mfma", "filter")) and used > 1 else 0
     launches = list(range(first, used))
     mean_ms = statistics.mean(statistics.mean(m["phase_ms"][i][p] for p in launches) for i in range(steps))
     bytes_launch = statistics.mean(m["phase_rows"][p] * row_bytes(w) + query_bytes(w) for p in launches)

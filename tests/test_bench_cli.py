@@ -40,3 +40,18 @@ def test_with_batch_keeps_the_descriptor(capi):
     assert (one.batch, one.k, desc.batch, desc.k) == (1, 100, 64, 10)
     assert one.corpus.data == desc.corpus.data and one.queries == desc.queries
     assert one.metric == capi.DOT and one.flags == capi.SEARCH_SORTED_POSTINGS
+
+
+@pytest.mark.parametrize("workload,name", [
+    ("f32-1m-b64", "filterScanKernel<0, 3, 1, 4, false>"),
+    ("f16-1m-b64", "mfmaFloatScanKernel<1, 384, false, false>"),
+    ("f32-1m-b1", "singlePassScanKernel"),
+    ("int8-10m", "mfmaScanKernel<24, 0>"),
+])
+def test_roofline_names_the_kernel_that_runs(capi, workload, name):
+    w = bench.WORKLOADS[workload]
+    assert bench.scan_kernel_name(w) == name
+    if name.startswith("filter"):  # its plan: every 8th tile, then the rest (a sketch is not a phase there)
+        corpus = capi.store_desc(1 << 20, w["n"], w["dim"], capi.F32)
+        rows = capi.search_phase_rows(capi.search_desc(corpus, 1 << 20, w["batch"], w["k"]))
+        assert len(rows) == 2 and sum(rows) == w["n"] and 7 * rows[0] >= rows[1] > 6 * rows[0]
