@@ -469,3 +469,36 @@ def test_hybrid(gpu, kind, n, dim, batch, k, metric, weight):
     desc.flags = capi.SEARCH_FORCE_EXACT_PASS
     exact = capi.search(desc)
     assert np.array_equal(idx, exact[0]) and np.array_equal(val.view(np.uint32), exact[1].view(np.uint32))
+
+
+# float32 batches of the matrix-core scan's widths: every 8th tile, then the rest with its exact threshold
+def test_two_phases(gpu):
+    capi = gpu
+    n, dim, batch, k = 400_003, 128, 40, 25
+    rows, queries = normalized(n, dim, 95), normalized(batch, dim, 96)
+    desc, ref = _desc(capi, "f32", rows, queries, k, 0)
+    assert sum(capi.search_phase_rows(desc)) == n
+    idx, val, flags = capi.search(desc)
+    assert not flags.any()
+    assert_topk_equivalent(idx, val, ref, k, float_tolerance(queries, rows, 0))
+    for flag in (capi.SEARCH_FORCE_EXACT_PASS, capi.SEARCH_TEST_TINY_SEGMENTS):
+        desc.flags = flag
+        other = capi.search(desc)
+        assert flag == capi.SEARCH_FORCE_EXACT_PASS or other[2].any()
+        assert np.array_equal(idx, other[0]) and np.array_equal(val.view(np.uint32), other[1].view(np.uint32))
+
+
+def test_infinite_scores_rank_as_in_the_split_scan(gpu):
+    # 256 and 384 components: launches of 32 to 128 queries rank an infinite score last, as the split scan of
+    # smaller corpora does (test_non_finite_rows_depend_on_the_scan); the 22 queries past 128 rank it first
+    capi = gpu
+    n, dim, batch, k = 400_003, 256, 150, 10
+    rows, queries = normalized(n, dim, 97), normalized(batch, dim, 98)
+    rows[7, 5] = np.inf
+    queries[:, 5] = np.abs(queries[:, 5]) + np.float32(0.01)
+    idx, val, _ = run(capi, rows, capi.F32, queries, k, 1)
+    assert not (idx[:128] == 7).any() and np.isfinite(val[:128]).all()
+    assert (idx[128:, 0] == 7).all() and np.isinf(val[128:, 0]).all()
+    rows[7] = 0.0
+    finite = run(capi, rows, capi.F32, queries, k, 1)
+    assert np.array_equal(idx[:128], finite[0][:128]) and np.array_equal(idx[128:, 1:], finite[0][128:, :-1])

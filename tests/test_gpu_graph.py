@@ -25,6 +25,14 @@ def _f16_desc(capi, n, dim, batch, k, seed):
     return capi.search_desc(store, capi.DeviceArray.from_host(queries), batch, k)
 
 
+def _f16_masked_desc(capi, n, dim, batch, k, seed):
+    desc = _f16_desc(capi, n, dim, batch, k, seed)
+    mask = (np.random.default_rng(seed).random(n) < 0.3).astype(np.uint8)
+    rows = capi.DeviceArray.from_host(mask)
+    desc.mask, desc.keep = rows.ptr, rows
+    return desc
+
+
 def _f32_desc(capi, n, dim, batch, k, seed):
     corpus = normalized(n, dim, seed)
     queries = normalized(batch, dim, seed + 1)
@@ -61,6 +69,10 @@ def _binary_desc(capi, n, dim, batch, k, seed):
     (_f16_desc, 150_000, 384, 1, 10),      # single pass, one query
     (_f16_desc, 150_000, 384, 16, 10),     # fp16 MFMA scan
     (_f32_desc, 200_000, 384, 64, 10),     # fp32 bf16-split MFMA scan
+    (_f16_desc, 150_000, 768, 16, 10),     # filter scan
+    (_f16_masked_desc, 150_000, 300, 20, 10),  # with a row list
+    (_int8_desc, 150_000, 640, 16, 10),    # of per-vector int8
+    (_f32_desc, 400_003, 256, 40, 10),     # in two phases
     (_binary_rescore_desc, 200_000, 1024, 1, 10),  # single pass of 1000 keys, group merges, rescore
     (_int8_desc, 1_000_000, 256, 256, 100),     # sketch plan: sketch, thresholds, one scan, merge
     (_int8_tiny_desc, 1_000_000, 256, 256, 100),  # sketch plan with every query rerun
