@@ -7,8 +7,8 @@
 // approximation plus bound reaches the query's threshold are scored exactly, as the VALU scan
 // scores them (scan_core.hpp), and only exact scores become keys. So the results are those of the VALU
 // scan bit for bit, and the approximation decides nothing but how many pairs are scored twice. Where that
-// is most of them (rows closer to each other than the bound, about 0.15% of |q| |x| for float32 and 0.05% for the
-// others; a query that is NaN) it costs: 1M rows within 2% of 16 topics, float32 x 384, 64 queries 0.34 ->
+// is most of them (rows closer to each other than the bound, about 0.15% of |q| |x| for float32 and 0.05%
+// for the others; a query that is NaN) it costs: 1M rows within 2% of 16 topics, float32 x 384, 64 queries 0.34 ->
 // 1.4 ms (the split scan 0.45), float16 x 768, 32 queries 0.34 -> 2.0 (the VALU scan 5.5).
 #pragma once
 

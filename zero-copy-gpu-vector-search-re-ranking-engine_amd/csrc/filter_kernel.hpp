@@ -4,7 +4,8 @@
 // Work split. One workgroup of 8 wavefronts per compute unit. The launch's query operands (up to
 // 8 groups of 16 queries) lie in LDS for the whole launch; every wavefront streams rows of its own
 // straight into registers, so no barrier runs in the loop (but for the cuts of a crowded search). A
-// wavefront's tile is kBlocks blocks of 16 rows, of which it keeps kPieces pieces of 256 bytes of
+// wavefront's tile is kBlocks blocks of 16 rows (fewer of them where few rows are to be shared by all
+// wavefronts, filterTileLog2), of which it keeps kPieces pieces of 256 bytes of
 // every row in flight (whole rows up to 1 KB), four 16-byte loads a lane, block and piece: as it
 // consumes a load it starts the same one of the next tile. That is 8 to 16 KB of consecutive
 // memory per wavefront, read at about one time; registers take rows at any alignment, which is why rows of no
@@ -15,12 +16,12 @@
 // touch 16 lines of 16 bytes each per quarter-wavefront and stream half as fast.
 //
 // What bounds it: HBM. Measured (kernel alone; the VALU scan it replaces took 17 to 6 times as long for
-// the whole search, the bf16 split scan 1.3): 1M x 768 float16, 32 queries, k = 100 272 us (5.6 of
-// the 7.07 TB/s a streaming read reaches), 1M x 384 float32, 64 queries 263 us (5.8), 500,009 x 256
-// float32 L2 87 us, 400,009 x 300 float16 49 us (4.9), 300,000 allowed rows of 1M x 384 float16 42 us
-// (5.5), 1M x 384 int8, 8 queries 77 us (5.0: it also converts its codes to halves; 94 while the
-// exact scores held all of a query's chunks and spilled registers). A ring of more registers (6 and 8 pieces) made the compiler spill: 297-310 us for the
-// first; tiles of 64 rows a piece at a time 577 us.
+// the whole search, the bf16 split scan 1.2): 1M x 768 float16, 32 queries, k = 100 279 us (5.5 of
+// the 7.07 TB/s a streaming read reaches), 1M x 384 float32, 64 queries 48 and 238 us in two launches (5.4),
+// 500,009 x 256 float32 L2 90 us (5.7), 400,009 x 300 float16 52 us (4.6), 300,000 allowed rows of 1M x 384
+// float16 43 us (5.4), 1M x 384 int8, 8 queries 80 us (4.8: it also converts its codes to halves; 94 while the
+// exact scores held all of a query's chunks and spilled registers). A ring of more registers (6 and 8
+// pieces) made the compiler spill: 297-310 us for the first; tiles of 64 rows a piece at a time 577 us.
 //
 // MFMA layout (16x16x32 f16): the queries are the first operand (lane l supplies query l % 16 and 8
 // dimensions), the rows the second (row l % 16, the same 8 dimensions), so a lane's results belong
