@@ -215,6 +215,12 @@ def test_phase_rows_cover_the_corpus_once(capi, n, dtype, int8_mode, batch, k):
     assert all(r > 0 for r in rows)
 
 
+@pytest.mark.parametrize("dim,dtype,batch", [(768, 3, 7), (256, 3, 7), (1024, 3, 7), (384, 1, 16)])
+def test_one_dense_phase_below_8192_rows(capi, dim, dtype, batch):
+    for n, phases in ((7_474, 1), (8_191, 1), (8_400, 2)):
+        assert len(capi.search_phase_rows(_desc(capi, n=n, dim=dim, dtype=dtype, batch=batch))) == phases
+
+
 @pytest.mark.parametrize("n,dim,dtype,batch,masked,filtered", [
     (5_000, 922, 0, 1, False, False),    # odd rows: a few thousand take the score matrix
     (10_000, 301, 2, 5, False, False),
