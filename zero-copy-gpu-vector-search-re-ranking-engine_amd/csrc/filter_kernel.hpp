@@ -295,7 +295,7 @@ void filterScanKernel(ScanArgs scan, FilterArgs args, PhaseArgs phase, EmitArgs 
     // ---- tiles ----
     const long long row_blocks = (rows + kFilterBlockRows - 1) / kFilterBlockRows;
     // (a short row list: smaller tiles, as filterTileLog2 makes them where the host knows the rows)
-    const int tile_log2 = list != nullptr ? filterTileLog2(rows, kBlocks * kFilterBlockRows, gridDim.x * kFilterWaves)
+    const int tile_log2 = list != nullptr ? filterTileLog2(rows, kBlocks * kFilterBlockRows, gridDim.x * kFilterWaves, 0)
                                           : args.tile_log2;
     long long tiles = list != nullptr ? (rows + (1LL << tile_log2) - 1) >> tile_log2 : phase.items;
     long long stride = 1;  // sketch: one block of every `stride`

@@ -423,7 +423,8 @@ FilterShape filterShape(const ScanArgs& scan, int width) {
         1 << filterTileLog2(scan.doc_count,
                             kFilterBlockRows * filterBlocks(filterSlots(static_cast<int>((bytes + 255) / 256)),
                                                             shape.groups_per_launch, scan.lexical != nullptr),
-                            deviceComputeUnits() * kFilterWaves);
+                            deviceComputeUnits() * kFilterWaves,
+                            8LL * scan.batch * width > scan.doc_count ? 0 : 4);  // (about two pairs per key are scored)
     launches = (groups + shape.groups_per_launch - 1) / shape.groups_per_launch;
     shape.groups = launches * shape.groups_per_launch;
     shape.supported = true;
