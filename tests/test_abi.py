@@ -225,7 +225,8 @@ def test_one_dense_phase_below_8192_rows(capi, dim, dtype, batch):
     (5_000, 922, 0, 1, False, False),    # odd rows: a few thousand take the score matrix
     (10_000, 301, 2, 5, False, False),
     (30_000, 301, 1, 16, False, True),
-    (80_000, 100, 1, 1, False, True),
+    (5_768, 969, 0, 24, False, True),
+    (160_000, 100, 1, 1, False, True),
     (10_000, 301, 0, 128, True, False),  # a mask that lets a few rows through leaves all their pairs
     (200_000, 301, 0, 128, True, True),
     (2_000, 384, 2, 9, False, False),    # whole chunks

@@ -398,17 +398,22 @@ bool filterPays(const ScanArgs& scan, const Plan& plan) {
     const std::size_t row_bytes = rowBytes(scan.dtype, scan.dim);
     const long long tiles = (scan.batch + 7) / 8;  // of the queries the VALU kernels take at a time
     if (row_bytes % 16 != 0) {
-        // The materialized pipeline's scalar scan takes about 0.22 ns per row, query tile and 64 components
-        // and its other launches 16 us, the filter scan 35 us (922 components 45) and the exact scores,
-        // against 2304 shapes: float16 x 100, 1 query, 40,000 rows 29 / 36, 80,000 39 / 37, 16 queries, 10,000
-        // rows 32 / 38, 40,000 56 / 40; float32 x 922, 1 query, 20,000 rows 49 / 59, 40,000 85 / 71; int8 x
-        // 301, 100 queries, 5,000 rows 77 / 56. With a mask the list takes 6 us, and where the mask lets through
-        // fewer rows than are selected a wavefront scores one row against every query, about 4 us each
-        // (3,000 x 922 int8, 5% allowed, 100 queries 73 / 129; 10,000 x 301 float32, 0.4%, 128 queries 86 / 214).
+        // Both plans' times, in ps, from 2000 shapes: the score matrix's scalar scan takes 90 per row, 64 components
+        // and query tile and 20 per query, the filter scan 22 us and 0.6 per 64 components more than the other's
+        // fixed 16, the rows' bytes at 6 TB/s, and 4500 per selected key. float16 x 100, 1 query, 40,000 rows 29 / 36,
+        // 160,000 66 / 43, 16 queries, 10,000 rows 32 / 38, 40,000 56 / 40; float32 x 922, 1 query, 20,000 rows 49 /
+        // 59, 40,000 85 / 71, 16 queries, 5,000 rows 62 / 55; 3,000 x 301, 100 queries, k = 50 55 / 69.
+        // With a mask the list takes 6 us, and where the mask lets through fewer rows than are selected a
+        // wavefront scores one row against every query, about 4 us each (3,000 x 922 int8, 5% allowed, 100
+        // queries 73 / 129; 10,000 x 301 float32, 0.4%, 128 queries 86 / 214; 17,399 x 799 float32 L2, 8%, 92
+        // queries, k = 162 221 / 298).
         const long long pieces = (scan.dim + 63) / 64;
-        const long long cost = n * tiles * pieces;
-        return scan.mask != nullptr ? cost >= 80'000 + (24'000 + 1'200LL * scan.batch) * pieces
-                                    : cost >= 120'000 + 16'000 * pieces + 5LL * scan.batch * plan.width;
+        const long long keys = static_cast<long long>(scan.batch) * plan.width;
+        if (scan.mask != nullptr) {
+            return n * tiles * pieces >= 60'000 + (24'000 + 1'200LL * scan.batch + 5 * keys) * pieces;
+        }
+        return n >= 2048 && n * pieces * (90 * tiles + 20 * scan.batch) >=
+                                22'000'000 + 600'000 * pieces + n * static_cast<long long>(row_bytes) / 6 + 4'500 * keys;
     }
     if (plan.use_mfma_float) {
         // Up to 8191 rows that scan is one dense phase (5,000 x 384 float32, 64 queries 26 against 42;
